@@ -6,16 +6,15 @@
 // per-g-point results), ISW_FORM_MIXED=1 with -ffp-contract=fast into isw_mix (`fast` = float and the transcendentals
 // in float, as the reference's MIXED build; every g-point sum stays FP64).
 //
-// Design (MI355X): the column pass is one 64-aligned block per column, one thread per g-point, the column's sub-level
-// properties staged once in LDS. Kernels are instantiated per layer count so that every per-g-point array (optical
-// depths; the shortwave's reflectances, transmittances and albedos) has a compile-time size and stays in VGPRs. The
-// shortwave computes its sub-levels from the bottom up, so the clear sky's adding and the all-sky albedos run in the
-// same loop (the clear sky needs nothing stored); between its two passes it keeps the albedos (and in FP64 the gas
-// depths), recomputing each sub-level's optics on the way down. Per-g results go to
-// LDS as float32 (the reference's red[][] width), then every wave sums whole rows: each lane adds its g-points in
-// order, in FP64, and a butterfly finishes the row -- a fixed order, so results repeat bit for bit. Blocks are
-// renumbered so that each XCD takes a contiguous range of columns (the sub-level reads of neighbouring columns share
-// cache lines).
+// Design (MI355X): a 64-aligned block takes columns in turn, one thread per g-point, the column's sub-level properties
+// staged once in LDS as what the walk needs (table offsets, bilinear weights, amounts). Kernels are instantiated per
+// layer count so that every per-g-point array has a compile-time size and stays in VGPRs, and each walks the sub-levels
+// once: what the walk back needs is kept as small linear maps per layer instead of being computed again. A column's table
+// rows are the same for all its g-points, so their bases are scalar and the lanes differ by g alone. Per-g results go to
+// LDS as float32 (the reference's red[][] width) and are summed in FP64 in a fixed order, so results repeat bit for bit.
+// Blocks are renumbered so that each XCD takes a contiguous range of columns (the sub-level reads of neighbouring columns
+// share cache lines). Measured at 40,962 columns x 7 layers, mixed: lw_column (256 g-points) 3.72 -> 1.44 ms, sw_column
+// (224) 6.86 -> 2.21 ms; FP64 at 2,562 x 3 (144 / 112): 192 -> 109 us and 273 -> 113 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -53,7 +52,7 @@ __device__ __forceinline__ double FPOWd(double x, double y) {
   return pow(x, y);
 #endif
 }
-// The column passes' exp and division: FP64 in the plain form (the reference's operations); in the mixed form the
+// The column passes' exp and quotient: FP64 in the plain form (the reference's operations); in the mixed form the
 // hardware's: exp as 2^(x log2 e) (v_exp_f32) and a / b as a times the hardware reciprocal, each within a few float
 // steps (the mixed form's bar against FP64 is 1e-4 of the fluxes).
 __device__ __forceinline__ fast fexp(fast x) {
@@ -63,11 +62,33 @@ __device__ __forceinline__ fast fexp(fast x) {
   return exp(x);
 #endif
 }
-__device__ __forceinline__ fast fdiv(fast a, fast b) {
+__device__ __forceinline__ fast fquot(fast a, fast b) {
 #if ISW_FORM_MIXED
-  return __fdividef(a, b);
+  return a * __builtin_amdgcn_rcpf(b);
 #else
   return a / b;
+#endif
+}
+// The shortwave's layer optics divide by 1 - (k mu0)^2, which passes through zero where the beam and the diffuse light
+// decay alike: what they lose to rounding there is a thousand times larger, so their quotients and square root are
+// rounded as IEEE's are: one Newton step on the hardware's reciprocal (or reciprocal root), then one on the residual, and
+// the fix-up for zeros and infinities. Six instructions besides the reciprocal where the compiler's division takes ten.
+__device__ __forceinline__ fast fdiv(fast a, fast b) {
+#if ISW_FORM_MIXED
+  float y = __builtin_amdgcn_rcpf(b);
+  y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+  const float q = a * y;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
+#else
+  return a / b;
+#endif
+}
+__device__ __forceinline__ fast fsqrt(fast x) {         // (x >= 1e-12)
+#if ISW_FORM_MIXED
+  const float y = __builtin_amdgcn_rsqf(x), s = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+#else
+  return sqrt(x);
 #endif
 }
 
@@ -222,158 +243,338 @@ __global__ void __launch_bounds__(64) k_lw_setup(int N, RadP P, isw_lw_tables t,
 #undef W
 }
 
-// ln k bilinear in (log p, T) on one table cell, then exp (air.cu:2266-2271).
-__device__ __forceinline__ fast kbil(const float* __restrict__ K, int NT, int NG, fast fp, fast ft) {
-  const fast v00 = K[0], v01 = K[NG], v10 = K[(size_t)NT * NG], v11 = K[(size_t)NT * NG + NG];
-  return fexp(v00 + (v10 - v00) * fp + (v01 - v00) * ft + (v00 - v01 - v10 + v11) * fp * ft);
+// A value that every lane holds alike, in a scalar register: the table rows a column reads are the same for all its
+// g-points, so their base addresses cost scalar arithmetic only and each load's lane offset is g.
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ float uni(float x) { return __int_as_float(uni(__float_as_int(x))); }
+__device__ __forceinline__ double uni(double x) {
+  return __hiloint2double(uni(__double2hiint(x)), uni(__double2loint(x)));
 }
 
-// Two-stream through one sub-level, far side's Planck radiance Bf to the near side's Bn, linear in optical depth,
-// diffusivity 1.66 (air.cu:2123-2127).
-__device__ __forceinline__ fast lw_through(fast I, fast tau, fast Bn, fast Bf) {
-  const fast x = tau * (fast)1.66, tr = fexp(-x);
-  const fast lin = x > (fast)1e-3 ? 1 - fdiv(1 - tr, x) : x * ((fast)0.5 - x / 6);
-  return I * tr + Bf * (1 - tr) + (Bn - Bf) * lin;
+// A table row's base address, kept in scalar registers as it is: without this the compiler folds the tables' fixed
+// offsets into per-lane addresses that it holds in registers over the whole kernel (two per table row and corner).
+typedef const __attribute__((address_space(1))) float* tabp;
+__device__ __forceinline__ tabp row_at(const float* tab, size_t off) {
+  tabp p = (tabp)tab + off;
+  asm("" : "+s"(p));
+  return p;
 }
 
-// Rows of per-g float values in LDS (rows x ngp) summed over g-points: each wave takes whole rows, each lane adds its
-// g-points in order in FP64, a butterfly finishes the row; sums[r] gets the result (every row, fixed order).
-template <int ROWS>
-__device__ __forceinline__ void g_sums(const float* red, int ngp, double* sums) {
-  const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6, nw = ngp >> 6;
-  for (int r = w; r < ROWS; r += nw) {
-    double v = 0;
-    for (int m = 0; m < nw; m++) v += (double)red[r * ngp + m * 64 + lane];
+// Pins a value computed here to this place: without it the compiler sinks the arithmetic to the value's use at the end
+// of the column and keeps its operands, two to three times as many, in registers instead.
+__device__ __forceinline__ void pin(fast& x) { asm volatile("" : "+v"(x)); }
+
+// A sub-level's place in the ln k tables: the element offset of its (log p, T) cell and the four corners' bilinear
+// weights. In the mixed form the weights carry log2 e, so that exp(ln k) is the hardware's 2^x of the weighted sum.
+struct Cell {
+  fast w00, w10, w01, w11;
+};
+__device__ __forceinline__ Cell cell_weights(fast fp, fast ft) {
+  const double s = ISW_FORM_MIXED ? 1.4426950408889634 : 1.0, p = fp, t = ft;
+  return Cell{(fast)((1 - p) * (1 - t) * s), (fast)(p * (1 - t) * s), (fast)((1 - p) * t * s), (fast)(p * t * s)};
+}
+__device__ __forceinline__ fast kexp(fast x) {
+#if ISW_FORM_MIXED
+  return __builtin_amdgcn_exp2f(x);
+#else
+  return exp(x);
+#endif
+}
+// One float at a 32-bit byte offset beside a scalar base: no 64-bit lane address.
+__device__ __forceinline__ float at(tabp p, unsigned o) {
+  asm("" : "+v"(o));
+  return *(tabp)((const __attribute__((address_space(1))) char*)p + o);
+}
+// The optical depth of one g-point (air.cu:2266-2271,2425-2437): per component k = exp of ln k bilinear in (log p, T),
+// times its amount a[c]. load() asks for every corner of a sub-level's cell at once (o: the lane's byte offsets of the four
+// corners in a component's table row), depth() uses them. (Loading a sub-level ahead instead was slower wherever its
+// registers cost a wave per SIMD: the other waves hide the tables' latency better.)
+template <int NCOMP>
+struct Corners {
+  float v[NCOMP][4];
+  __device__ __forceinline__ void load(const float* logk, size_t cell, size_t cs, const unsigned (&o)[4]) {
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) sums[r] = v;
+    for (int c = 0; c < NCOMP; c++) {
+      const tabp K = row_at(logk, cell + c * cs);
+#pragma unroll
+      for (int m = 0; m < 4; m++) v[c][m] = at(K, o[m]);
+    }
+  }
+  __device__ __forceinline__ fast depth(const Cell& q, const fast* a) const {
+    fast tau = 0;
+#pragma unroll
+    for (int c = 0; c < NCOMP; c++)
+      tau += a[c] * kexp(q.w00 * (fast)v[c][0] + q.w10 * (fast)v[c][1] + q.w01 * (fast)v[c][2] + q.w11 * (fast)v[c][3]);
+    return fmax((fast)0, tau);
+  }
+  // The same by the differences of ln k on the cell, water's two tables blended by fh: each operation's rounding then as
+  // the layer optics' comment asks.
+  __device__ __forceinline__ fast blend(fast fp, fast ft, const fast* u, fast fh) const {
+    fast lk[NCOMP];
+#pragma unroll
+    for (int c = 0; c < NCOMP; c++) {
+      const fast v00 = v[c][0], v10 = v[c][1], v01 = v[c][2], v11 = v[c][3];
+      lk[c] = fexp(v00 + (v10 - v00) * fp + (v01 - v00) * ft + (v00 - v01 - v10 + v11) * fp * ft);
+    }
+    static_assert(NCOMP == 7, "the shortwave's components");
+    return fmax((fast)0, u[0] * (lk[0] + (lk[1] - lk[0]) * fh) + u[1] * lk[2] + u[2] * lk[3] + u[3] * lk[4] +
+                             u[4] * lk[5] + u[5] * lk[6]);
+  }
+};
+
+// Per-g float values in LDS summed over the g-points: g-point m's values at red[m * S ..], S odd, so that a wave's writes
+// fall on different banks and every value's address is the lane's own plus a constant (with rows g-points long, their
+// run-time length cost a register per row for the addresses). Eight lanes per row, each adding every eighth g-point in
+// FP64, then three exchanges: a fixed order, so results repeat bit for bit. Lane 0 of the eight gets the row's sum.
+template <int ROWS, int S, class F>
+__device__ __forceinline__ void g_sums(const float* red, int NG, F&& put) {
+  static_assert(S % 2 == 1 && ROWS <= S, "odd stride");
+  const int part = (int)threadIdx.x & 7, nr = (int)blockDim.x >> 3;
+  for (int r = (int)threadIdx.x >> 3; r < ROWS; r += nr) {
+    double v = 0;
+    for (int m = part; m < NG; m += 8) v += (double)red[m * S + r];
+#pragma unroll
+    for (int o = 4; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    if (part == 0) put(r, v);
   }
 }
 
+// f(S), f(S - 1), .., f(0), each with its own constant.
+template <int S, class F>
+__device__ __forceinline__ void down_from(F&& f) {
+  f(S);
+  if constexpr (S > 0) down_from<S - 1>(f);
+}
+
+// The columns a block takes in turn: enough of them to share the block's set-up, few enough to leave several blocks per
+// slot of the chip (256 CUs, about three blocks each) so that the last ones do not run alone.
+static inline int cols_per_block(int N) {
+  const int c = N / (256 * 3 * 4);
+  return c < 1 ? 1 : c > 8 ? 8 : c;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
-// lw_column (air.cu:2231-2348): one block per column, one thread per g-point (block = NG rounded up to 64).
+// lw_column (air.cu:2231-2348): a block takes its columns in turn, one thread per g-point (block = NG rounded up to 64).
+// One walk down the sub-levels does everything that costs: each sub-level's transmission t and its emission both ways,
+// I' = I t + E down the walk at once, and the way up as the layer's affine maps (T, E) from its bottom to the three
+// edges that results need, composed inside the layer (clear and cloudy chains blended by the cover, as the fluxes are).
+// The way up is then two multiply-adds per edge. (Recomputing the emission on the way up, with the tables' rows
+// addressed per lane, the pass took 3.74 ms at 40,962 x 7 x 256 in the mixed form.)
 // ---------------------------------------------------------------------------------------------------------------
 template <int L>
-__global__ void __launch_bounds__(NGMAX) k_lw_column(int N, RadP P, isw_lw_tables t, const float* __restrict__ sub,
-                                                      const double* __restrict__ Ts, double* __restrict__ radf) {
-  constexpr int NSS = NSUB * L, RW = L + 1, E0 = 3 * RW + 3, ROWS = E0 + 6 * L;
-  extern __shared__ float red[];                       // ROWS x ngp
-  __shared__ fast sTt[NSS], sTb[NSS], sfp[NSS], sft[NSS], su[NSS][5], sfh[NSS], stc[NSS], sfc[NSS], scia[NSS];
-  __shared__ int sip[NSS], sit[NSS];
-  __shared__ double sums[ROWS];
-  const int i = xblock(), g = (int)threadIdx.x, ngp = (int)blockDim.x;
-  const int NG = t.NG, NT = t.NT, NTP = t.NTP;
-  if (g < NSS) {
-    const int s = g;
+struct LwRows {
+  static constexpr int NUP = 4 + 6 * L, NDN = 3 * L;
+  // the sums of the way down before the way up, in the same LDS, where all of them at once would keep a CU from holding
+  // three blocks (at 7 layers: 1.41 ms against 1.89 ms with two blocks)
+  static constexpr bool SPLIT = (NUP + NDN) * NGMAX * 4 + 2600 > 160 * 1024 / 3;
+  static constexpr int DN0 = SPLIT ? 0 : NUP, S = (SPLIT ? NUP : NUP + NDN) | 1;
+};
+
+template <int L>
+__global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw_lw_tables t,
+                                                      const float* __restrict__ sub, const double* __restrict__ Ts,
+                                                      double* __restrict__ radf) {
+  constexpr int NSS = NSUB * L, RW = L + 1, E0 = 3 * RW + 3;
+  using R = LwRows<L>;
+  extern __shared__ float red[];                       // R::S per g-point
+  __shared__ Cell sq[NSS];
+  __shared__ fast sa[NSS][6], scl[NSS], sft[NSS], scia[NSS], sfc[L];   // (amounts; cloud; T share; CIA; cover)
+  __shared__ fast spt[NSS + 1], spb[NSS];              // Planck table shares (the last: the surface's)
+  __shared__ int so[NSS], sit[NSS], sjt[NSS + 1], sjb[NSS];
+  const unsigned g = threadIdx.x, NG = t.NG, row = (unsigned)(t.NT * t.NG);
+  const unsigned o4[4] = {4 * g, 4 * (g + row), 4 * (g + NG), 4 * (g + row + NG)};
+  const size_t cs = (size_t)t.NP * t.NT * t.NG;
+  const int i0 = xblock() * cpb, i1 = min(i0 + cpb, N);
+  auto planck_at = [&](fast T, int& j) -> fast {
+    const float y = fminf(fmaxf((float)(T - (fast)t.tp0), 0.f), (float)((fast)(t.NTP - 1) - (fast)1e-4f));
+    j = (int)y;
+    return (fast)y - (fast)j;
+  };
+  auto stage = [&](int i) {
+    if (g < NSS) {
+      const int s = g;
 #define R_(v) sub[((size_t)s * NVP + (v)) * N + i]
-    sTt[s] = R_(0);
-    sTb[s] = R_(1);
-    // lw_setup writes the positions inside the tables; clamped again here so that no input reads outside them
-    const fast x = clampf_pos(R_(2), t.NP), y = clampf_pos(R_(3), NT);
-    sip[s] = (int)x;
-    sfp[s] = x - (fast)sip[s];
-    sit[s] = (int)y;
-    sft[s] = y - (fast)sit[s];
+      // lw_setup writes the positions inside the tables; clamped again here so that no input reads outside them
+      const fast x = clampf_pos(R_(2), t.NP), y = clampf_pos(R_(3), t.NT);
+      const int ip = (int)x, it = (int)y;
+      so[s] = (ip * t.NT + it) * t.NG;
+      sit[s] = it * t.NG;
+      sft[s] = y - (fast)it;
+      sq[s] = cell_weights(x - (fast)ip, y - (fast)it);
+      const fast u0 = R_(4), fh = R_(9), df = (fast)1.66;
+      sa[s][0] = df * (u0 * (1 - fh));                 // (water's two tables blended by its share; diffusivity 1.66)
+      sa[s][1] = df * (u0 * fh);
 #pragma unroll
-    for (int c = 0; c < 5; c++) su[s][c] = R_(4 + c);
-    sfh[s] = R_(9);
-    stc[s] = R_(10);
-    sfc[s] = R_(11);
-    scia[s] = R_(14);
+      for (int c = 1; c < 5; c++) sa[s][c + 1] = df * (fast)R_(4 + c);
+      scl[s] = R_(10);
+      if (s % NSUB == 0) sfc[s / NSUB] = R_(11);
+      scia[s] = df * (fast)R_(14);
+      int j;
+      spt[s] = planck_at(R_(0), j);
+      sjt[s] = j * t.NG;
+      spb[s] = planck_at(R_(1), j);
+      sjb[s] = j * t.NG;
 #undef R_
-  }
-  __syncthreads();
-#define RED(r, v) red[(r) * ngp + g] = (float)(v)
-  if (g < NG) {
-    const fast refl = P.lw_refl > 0 ? (fast)(1 - P.eps_s) : (fast)0;
-    const size_t cs = (size_t)t.NP * NT * NG;
-    fast tau[NSS];
-#pragma unroll
-    for (int s = 0; s < NSS; s++) {
-      const float* K = t.logk + ((size_t)sip[s] * NT + sit[s]) * NG + g;
-      const fast fp = sfp[s], ft = sft[s];
-      fast lk[6];
-#pragma unroll
-      for (int c = 0; c < 6; c++) lk[c] = kbil(K + c * cs, NT, NG, fp, ft);
-      tau[s] = fmax((fast)0, su[s][0] * (lk[0] + (lk[1] - lk[0]) * sfh[s]) + su[s][1] * lk[2] + su[s][2] * lk[3] +
-                                 su[s][3] * lk[4] + su[s][4] * lk[5]);
-      if (t.cia) {
-        const float* C = t.cia + (size_t)sit[s] * NG + g;
-        tau[s] += scia[s] * (C[0] + (C[NG] - C[0]) * ft);
-      }
     }
-    const float* pg = t.planck;
-    auto Bof = [&](fast T) -> fast {
-      const float y = fminf(fmaxf((float)(T - (fast)t.tp0), 0.f), (float)((fast)(NTP - 1) - (fast)1e-4f));
-      const int j = (int)y;
-      const float b0 = pg[(size_t)j * NG + g], b1 = pg[(size_t)(j + 1) * NG + g];
-      return b0 + (fast)(b1 - b0) * ((fast)y - (fast)j);
-    };
-    const fast PIf = (fast)PI_;
+    if (g == NSS) {                                    // (a block has 64 threads or more, NSS at most 32)
+      int j;
+      spt[NSS] = planck_at((fast)Ts[i], j);
+      sjt[NSS] = j * t.NG;
+    }
+  };
+  if (i0 >= i1) return;
+  stage(i0);
+  __syncthreads();
+#define UP(r, v) red[g * R::S + (r)] = (float)(v)
+#define DOWN(r, v) red[g * R::S + R::DN0 + (r)] = (float)(v)
+  for (int i = i0; i < i1; i++) {
+    const fast refl = P.lw_refl > 0 ? (fast)(1 - P.eps_s) : (fast)0, PIf = (fast)PI_;
     fast I = 0, Icl = 0;
-    RED(RW, 0.f);
+    fast mT[L][3], mE[L][3], cT[L], cE[L];
+    // what a sub-level reads from the tables: its gases' corners, the Planck rows of its two edges
+    struct {
+      Corners<6> k;
+      float t0, t1, b0, b1;
+    } row_s;
+    auto load = [&](int s) {
+      const tabp pt = row_at(t.planck, uni(sjt[s])), pb = row_at(t.planck, uni(sjb[s]));
+      row_s.t0 = at(pt, o4[0]); row_s.t1 = at(pt, o4[2]);
+      row_s.b0 = at(pb, o4[0]); row_s.b1 = at(pb, o4[2]);
+      row_s.k.load(t.logk, (size_t)uni(so[s]), cs, o4);
+    };
+    if (g < NG) {
 #pragma unroll
-    for (int k = 0; k < L; k++) {
-      const fast f = sfc[k * NSUB];
-      fast Ic = I, Id = I;
+      for (int k = 0; k < L; k++) {
+        const fast f = uni(sfc[k]);
+        fast Ic = I, Id = I;
+        fast tr[NSUB], eu[NSUB], tr2[NSUB], eu2[NSUB];
 #pragma unroll
-      for (int s = k * NSUB; s < (k + 1) * NSUB; s++) {
-        const fast Bt = Bof(sTt[s]), Bb = Bof(sTb[s]);
-        Ic = lw_through(Ic, tau[s], Bb, Bt);
-        if (refl > 0) Icl = lw_through(Icl, tau[s], Bb, Bt);
-        if (f > 0) Id = lw_through(Id, tau[s] + stc[s] / (fast)1.66, Bb, Bt);
-        if (s == k * NSUB) RED(E0 + 6 * k + 1, PIf * (f > 0 ? (1 - f) * Ic + f * Id : Ic));
-        if (s == (k + 1) * NSUB - 2) RED(E0 + 6 * k + 4, PIf * (f > 0 ? (1 - f) * Ic + f * Id : Ic));
-      }
-      I = f > 0 ? (1 - f) * Ic + f * Id : Ic;
-      RED(RW + k + 1, PIf * I);
-    }
-    const fast Bs = Bof((fast)Ts[i]);
-    fast Iu = refl * I, tr = 1, Iuc = refl * Icl, trc = 1;
-    RED(L, PIf * Iu);
-    RED(2 * RW + L, Bs);
-#pragma unroll
-    for (int k = L - 1; k >= 0; k--) {
-      const fast f = sfc[k * NSUB];
-      fast Ic = Iu, Id = Iu, tc = tr, td = tr;
-#pragma unroll
-      for (int s = (k + 1) * NSUB - 1; s >= k * NSUB; s--) {
-        const fast Bt = Bof(sTt[s]), Bb = Bof(sTb[s]);
-        const fast t1 = fexp(-tau[s] * (fast)1.66);
-        Iuc = lw_through(Iuc, tau[s], Bt, Bb);
-        trc *= t1;
-        Ic = lw_through(Ic, tau[s], Bt, Bb);
-        tc *= t1;
-        if (f > 0) {
-          Id = lw_through(Id, tau[s] + stc[s] / (fast)1.66, Bt, Bb);
-          td *= t1 * fexp(-stc[s]);
+        for (int j = 0; j < NSUB; j++) {
+          const int s = k * NSUB + j;
+          __builtin_amdgcn_sched_barrier(0);           // (sub-level by sub-level, or the registers run out)
+          load(s);
+          fast x = row_s.k.depth(sq[s], sa[s]);          // (1.66 times the optical depth)
+          if (t.cia) {
+            const tabp C = row_at(t.cia, uni(sit[s]));
+            x += scia[s] * ((fast)at(C, o4[0]) + ((fast)at(C, o4[2]) - (fast)at(C, o4[0])) * sft[s]);
+          }
+          // two-stream through the sub-level, the Planck radiance linear in optical depth, diffusivity 1.66
+          // (air.cu:2123-2127): t = e^-x, E = B_far (1 - t) + (B_near - B_far) lin
+          const fast Bt = row_s.t0 + (fast)(row_s.t1 - row_s.t0) * spt[s], Bb = row_s.b0 + (fast)(row_s.b1 - row_s.b0) * spb[s];
+          auto through = [&](fast y, fast& tt, fast& ed, fast& eup) {
+            tt = fexp(-y);
+            const fast om = 1 - tt, thin = y * ((fast)0.5 - y * (fast)(1.0 / 6.0)), thick = 1 - fquot(om, y);
+            const fast lin = y > (fast)1e-3 ? thick : thin;
+            ed = Bt * om + (Bb - Bt) * lin;
+            eup = Bb * om + (Bt - Bb) * lin;
+          };
+          fast ed;
+          through(x, tr[j], ed, eu[j]);
+          Ic = Ic * tr[j] + ed;
+          if (refl > 0) Icl = Icl * tr[j] + ed;
+          if (f > 0) {
+            tr2[j] = tr[j];
+            eu2[j] = eu[j];
+            fast ed2 = ed;
+            const fast cl = uni(scl[s]);
+            if (cl > 0) through(x + cl, tr2[j], ed2, eu2[j]);
+            Id = Id * tr2[j] + ed2;
+          }
+          const fast mix = f > 0 ? (1 - f) * Ic + f * Id : Ic;
+          if (j == 0) DOWN(3 * k + 1, PIf * mix);
+          if (j == NSUB - 2) DOWN(3 * k + 2, PIf * mix);
+          if (j == NSUB - 1) I = mix;
         }
-        const int e = s == (k + 1) * NSUB - 1 ? 3 : (s == k * NSUB + 1 ? 0 : -1);
-        if (e >= 0) {
-          RED(E0 + 6 * k + e, PIf * (f > 0 ? (1 - f) * Ic + f * Id : Ic));
-          RED(E0 + 6 * k + e + 2, (f > 0 ? (1 - f) * tc + f * td : tc) * Bs);
+        DOWN(3 * k, PIf * I);
+        fast T1 = 1, E1 = 0, T2 = 1, E2 = 0;
+#pragma unroll
+        for (int j = NSUB - 1; j >= 0; j--) {
+          E1 = E1 * tr[j] + eu[j];
+          T1 *= tr[j];
+          if (f > 0) {
+            E2 = E2 * tr2[j] + eu2[j];
+            T2 *= tr2[j];
+          }
+          const int e = j == NSUB - 1 ? 0 : j == 1 ? 1 : j == 0 ? 2 : -1;
+          if (e >= 0) {
+            mT[k][e] = f > 0 ? (1 - f) * T1 + f * T2 : T1;
+            mE[k][e] = f > 0 ? (1 - f) * E1 + f * E2 : E1;
+          }
         }
+        cT[k] = T1;
+        cE[k] = E1;
+#pragma unroll
+        for (int e = 0; e < 3; e++) { pin(mT[k][e]); pin(mE[k][e]); }
+        pin(cT[k]); pin(cE[k]); pin(I); pin(Icl);
       }
-      Iu = f > 0 ? (1 - f) * Ic + f * Id : Ic;
-      tr = f > 0 ? (1 - f) * tc + f * td : tc;
-      RED(k, PIf * Iu);
-      RED(2 * RW + k, tr * Bs);
     }
-    RED(3 * RW, PIf * Iuc);
-    RED(3 * RW + 1, trc * Bs);
-    RED(3 * RW + 2, Bs);
-  } else {
-    for (int r = 0; r < ROWS; r++) RED(r, 0.f);
+    // the sums of the way down: radf's rows RW + k + 1 and the layers' inner edges
+    auto sums_down = [&]() {
+      g_sums<R::NDN, R::S>(red + R::DN0, (int)NG, [&](int q, double w) {
+        const int k = q / 3, m = q - 3 * k;
+        radf[(size_t)(m == 0 ? RW + k + 1 : E0 + 6 * k + (m == 1 ? 1 : 4)) * N + i] = w;
+      });
+    };
+    if constexpr (R::SPLIT) {
+      __syncthreads();
+      sums_down();
+      __syncthreads();
+    }
+    if (g < NG) {
+      const tabp ps = row_at(t.planck, uni(sjt[NSS]));
+      const float b0 = at(ps, o4[0]), b1 = at(ps, o4[2]);
+      const fast Bs = b0 + (fast)(b1 - b0) * spt[NSS];
+      fast Iu = refl * I, trs = Bs, Iuc = refl * Icl, trc = Bs;       // (the transmissions weighted by Bs)
+      UP(0, PIf * Iu);
+#pragma unroll
+      for (int k = L - 1; k >= 0; k--) {
+        UP(4 + 6 * k, PIf * (Iu * mT[k][0] + mE[k][0]));
+        UP(4 + 6 * k + 1, trs * mT[k][0]);
+        UP(4 + 6 * k + 2, PIf * (Iu * mT[k][1] + mE[k][1]));
+        UP(4 + 6 * k + 3, trs * mT[k][1]);
+        Iu = Iu * mT[k][2] + mE[k][2];
+        trs *= mT[k][2];
+        Iuc = Iuc * cT[k] + cE[k];
+        trc *= cT[k];
+        UP(4 + 6 * k + 4, PIf * Iu);
+        UP(4 + 6 * k + 5, trs);
+      }
+      UP(1, PIf * Iuc);
+      UP(2, trc);
+      UP(3, Bs);
+    }
+    __syncthreads();
+    if constexpr (!R::SPLIT) sums_down();
+    {
+      // the surface's Planck sum (each wave by itself), then the rows, the transmissions over it
+      double bsum = 0;
+      for (int m = (int)threadIdx.x & 63; m < (int)NG; m += 64) bsum += (double)red[m * R::S + 3];
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) bsum += __shfl_xor(bsum, o);
+      g_sums<R::NUP, R::S>(red, (int)NG, [&](int q, double w) {
+        int r;
+        bool over = false;
+        if (q < 4) {
+          r = q == 0 ? L : 3 * RW + q - 1;
+          over = q == 2;
+        } else {
+          const int k = (q - 4) / 6, m = q - 4 - 6 * k;
+          r = m == 0 ? E0 + 6 * k + 3 : m == 1 ? E0 + 6 * k + 5 : m == 2 ? E0 + 6 * k : m == 3 ? E0 + 6 * k + 2
+              : m == 4 ? k : 2 * RW + k;
+          over = m & 1;
+        }
+        radf[(size_t)r * N + i] = over ? w / bsum : w;
+        if (q == 3) {
+          radf[(size_t)RW * N + i] = 0.0;              // (no light from above)
+          radf[(size_t)(2 * RW + L) * N + i] = bsum / bsum;
+        }
+      });
+    }
+    if (i + 1 < i1) stage(i + 1);
+    __syncthreads();
   }
-#undef RED
-  __syncthreads();
-  g_sums<ROWS>(red, ngp, sums);
-  __syncthreads();
-  if (g < ROWS) {
-    double v = sums[g];
-    if ((g >= 2 * RW && g < 3 * RW) || g == 3 * RW + 1 || (g >= E0 && (g - E0) % 3 == 2)) v /= sums[3 * RW + 2];
-    radf[(size_t)g * N + i] = v;
-  }
+#undef UP
+#undef DOWN
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -389,7 +590,7 @@ __device__ __forceinline__ void sw_layer(fast tau, fast ssa, fast g, fast mu0, f
   const fast g1 = (7 - ssa * (4 + 3 * g)) / 4, g2 = -(1 - ssa * (4 - 3 * g)) / 4, g3 = (2 - 3 * g * mu0) / 4;
   const fast g4 = 1 - g3;
   const fast a1 = g1 * g4 + g2 * g3, a2 = g1 * g3 + g2 * g4;
-  const fast k = sqrt(fmax((g1 - g2) * (g1 + g2), (fast)1e-12));
+  const fast k = fsqrt(fmax((g1 - g2) * (g1 + g2), (fast)1e-12));
   const fast e = fexp(-k * tau), e2 = e * e, k2e = 2 * k * e;
   fast rf = fdiv(1, k + g1 + (k - g1) * e2);
   Rd = g2 * (1 - e2) * rf;
@@ -417,184 +618,213 @@ __device__ double sun_lon(double t, const RadP& P) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// sw_column (air.cu:2384-2511): one block per column, one thread per g-point.
+// sw_column (air.cu:2384-2511): a block takes its columns in turn, one thread per g-point. One walk up the sub-levels
+// does everything that costs (table look-ups and optics once each): the clear and all-sky albedos below every edge, and
+// each sub-level's map of the light going down through it, Fdir' = d Fdir, Fdif' = a Fdif + c Fdir, with what lies
+// below already known. Only the nets at three edges per layer are wanted, so a layer keeps three maps (the second and
+// third sub-level's composed) with the albedos below each, 15 values per layer, and the way down is five multiply-adds
+// per edge. What bounds it then is the vector ALU: about 240 instructions and 17 transcendentals per sub-level. (Evaluating look-ups and optics again on the way down, with the tables' rows addressed per
+// lane and the sun's position found anew by one lane per column, the pass took 6.89 ms at 40,962 x 7 x 224 in the mixed
+// form.) The sun's direction at the four times of the interval is found once per block, one lane each.
 // ---------------------------------------------------------------------------------------------------------------
 template <int L>
-__global__ void __launch_bounds__(NGMAX) k_sw_column(int N, RadP P, isw_sw_tables t, isw_air air,
+__global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int N, int cpb, RadP P, isw_sw_tables t, isw_air air,
                                                       const float* __restrict__ sub, int mode,
                                                       const double* __restrict__ tnow, double interval,
                                                       const double* __restrict__ pos, const double* __restrict__ alb,
                                                       const double* __restrict__ cloudo, double* __restrict__ swf) {
-  constexpr int NSS = NSUB * L, ROWS = 3 * L + 2;
-  extern __shared__ float red[];                       // ROWS x ngp
-  __shared__ fast su[NSS][6], sfh[NSS], sfp[NSS], sft[NSS], sr[NSS], sh[NSS], stc[NSS], sfc[NSS], sli[NSS], scia[NSS];
-  __shared__ int sip[NSS], sit[NSS];
-  __shared__ fast smu;
-  __shared__ double sums[ROWS];
-  const int i = xblock(), g = (int)threadIdx.x, ngp = (int)blockDim.x;
-  const int NG = t.NG, NT = t.NT;
-  if (g < NSS) {
-    const int s = g, k = s / NSUB;
+  constexpr int NSS = NSUB * L, S = 6 * L + 1;
+  // The mixed form keeps the edges' albedos in the LDS slots that the sums use once they are spent, from four layers on:
+  // three waves per SIMD instead of two (15% at 7 layers; three layers fit anyway and lost 5% to it).
+  constexpr bool IN_LDS = ISW_FORM_MIXED && L >= 4;
+  extern __shared__ float red[];                       // S per g-point
+  __shared__ fast su[NSS][6], sfh[NSS], sfp[NSS], sr[NSS], sh[NSS], stc[NSS], sfc[NSS], sli[NSS], sft[NSS], scia[NSS];
+  __shared__ int so[NSS], sit[NSS];
+  __shared__ fast smu, salb;
+  __shared__ double sdir[4][3];                        // the sun's direction over the interval
+  const unsigned g = threadIdx.x, NG = t.NG, row = (unsigned)(t.NT * t.NG);
+  const unsigned o4[4] = {4 * g, 4 * (g + row), 4 * (g + NG), 4 * (g + row + NG)};
+  const size_t cs = (size_t)t.NP * t.NT * t.NG;
+  const int i0 = xblock() * cpb, i1 = min(i0 + cpb, N);
+  if (mode == 0 && g < 4) {
+    const double tt = tnow[0] + (g + 0.5) * interval / 4;
+    const double ang = sun_lon(tt, P), dec = asin(sin(P.tilt) * sin(ang));
+    const double rot = 2 * PI_ * fmod(tt, P.day_s) / P.day_s;
+    sdir[g][0] = cos(dec) * cos(-rot);
+    sdir[g][1] = cos(dec) * sin(-rot);
+    sdir[g][2] = sin(dec);
+  }
+  auto stage = [&](int i) {
+    if (g < NSS) {
+      const int s = g, k = s / NSUB;
 #define R_(v) sub[((size_t)s * NVP + (v)) * N + i]
-    // (positions clamped to this table's axes: the same values for lw_setup's sub-levels when the tables share their
-    // pressure axis, and no read outside the table for any input)
-    const fast x = clampf_pos(R_(2), t.NP);
-    const fast y = fmaxf(fminf((fast)R_(3) * (fast)t.yscale, (fast)(NT - 1) - 1e-4f), 0.f);
-    sip[s] = (int)x;
-    sfp[s] = x - (fast)sip[s];
-    sit[s] = (int)y;
-    sft[s] = y - (fast)sit[s];
+      // (positions clamped to this table's axes: the same values for lw_setup's sub-levels when the tables share their
+      // pressure axis, and no read outside the table for any input)
+      const fast x = clampf_pos(R_(2), t.NP);
+      const fast y = fmaxf(fminf((fast)R_(3) * (fast)t.yscale, (fast)(t.NT - 1) - 1e-4f), 0.f);
+      const int ip = (int)x, it = (int)y;
+      so[s] = (ip * t.NT + it) * t.NG;
+      sit[s] = it * t.NG;
+      sft[s] = y - (fast)it;
+      sfp[s] = x - (fast)ip;
 #pragma unroll
-    for (int c = 0; c < 5; c++) su[s][c] = R_(4 + c);
-    su[s][5] = (fast)air.o2 * R_(12);
-    sfh[s] = R_(9);
-    sr[s] = R_(12);
-    sh[s] = R_(13);
-    scia[s] = R_(14);
-    const bool cl = R_(10) > 0 && cloudo;
-    sfc[s] = cl ? (fast)cloudo[(size_t)k * N + i] : (fast)0;
-    stc[s] = cl ? (fast)(t.inhom * cloudo[(size_t)(2 * L + 3 + k) * N + i]) : (fast)0;
-    sli[s] = cl && t.cssa_i ? (fast)cloudo[(size_t)(3 * L + 3 + k) * N + i] : (fast)1;
+      for (int c = 0; c < 5; c++) su[s][c] = R_(4 + c);
+      su[s][5] = (fast)air.o2 * R_(12);
+      sfh[s] = R_(9);
+      sr[s] = R_(12);
+      sh[s] = R_(13);
+      scia[s] = R_(14);
+      const bool cl = R_(10) > 0 && cloudo;
+      sfc[s] = cl ? (fast)cloudo[(size_t)k * N + i] : (fast)0;
+      stc[s] = cl ? (fast)(t.inhom * cloudo[(size_t)(2 * L + 3 + k) * N + i]) : (fast)0;
+      sli[s] = cl && t.cssa_i ? (fast)cloudo[(size_t)(3 * L + 3 + k) * N + i] : (fast)1;
 #undef R_
-  }
-  if (g == ngp - 1) {                                 // the sun: the mean of its cosine over the interval's daylight
-    fast m = 0.5;
-    if (mode == 0) {
-      fast sum = 0;
-      int lit = 0;
-      for (int j = 0; j < 4; j++) {
-        const double tt = tnow[0] + (j + 0.5) * interval / 4;
-        const double ang = sun_lon(tt, P), dec = asin(sin(P.tilt) * sin(ang));
-        const double rot = 2 * PI_ * fmod(tt, P.day_s) / P.day_s;
-        const double cz = pos[3 * i] * cos(dec) * cos(-rot) + pos[3 * i + 1] * cos(dec) * sin(-rot) +
-                          pos[3 * i + 2] * sin(dec);
-        if (cz > 0) {
-          sum += (fast)cz;
-          lit++;
+    }
+    if (g == blockDim.x - 1) {                         // the sun: the mean of its cosine over the interval's daylight
+      fast m = 0.5;
+      if (mode == 0) {
+        fast sum = 0;
+        int lit = 0;
+        for (int j = 0; j < 4; j++) {
+          const double cz = pos[3 * (size_t)i] * sdir[j][0] + pos[3 * (size_t)i + 1] * sdir[j][1] +
+                            pos[3 * (size_t)i + 2] * sdir[j][2];
+          if (cz > 0) {
+            sum += (fast)cz;
+            lit++;
+          }
         }
+        m = lit ? sum / lit : (fast)0.05;
       }
-      m = lit ? sum / lit : (fast)0.05;
+      smu = fmax(m, (fast)0.02);
+      salb = (fast)alb[i];
     }
-    smu = fmax(m, (fast)0.02);
-  }
+  };
+  if (i0 >= i1) return;
+  __syncthreads();                                     // (the sun's directions)
+  stage(i0);
   __syncthreads();
-#define RED(r, v) red[(r) * ngp + g] = (float)(v)
-  if (g < NG) {
-    const fast mu0 = smu, a = (fast)alb[i];
-    const size_t cs = (size_t)t.NP * NT * NG;
-    const fast cssa = t.cssa[g], ray = t.ray[g], hzf = t.hzf[g];
-    const fast cssa_i = t.cssa_i ? (fast)t.cssa_i[g] : (fast)0, g_i = t.g_i ? (fast)t.g_i[g] : (fast)0;
-    // Sub-level s's optics from its gas optical depth tg: the clear sky's (c*) and the all-sky's (the cloud's share
-    // mixed in), as the reference computes them (air.cu:2440-2458). Evaluated twice per sub-level, in the albedos'
-    // pass up and the fluxes' pass down, so that only tg and the albedos are kept between the passes (a third of the
-    // registers that keeping every reflectance and transmittance would need; the table lookups are not repeated).
-    auto optics = [&](int s, fast tg, fast& cRd, fast& cTd, fast& cRs, fast& cTs, fast& cTdd, fast& rd, fast& td,
-                      fast& rs, fast& ts, fast& tdd) {
-      const fast trs = ray * sr[s] * (fast)air.ray, ths = (fast)t.tau550 * hzf * sh[s];
-      const fast tt = tg + trs + ths, sc = trs + (fast)t.hssa * ths;
-      const fast ssa = tt > 0 ? fmin(fdiv(sc, tt), (fast)(1 - 1e-6)) : (fast)0;
-      const fast ga = sc > 0 ? fdiv((fast)t.hg * (fast)t.hssa * ths, sc) : (fast)0;
-      sw_layer(tt, ssa, ga, mu0, cRd, cTd, cRs, cTs, cTdd);
-      rd = cRd; td = cTd; rs = cRs; ts = cTs; tdd = cTdd;
-      const fast f = sfc[s];
-      if (f > 0 && stc[s] > 0) {
-        const fast tc = stc[s], t2 = tt + tc;
-        fast cw = cssa, cg = (fast)P.cloud_g;
-        if (t.cssa_i) {
-          const fast sl = sli[s], wl = sl * cssa, wi = (1 - sl) * cssa_i;
-          cw = wl + wi;
-          cg = cw > 0 ? fdiv(wl * (fast)P.cloud_g + wi * g_i, cw) : cg;
+  // (volatile: else the kept albedos stay in registers too)
+  volatile __attribute__((address_space(3))) float* slot = (volatile __attribute__((address_space(3))) float*)(red + g * S);
+  const unsigned gc = g < NG ? g : 0;
+  const fast cssa = t.cssa[gc], ray = t.ray[gc], hzf = t.hzf[gc], wg = t.sun[gc];
+  const fast cssa_i = t.cssa_i ? (fast)t.cssa_i[gc] : (fast)0, g_i = t.g_i ? (fast)t.g_i[gc] : (fast)0;
+  for (int i = i0; i < i1; i++) {
+    if (g < NG) {
+      const fast mu0 = smu;
+      fast Ad = salb, As = Ad, cAd = Ad, cAs = Ad;
+      // per layer and wanted edge (below the first, the third and the last sub-level): the map down to it, 1 - Ad and
+      // 1 - As there
+      fast md[L][3], ma[L][3], mc[L][3], nd[L][3], ns[L][3];
+      auto walk = [&](int s) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);             // (sub-level by sub-level: see ISW_RAD_WAVES)
+        Corners<7> row_s;
+        row_s.load(t.logk, (size_t)uni(so[s]), cs, o4);
+        fast tg = row_s.blend(sfp[s], sft[s], su[s], sfh[s]);
+        if (t.cia) {
+          const tabp C = row_at(t.cia, uni(sit[s]));
+          tg += scia[s] * ((fast)at(C, o4[0]) + ((fast)at(C, o4[2]) - (fast)at(C, o4[0])) * sft[s]);
         }
-        const fast sc2 = sc + cw * tc;
-        const fast g2 = fdiv(ga * sc + cg * cw * tc, sc2);
-        fast r1, t1, r2, t3, d1;
-        sw_layer(t2, fmin(fdiv(sc2, t2), (fast)(1 - 1e-6)), g2, mu0, r1, t1, r2, t3, d1);
-        rd = (1 - f) * cRd + f * r1;
-        td = (1 - f) * cTd + f * t1;
-        rs = (1 - f) * cRs + f * r2;
-        ts = (1 - f) * cTs + f * t3;
-        tdd = (1 - f) * cTdd + f * d1;
-      }
-    };
-    // sub-level s's gas optical depth from the tables (air.cu:2425-2437)
-    auto gas = [&](int s) -> fast {
-      const float* K = t.logk + ((size_t)sip[s] * NT + sit[s]) * NG + g;
-      const fast fp = sfp[s], ft = sft[s];
-      fast lk[7];
+        // the sub-level's optics: molecules, haze and gas (air.cu:2440-2458), with the cloud's share mixed in
+        const fast trs = ray * sr[s] * (fast)air.ray, ths = (fast)t.tau550 * hzf * sh[s];
+        const fast tt = tg + trs + ths, sc = trs + (fast)t.hssa * ths;
+        const fast ssa = tt > 0 ? fmin(fdiv(sc, tt), (fast)(1 - 1e-6)) : (fast)0;
+        const fast ga = sc > 0 ? fdiv((fast)t.hg * (fast)t.hssa * ths, sc) : (fast)0;
+        fast cRd, cTd, cRs, cTs, cTdd;
+        sw_layer(tt, ssa, ga, mu0, cRd, cTd, cRs, cTs, cTdd);
+        fast rd = cRd, td = cTd, rs = cRs, ts = cTs, tdd = cTdd;
+        const fast f = uni(sfc[s]), tc = uni(stc[s]);
+        if (f > 0 && tc > 0) {
+          const fast t2 = tt + tc;
+          fast cw = cssa, cg = (fast)P.cloud_g;
+          if (t.cssa_i) {
+            const fast sl = sli[s], wl = sl * cssa, wi = (1 - sl) * cssa_i;
+            cw = wl + wi;
+            cg = cw > 0 ? fdiv(wl * (fast)P.cloud_g + wi * g_i, cw) : cg;
+          }
+          const fast sc2 = sc + cw * tc;
+          const fast g2 = fdiv(ga * sc + cg * cw * tc, sc2);
+          fast r1, t1, r2, t3, d1;
+          sw_layer(t2, fmin(fdiv(sc2, t2), (fast)(1 - 1e-6)), g2, mu0, r1, t1, r2, t3, d1);
+          rd = (1 - f) * cRd + f * r1;
+          td = (1 - f) * cTd + f * t1;
+          rs = (1 - f) * cRs + f * r2;
+          ts = (1 - f) * cTs + f * t3;
+          tdd = (1 - f) * cTdd + f * d1;
+        }
+        {
+          const fast cden = fquot(1, 1 - cAd * cRd);
+          const fast n = cRd + cTd * cTd * cAd * cden;
+          cAs = cRs + (cTdd * cAs + cTs * cAd) * cTd * cden;
+          cAd = n;
+        }
+        const fast den = fquot(1, 1 - Ad * rd), ta = td * den;
+        const fast cm = (rd * As * tdd + ts) * den;
+        const int k = s / NSUB, j = s % NSUB;
+        const int e = j == 0 ? 0 : j == NSUB - 1 ? 2 : 1;
+        if (e == 1 && j == 1) {                        // composed with the sub-level below it
+          mc[k][1] = ma[k][1] * cm + mc[k][1] * tdd;
+          ma[k][1] *= ta;
+          md[k][1] *= tdd;
+          pin(mc[k][1]); pin(ma[k][1]); pin(md[k][1]);
+        } else {
+          md[k][e] = tdd;
+          ma[k][e] = ta;
+          mc[k][e] = cm;
+          pin(mc[k][e]); pin(ma[k][e]); pin(md[k][e]);
+          if constexpr (IN_LDS) {
+            slot[2 * (3 * k + e)] = 1 - Ad;
+            slot[2 * (3 * k + e) + 1] = 1 - As;
+          } else {
+            nd[k][e] = 1 - Ad;
+            ns[k][e] = 1 - As;
+            pin(nd[k][e]); pin(ns[k][e]);
+          }
+        }
+        const fast nAd = rd + td * Ad * ta;
+        As = rs + (tdd * As + ts * Ad) * ta;
+        Ad = nAd;
+        pin(As); pin(Ad); pin(cAs); pin(cAd);
+      };
+      // (the mixed form's walk is unrolled by recursion at any length, the loop's own limit on size is below it; the FP64
+      // form's as far as the compiler goes, the rest of the maps then in scratch: 1.45 ms at 9,000 x 7 against 1.6 ms)
+      if constexpr (ISW_FORM_MIXED) {
+        down_from<NSS - 1>(walk);
+      } else {
 #pragma unroll
-      for (int c = 0; c < 7; c++) lk[c] = kbil(K + c * cs, NT, NG, fp, ft);
-      fast tg = fmax((fast)0, su[s][0] * (lk[0] + (lk[1] - lk[0]) * sfh[s]) + su[s][1] * lk[2] + su[s][2] * lk[3] +
-                                  su[s][3] * lk[4] + su[s][4] * lk[5] + su[s][5] * lk[6]);
-      if (t.cia) {
-        const float* C = t.cia + (size_t)sit[s] * NG + g;
-        tg += scia[s] * (C[0] + (C[NG] - C[0]) * ft);
+        for (int s = NSS - 1; s >= 0; s--) walk(s);
       }
-      return tg;
-    };
-    // bottom up: the gas optical depths, the clear sky's albedos (nothing kept) and the all-sky's. The FP64 form keeps
-    // each sub-level's gas depth for the way down; the mixed form looks the tables up again instead (measured at
-    // 7 layers: 243 VGPRs and two waves per SIMD against one, the pass 6.9 ms against 10.2 ms; in FP64 keeping wins)
-#if ISW_FORM_MIXED
-#define ISW_GAS_DOWN(s) gas(s)
-    fast Ad[NSS + 1], As[NSS + 1];
-#else
-#define ISW_GAS_DOWN(s) tgs[s]
-    fast tgs[NSS], Ad[NSS + 1], As[NSS + 1];
-#endif
-    Ad[NSS] = a;
-    As[NSS] = a;
-    fast cAd = a, cAs = a;
+      // top down: the nets at the edges, each layer's absorption, its top and bottom sub-level's, the surface's
+      fast Fdir = 1, Fdif = 0, net = 1 - As;
 #pragma unroll
-    for (int s = NSS - 1; s >= 0; s--) {
-      const fast tg = gas(s);
-#if !ISW_FORM_MIXED
-      tgs[s] = tg;
-#endif
-      fast cRd, cTd, cRs, cTs, cTdd, rd, td, rs, ts, tdd;
-      optics(s, tg, cRd, cTd, cRs, cTs, cTdd, rd, td, rs, ts, tdd);
-      {
-        const fast den = fdiv(1, 1 - cAd * cRd);
-        const fast nAd = cRd + cTd * cTd * cAd * den;
-        cAs = cRs + (cTdd * cAs + cTs * cAd) * cTd * den;
-        cAd = nAd;
+      for (int k = 0; k < L; k++) {
+        const fast top = net;
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+          Fdif = ma[k][e] * Fdif + mc[k][e] * Fdir;
+          Fdir *= md[k][e];
+          const int q = 2 * (3 * k + e);
+          if constexpr (IN_LDS) {
+            nd[k][e] = slot[q];
+            ns[k][e] = slot[q + 1];
+          }
+          const fast n2 = Fdir * ns[k][e] + Fdif * nd[k][e];
+          if (e != 1) slot[q] = (float)(wg * (net - n2));
+          net = n2;
+        }
+        slot[2 * (3 * k + 2) + 1] = (float)(wg * (top - net));
       }
-      const fast den = fdiv(1, 1 - Ad[s + 1] * rd);
-      Ad[s] = rd + td * td * Ad[s + 1] * den;
-      As[s] = rs + (tdd * As[s + 1] + ts * Ad[s + 1]) * td * den;
+      slot[2] = (float)(wg * net);
+      slot[3] = (float)(wg * cAs);
     }
-    // top down: the fluxes, each layer's absorption, its top and bottom sub-level's, the surface's
-    const fast wg = t.sun[g];
-    fast Fdir = 1, Fdif = 0, net = 1 - As[0], absk = 0;
-#pragma unroll
-    for (int s = 0; s < NSS; s++) {
-      fast cRd, cTd, cRs, cTs, cTdd, rd, td, rs, ts, tdd;
-      optics(s, ISW_GAS_DOWN(s), cRd, cTd, cRs, cTs, cTdd, rd, td, rs, ts, tdd);
-#undef ISW_GAS_DOWN
-      const fast den = fdiv(1, 1 - Ad[s + 1] * rd);
-      const fast Fdn = Fdir * tdd;
-      Fdif = (td * Fdif + rd * As[s + 1] * Fdn + ts * Fdir) * den;
-      Fdir = Fdn;
-      const fast n2 = Fdir + Fdif - (Ad[s + 1] * Fdif + As[s + 1] * Fdir);
-      const int k = s / NSUB;
-      if (s % NSUB == 0) absk = 0;
-      absk += net - n2;
-      if (s % NSUB == 0) RED(L + 2 + 2 * k, wg * (net - n2));
-      if (s % NSUB == NSUB - 1) {
-        RED(L + 3 + 2 * k, wg * (net - n2));
-        RED(k, wg * absk);
-      }
-      net = n2;
-    }
-    RED(L, wg * net);
-    RED(L + 1, wg * cAs);
-  } else {
-    for (int r = 0; r < ROWS; r++) RED(r, 0.f);
+    __syncthreads();
+    g_sums<6 * L, S>(red, (int)NG, [&](int q, double v) {
+      const int k = q / 6, m = q - 6 * k;              // (layer, slot: 0 the top sub-level's, 4 the bottom's, 5 its own)
+      const int r = m == 0 ? L + 2 + 2 * k : m == 4 ? L + 3 + 2 * k : m == 5 ? k : k == 0 && m >= 2 ? L + m - 2 : -1;
+      if (r >= 0) swf[(size_t)r * N + i] = v;
+    });
+    if (i + 1 < i1) stage(i + 1);
+    __syncthreads();
   }
-#undef RED
-  __syncthreads();
-  g_sums<ROWS>(red, ngp, sums);
-  __syncthreads();
-  if (g < ROWS) swf[(size_t)g * N + i] = sums[g];
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -604,14 +834,14 @@ static inline int ngpad(int NG) { return (NG + 63) / 64 * 64; }
 
 #define ISW_BY_L(CALL)                                                                                   \
   switch (L) {                                                                                           \
-    case 1: CALL(1); break;                                                                              \
-    case 2: CALL(2); break;                                                                              \
-    case 3: CALL(3); break;                                                                              \
-    case 4: CALL(4); break;                                                                              \
-    case 5: CALL(5); break;                                                                              \
-    case 6: CALL(6); break;                                                                              \
-    case 7: CALL(7); break;                                                                              \
-    case 8: CALL(8); break;                                                                              \
+    case 1: { CALL(1); } break;                                                                              \
+    case 2: { CALL(2); } break;                                                                          \
+    case 3: { CALL(3); } break;                                                                          \
+    case 4: { CALL(4); } break;                                                                          \
+    case 5: { CALL(5); } break;                                                                          \
+    case 6: { CALL(6); } break;                                                                          \
+    case 7: { CALL(7); } break;                                                                          \
+    case 8: { CALL(8); } break;                                                                          \
     default: return ISW_EBADARG;                                                                         \
   }
 
@@ -634,13 +864,15 @@ int lw_column(int N, int L, const double* par, const isw_lw_tables* t, const flo
               double* radf, hipStream_t st) {
   const RadP P = make_radp(par);
   const int ngp = ngpad(t->NG), rows = 3 * (L + 1) + 3 + 6 * L;
-  const size_t shm = (size_t)rows * ngp * sizeof(float);
+  const int cpb = cols_per_block(N);
+  const unsigned nb = (unsigned)((N + cpb - 1) / cpb);
   const double bytes = (double)NSUB * L * NVP * N * 4 + (double)N * 8 + (double)rows * N * 8 +
                        (double)t->NC * t->NP * t->NT * t->NG * 4 + (double)t->NTP * t->NG * 4;
+  // (at most 54 KB of LDS, at eight layers)
 #define CALL(LL)                                                                                              \
-  if (shm > 65536) hipFuncSetAttribute((const void*)k_lw_column<LL>, hipFuncAttributeMaxDynamicSharedMemorySize,    \
-                                       (int)shm);                                                                   \
-  ISW_LAUNCH_SHM("lw_column", bytes, k_lw_column<LL>, dim3((unsigned)N), dim3((unsigned)ngp), shm, N, P, *t, sub, Ts, radf)
+  const size_t shm = (size_t)LwRows<LL>::S * ngp * sizeof(float);                                                    \
+  ISW_LAUNCH_SHM("lw_column", bytes, k_lw_column<LL>, dim3(nb), dim3((unsigned)ngp), shm, N, cpb, P, *t, sub, Ts, \
+                 radf)
   ISW_BY_L(CALL)
 #undef CALL
   return (int)hipGetLastError();
@@ -651,12 +883,14 @@ int sw_column(int N, int L, const double* par, const isw_sw_tables* t, const isw
               double* swf, hipStream_t st) {
   const RadP P = make_radp(par);
   const int ngp = ngpad(t->NG), rows = 3 * L + 2;
-  const size_t shm = (size_t)rows * ngp * sizeof(float);
+  const size_t shm = (size_t)(6 * L + 1) * ngp * sizeof(float);
+  const int cpb = cols_per_block(N);
+  const unsigned nb = (unsigned)((N + cpb - 1) / cpb);
   const double bytes = (double)NSUB * L * NVP * N * 4 + (double)N * 8 * (1 + (mode == 0 ? 3 : 0)) +
                        (cloudo ? 3.0 * L * N * 8 : 0) + (double)rows * N * 8 + (double)t->NC * t->NP * t->NT * t->NG * 4;
 #define CALL(LL)                                                                                              \
-  ISW_LAUNCH_SHM("sw_column", bytes, k_sw_column<LL>, dim3((unsigned)N), dim3((unsigned)ngp), shm, N, P, *t, *air, \
-                 sub, mode, tnow, interval, pos, alb, cloudo, swf)
+  ISW_LAUNCH_SHM("sw_column", bytes, k_sw_column<LL>, dim3(nb), dim3((unsigned)ngp), shm, N, cpb, P, *t, *air, sub, \
+                 mode, tnow, interval, pos, alb, cloudo, swf)
   ISW_BY_L(CALL)
 #undef CALL
   return (int)hipGetLastError();

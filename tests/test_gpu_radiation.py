@@ -162,3 +162,21 @@ def test_full_workload_size():
         assert np.array_equal(radf, radf2) and np.array_equal(swf, swf2) and np.array_equal(sub, sub2)
         _, _, swc = run_gpu(c, pos, par, L, lwk, swk, prec, clouds=False)
         assert np.allclose(swc[:L].sum(0) + swc[L] + swc[L + 1], 1.0, atol=2e-5)
+
+
+@pytest.mark.parametrize('N,L,lwb,swb', [(1, 2, 4, 4), (257, 3, 5, 3), (6145, 4, 1, 1), (67, 6, 15, 13), (65, 8, 16, 16)])
+def test_columns_at_the_edges(N, L, lwb, swb):
+    """One column, an odd number of them shared out two to a block, one and several waves of g-points (a last one part
+    full, a full block), the layer counts whose sums go through LDS in two parts or whose albedos wait there: both forms
+    against the oracle on the same sub-levels, at the bars above."""
+    from insilica.ktables import synthetic_lw, synthetic_sw
+    print(f'case: radiation N={N} L={L} {16 * lwb} / {16 * swb} g-points', flush=True)
+    c, pos, par = case(N, L, 20 + L)
+    lwk, swk = synthetic_lw(bands=lwb, seed=L), synthetic_sw(bands=swb, seed=L + 1)
+    for prec, tol in (('double', 1e-8), ('mixed', 1e-4)):
+        sub, radf, swf = run_gpu(c, pos, par, L, lwk, swk, prec)
+        ora, osw = run_oracle(c, pos, par, L, lwk, swk, sub)
+        e_lw = np.max(np.abs(radf - ora) / lw_scale(ora, L))
+        e_sw = np.max(np.abs(swf - osw))
+        print(f'{prec}: lw {e_lw:.2e} sw {e_sw:.2e}', flush=True)
+        assert e_lw <= tol and e_sw <= tol
