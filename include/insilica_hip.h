@@ -36,8 +36,8 @@ extern "C" {
 #define ISW_EBADARG 9001
 #define ISW_LMAX 8
 #define ISW_KSOIL 16
-#define ISW_PAIR_THREADS 256 /* threads per block of the two-sub-step patch kernel: the most edges a patch may own,
-                              * and the most cells of patch and halo */
+#define ISW_PAIR_THREADS 256 /* with the ph2_* tables, the most edges a patch may own and the most cells of patch and
+                              * halo */
 
 /* The mesh on the device (reference: src/insilica/gpu.py:55-80 DeviceGrid; tables from src/insilica/grid/trisk.py).
  * rA, rde, rAV: 1/areaCell, 1/de, 1/areaV; wf, d2wtf: FP32 copies of w and d2wt (read by the mixed form only).
@@ -49,21 +49,21 @@ typedef struct isw_grid {
   const double *le, *de, *areaCell, *areaV, *fV, *kite, *w, *d2wt;
   const double *rA, *rde, *rAV;
   const float *wf, *d2wtf;
-  /* Patches for the air's fast sub-steps in one launch each (optional: ph_off NULL keeps two launches per sub-step;
-   * no counterpart in the reference). Patch b (of npatch) holds the cells [b pcells, (b + 1) pcells); its halo cells
+  /* Patches of consecutive cells (optional; no counterpart in the reference): the transport's fused passes read their
+   * edge lists, with pi_* below. Patch b (of npatch) holds the cells [b pcells, (b + 1) pcells); its halo cells
    * (the second cells of its edges outside it) ph_cell[ph_off[b] .. ph_off[b + 1]); its edges (those whose first cell
    * eI is in it) pe_edge[pe_off[b] .. pe_off[b + 1]), each with its cells' slots pe_slot = sI | sJ << 16 (a cell of
    * the patch at its offset in it, a halo cell at pcells + its index in the halo); pslots: the most slots a patch uses;
    * pown: the most edges a patch owns (max of pe_off[b + 1] - pe_off[b]). */
   int32_t npatch, pcells, pslots, pown;
   const int32_t *ph_off, *ph_cell, *pe_off, *pe_edge, *pe_slot;
-  /* Two air fast sub-steps per launch on the same patches (optional: ph2_off NULL keeps one per launch). The first
-   * sub-step's cells: patch, halo and the halo's halo ph2_cell[ph2_off[b] ..] (slots after the halo's); its winds on
+  /* Two air fast sub-steps per launch on the same patches (optional; checked when given, but no kernel reads these
+   * tables now: the rg_* tables below take their place). The first sub-step's cells: patch, halo and the halo's halo ph2_cell[ph2_off[b] ..] (slots after the halo's); its winds on
    * every edge of patch and halo: the patch's edges (slots 0 .. ne - 1) and px_edge[px_off[b] ..] (slots from ne),
    * with their cells' slots px_slot (as pe_slot); pc_eslot[3 pc_off[b] ..]: each patch-then-halo cell's six edge
-   * slots, two per int32 (0xffff: no edge); pslots2, pedges2: the most cell and edge slots a patch uses. The pair
-   * kernel steps each owned edge on its own thread of a 256-thread block, so these tables are refused (ISW_EBADARG)
-   * when a patch owns more than 256 edges (pown > 256) or its patch and halo hold more than 256 cells (pslots > 256). */
+   * slots, two per int32 (0xffff: no edge); pslots2, pedges2: the most cell and edge slots a patch uses. Refused
+   * (ISW_EBADARG) when a patch owns more than 256 edges (pown > 256) or its patch and halo hold more than 256 cells
+   * (pslots > 256). */
   int32_t pslots2, pedges2;
   const int32_t *ph2_off, *ph2_cell, *px_off, *px_edge, *px_slot, *pc_off, *pc_eslot;
   /* The transport's fused flux-and-stage passes on the same patches (optional: pi_off NULL keeps a flux pass and a
@@ -73,9 +73,21 @@ typedef struct isw_grid {
    * ptedges: the most edges a patch uses (ne + its incoming edges). */
   int32_t ptedges, pad3_;
   const int32_t *pi_off, *pi_edge, *tc_slot;
-  /* eslot (E x 2): each edge's slot in its first and its second cell's cellEdge ring (required with ph_off: the
-   * stage's coefficients are written at those slots) */
+  /* eslot (E x 2): each edge's slot in its first and its second cell's cellEdge ring (required with ph_off) */
   const int8_t *eslot;
+  /* The fast sub-steps' patches (optional: rg_head NULL steps them one per pass over the mesh): compact patches of
+   * cells with rg_k (1 to 5) rings of neighbours, on which up to rg_k sub-steps run in one launch. Patch b's record
+   * rg_head[16 b ..]: its first entry in rg_cell (and, times 3, in rg_slot) and in rg_edge (and rg_ecell), the edges it
+   * owns, the cells within ring 0 .. rg_k, the edges touching those. rg_cell: its cells, ring by ring; rg_slot: per
+   * cell its six edges' places in the patch's edge list in cellEdge order, two to an int32, with 0x8000 set for a
+   * negative cellSign and 0x7fff for no edge; rg_edge: the owned edges (whose first cell is the patch's own), then the
+   * others ring by ring; rg_ecell: the places of an edge's first | second << 16 cell in the patch's cell list (not read
+   * for edges that touch ring rg_k only). rg_npatch patches; rg_owned: the most edges one owns; rg_cells, rg_edges: per ring,
+   * the most cells and edges one has within it. In a batch a patch's cells are of one world. (csrc/mesh.cpp
+   * isw_mesh_rings builds them.) */
+  int32_t rg_k, rg_npatch, rg_owned, pad4_;
+  int32_t rg_cells[6], rg_edges[6];
+  const int32_t *rg_head, *rg_cell, *rg_slot, *rg_edge, *rg_ecell;
 } isw_grid;
 
 /* A batch of worlds stepped together on one mesh: the disjoint union of the worlds' meshes (all of one level, so of
@@ -119,9 +131,9 @@ typedef struct isw_layers {
    * times |u| from the edge's normal and TRiSK tangential winds). */
   const double *tide, *cbot;
   double cd_bot;
-  /* The air's fast sub-steps' coefficients per cell slot and layer, sign * l_e * h_e at [(layer * N + cell) * 6 +
-   * slot] (L*N*6), written once per stage with the edge thicknesses: cfc (doubles, plain FP64 form) or cfcf (floats,
-   * mixed form); the form's one is required for air layers when the grid has patch tables. */
+  /* The air's fast sub-steps' flux coefficients l_e * h_e per edge and layer (L, E), written once per stage with the
+   * edge thicknesses: cfc (doubles, plain FP64 form) or cfcf (floats, mixed form); the form's one is required for air
+   * layers when the grid has patch or ring tables. */
   double *cfc;
   float *cfcf;
 } isw_layers;

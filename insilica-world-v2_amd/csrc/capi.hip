@@ -93,7 +93,7 @@ bool grid_ok(const isw_grid* g) {
   if (!(g && g->N > 0 && g->E > 0 && g->NV > 0 && g->eI && g->eJ && g->cellEdge && g->cellEdgeAsc && g->cellSign &&
         g->le && g->de && g->areaCell))
     return false;
-  // the fast sub-steps' patches, when given: every table, a patch count that covers the cells, slots for a patch
+  // the patches of consecutive cells, when given: every table, a patch count that covers the cells, slots for a patch
   if (g->ph_off && !(g->ph_cell && g->pe_off && g->pe_edge && g->pe_slot && g->eslot && g->pcells > 0 &&
                      g->npatch == (g->N + g->pcells - 1) / g->pcells && g->pslots >= g->pcells &&
                      g->pslots < (1 << 15) && g->pown > 0))
@@ -101,8 +101,15 @@ bool grid_ok(const isw_grid* g) {
   // the transport's fused stages: their incoming edges, each cell's slots, the most edges a patch uses
   if (g->pi_off && !(g->ph_off && g->pi_edge && g->tc_slot && g->ptedges > 0 && g->ptedges < (1 << 14)))
     return false;
-  // the pair kernel's patches: one thread of its ISW_PAIR_THREADS-thread block per owned edge, and per cell of patch
-  // and halo (at most pslots of them)
+  // the ring tables: every table, a depth the patch records hold, a patch and its rings not empty
+  if (g->rg_head && !(g->rg_cell && g->rg_slot && g->rg_edge && g->rg_ecell && g->rg_k >= 1 && g->rg_k <= 5 &&
+                      g->rg_npatch > 0 && g->rg_owned > 0))
+    return false;
+  for (int r = 0; g->rg_head && r <= g->rg_k; r++)
+    if (g->rg_cells[r] < 1 || g->rg_edges[r] < g->rg_owned || g->rg_cells[r] >= 0x7fff || g->rg_edges[r] >= 0x7fff)
+      return false;
+  // the two-sub-step patches (no kernel reads them now; what was refused stays refused): at most ISW_PAIR_THREADS owned
+  // edges, and as many cells of patch and halo (at most pslots of them)
   return !g->ph2_off || (g->ph_off && g->ph2_cell && g->px_off && g->px_edge && g->px_slot && g->pc_off &&
                          g->pc_eslot && g->pslots2 >= g->pslots && g->pslots2 < (1 << 15) && g->pedges2 > 0 &&
                          g->pedges2 < 0xffff && g->pown <= ISW_PAIR_THREADS && g->pslots <= ISW_PAIR_THREADS);
@@ -112,8 +119,8 @@ bool layers_ok(const isw_grid* g, const isw_layers* s) {
   if (!grid_ok(g) || !s || s->L < 1 || s->L > ISW_LMAX) return false;
   if (s->prec != ISW_FP64 && s->prec != ISW_MIXED) return false;
   if (s->prec == ISW_MIXED && (!s->pkf || !g->wf || !g->rA || !g->rde || !g->rAV)) return false;
-  // (the patch kernels read the stage's coefficients per cell slot)
-  if (s->air && g->ph_off && (s->prec == ISW_MIXED ? !s->cfcf : !s->cfc)) return false;
+  // (the fast sub-steps' kernels read the stage's flux coefficients)
+  if (s->air && (g->ph_off || g->rg_head) && (s->prec == ISW_MIXED ? !s->cfcf : !s->cfc)) return false;
   if (s->prec == ISW_FP64 && !s->pk) return false;
   const isw_batch* b = s->batch;
   if (b && (b->nworlds < 1 || !b->wc || !b->we || !b->nsub || !b->grav || !b->nu4 || !b->tau || !b->inv_n ||

@@ -8,7 +8,8 @@
 // Design (MI355X): one thread per cell, edge or vertex, 256-thread blocks (four 64-wide waves), layer-major arrays so
 // consecutive threads touch consecutive words. The reference's one-kernel-per-loop structure is fused wherever a
 // value can be recomputed bit for bit instead of stored and re-read: the Bernoulli (cell) and PV (vertex) passes run
-// in one launch; the air fast sub-steps read the stage's start state directly (no copies); the stage flux
+// in one launch; the fast sub-steps run several to a launch on patches with rings of neighbours (k_af_rings, k_bt_rings),
+// read the stage's start state directly (no copies) and keep it in registers and LDS between them; the stage flux
 // F = h_e * mean(u) is recomputed inside the limiter and the divergence instead of being stored, the limited
 // flux's volume Fm is written by each edge's eI cell, and the wall mask is applied inside the kernels that write.
 // Every sum keeps the reference's order (a cell's edges in cellEdge or cellEdgeAsc order, a vertex's three in table
@@ -17,6 +18,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "insilica_hip.h"
 #include "diag.hpp"
@@ -65,19 +67,6 @@ __device__ __forceinline__ void ring6(const int* __restrict__ tab, int i, int (&
   e[0] = a.x; e[1] = a.y; e[2] = b.x; e[3] = b.y; e[4] = c.x; e[5] = c.y;
 }
 __device__ __forceinline__ int ok0(int e) { return e < 0 ? 0 : e; }
-
-// A cell's six per-slot coefficients of one layer (contiguous, 16-byte aligned as doubles, 8-byte as floats), in
-// three vector loads.
-__device__ __forceinline__ void load6(const double* p, double (&c)[6]) {
-  const double2* q = reinterpret_cast<const double2*>(p);
-  const double2 a = q[0], b = q[1], d = q[2];
-  c[0] = a.x; c[1] = a.y; c[2] = b.x; c[3] = b.y; c[4] = d.x; c[5] = d.y;
-}
-__device__ __forceinline__ void load6(const float* p, double (&c)[6]) {
-  const float2* q = reinterpret_cast<const float2*>(p);
-  const float2 a = q[0], b = q[1], d = q[2];
-  c[0] = a.x; c[1] = a.y; c[2] = b.x; c[3] = b.y; c[4] = d.x; c[5] = d.y;
-}
 
 // Settings of a layer stack passed by value (reference: Layers.__init__, src/insilica/layers.py:161-218).
 struct LP {
@@ -367,14 +356,7 @@ __global__ __launch_bounds__(BS) void k_edge_hq(isw_grid g, int L, double shelf,
   const double hv = edge_h(h[(size_t)l * N + g.eI[e]], h[(size_t)l * N + g.eJ[e]], shelf);
   const double qv = 0.5 * (q[(size_t)l * NV + g.ev1[e]] + q[(size_t)l * NV + g.ev2[e]]);
   he[t] = hv;
-  if (cf) {
-    // the air's fast sub-steps' coefficient sign * l_e * h_e at this edge's slot in each of its two cells (the
-    // product the mass step forms, in its order: (sign * l_e) * h_e)
-    const int a = g.eI[e], c = g.eJ[e], sa = g.eslot[2 * e], sc = g.eslot[2 * e + 1];
-    const double le = g.le[e];
-    cf[((size_t)l * N + a) * 6 + sa] = (fast)((double)g.cellSign[a * 6 + sa] * le * hv);
-    cf[((size_t)l * N + c) * 6 + sc] = (fast)((double)g.cellSign[c * 6 + sc] * le * hv);
-  }
+  if (cf) cf[t] = (fast)(g.le[e] * hv);          // (the air's fast sub-steps' flux coefficient)
   fast* pp = pk + ((size_t)e * L + l) * 3;
   pp[0] = (fast)hv; pp[1] = (fast)u[t]; pp[2] = (fast)qv;
 }
@@ -566,439 +548,322 @@ __global__ __launch_bounds__(BS) void k_af_u(isw_grid g, int L, Div dv, LP p, in
   (sb.last ? un : uf)[t] = v + sb.tau * (DIVBY(-(pl[g.eJ[e]] - pl[g.eI[e]]), dv.de[e]) + Tp[t] + G[e]);
 }
 
-// One air fast sub-step in one launch, on patches of consecutive (Hilbert-ordered, so compact) cells: each block
-// takes the mass step and Phi* of its patch's cells and of the halo cells across its edges (the halo's recomputed
-// from the same inputs, so every copy is the same to the bit), keeps Phi* in LDS, then steps the wind on the edges
-// whose first cell is in the patch. The arithmetic is k_af_muphi's and k_af_u's in their order. Masses and winds
-// alternate between two buffers (a neighbour block may still read this sub-step's inputs), so in/out never alias.
-// Patch tables (isw_grid): patch b holds cells [b pcells, (b + 1) pcells), its halo cells ph_cell[ph_off[b] ..],
-// its edges pe_edge[pe_off[b] ..] with their cells' LDS slots pe_slot (first | second << 16; halo slots from pcells).
-constexpr int FBS = ISW_PAIR_THREADS;
-template <int L>
-__global__ __launch_bounds__(FBS) void k_af_patch(isw_grid g, LP p, Div dv, int stage, int it, int n, double tau,
+// ---------------------------------------------------------------------------------------------------------------
+// Several fast sub-steps in one launch, on the grid's patches (tables rg_*): a block holds its patch's cells and the
+// rings of neighbours within m cells of it, takes the state of all of them in registers once, and steps m times. The
+// first step's masses are those of every ring, and each further step's reach one ring less, so the m-th step's are the
+// patch's own; what neighbours recompute they compute from the same inputs in the same order, so every copy is the same to
+// the bit. Between the steps only LDS is touched: the edges' threads leave each flux coef * u there, the cells' threads
+// leave each potential. So a launch pays its chain of dependent loads (arguments, the patch's record, the index lists,
+// the values) once for m steps, about 6 us of it before the first step at level 6 (three layers, mixed: 7.7 us for one
+// step, 9.4 for two, 11.2 for three); what bounds each further step is LDS: six fluxes per cell, two potentials per edge. Two buffers alternate for masses and winds, as a neighbour block may still read a launch's
+// inputs. A patch's cells are of one world, so a batch's counts and lengths are the block's.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int RBS = 256;
+// The sub-steps a launch takes. Air: 3 (level 6, three layers, nfast 15, the 28 sub-steps of a step: 216 us at one per
+// launch, 140 at two, 112 at three; at four a patch needs two cells and four edges to a thread, 190 registers and two
+// blocks per CU: 125 us. 384 threads with one cell each at five: 113 us). Ocean (one value per cell): 4 (level 7, 70
+// sub-steps: 815 us at one, 535 at two, 528 at three, 498 at four; five need five edges to a thread and gain nothing).
+constexpr int AIR_STEPS = 3, SEA_STEPS = 4;
+
+struct Ring {
+  int c0, e0, own;                                 // the patch's first entries in the lists, its owned edges
+  const int* head;
+  int k;
+  __device__ __forceinline__ int cells(int r) const { return head[3 + r]; }
+  __device__ __forceinline__ int edges(int r) const { return head[4 + k + r]; }
+};
+__device__ __forceinline__ Ring ring_of(const isw_grid& g) {
+  const int* h = g.rg_head + 16 * (size_t)xblock();
+  return Ring{h[0], h[1], h[2], h, g.rg_k};
+}
+// A batch's sub-steps left to this launch (at most m) and their length, for the block's world.
+__device__ __forceinline__ bool ring_sub(const LP& p, int cell, int stage, int it0, int n, int& m, double& tau,
+                                         bool& last) {
+  if (p.wc) {
+    const int w = p.wc[cell];
+    n = p.wn[w * 3 + stage];
+    tau = p.wtau[w * 3 + stage];
+  }
+  m = min(m, n - it0);
+  last = it0 + m == n;
+  return m > 0;
+}
+// A cell's six edges in the fluxes left in LDS: their places (in cellEdge order; a missing edge's is `none`, which holds
+// 0) and the signs of the cell on them, as the sign bit to flip.
+struct RingCell {
+  int at[6];
+  unsigned flip[6];
+  __device__ __forceinline__ void set(const int* __restrict__ s, int none) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const unsigned w = (unsigned)s[k];
+      const int q0 = (int)(w & 0x7fffu), q1 = (int)(w >> 16 & 0x7fffu);
+      at[2 * k] = q0 == 0x7fff ? none : q0;
+      at[2 * k + 1] = q1 == 0x7fff ? none : q1;
+      flip[2 * k] = (w & 0x8000u) << 16;
+      flip[2 * k + 1] = w & 0x80000000u;
+    }
+  }
+  __device__ __forceinline__ double div(const double* F) const {
+    double t[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      const double f = F[at[k]];
+      t[k] = __hiloint2double((int)((unsigned)__double2hiint(f) ^ flip[k]), __double2loint(f));
+    }
+    return ((((t[0] + t[1]) + t[2]) + t[3]) + t[4]) + t[5];
+  }
+};
+// x / d with r = 1 / d at hand: the plain form's rounds as the division does (a quotient corrected by its exact
+// remainder), the mixed form's is the product (its Div holds reciprocals).
+__device__ __forceinline__ double over(double x, double d, double r) {
+#if ISW_FORM_MIXED
+  return x * d;
+#else
+  const double q = x * r;
+  return __builtin_fma(__builtin_fma(-q, d, x), r, q);
+#endif
+}
+__device__ __forceinline__ double recip(double d) {
+#if ISW_FORM_MIXED
+  return d;
+#else
+  return 1.0 / d;
+#endif
+}
+
+// The air's: EPT edges and CPT cells to a thread.
+template <int L, int EPT, int CPT>
+__global__ __launch_bounds__(RBS) void k_af_rings(isw_grid g, LP p, Div dv, int stage, int it0, int m, int n, double tau,
                                                   const fast* __restrict__ coef, const double* __restrict__ uin,
                                                   const double* __restrict__ mu_src, double* __restrict__ mu_out,
                                                   const double* __restrict__ S, const double* __restrict__ Tp,
                                                   const double* __restrict__ G, double* __restrict__ acc,
                                                   double* __restrict__ uout, double* __restrict__ un) {
-  extern __shared__ double sphi[];                 // [L][pslots]
-  const int N = g.N, E = g.E, PC = g.pcells, PS = g.pslots;
-  const int b = xblock();
-  const int c0 = b * PC, nown = min(PC, N - c0);
-  const int h0 = g.ph_off[b], nh = g.ph_off[b + 1] - h0;
-  const int e0 = g.pe_off[b], ne = g.pe_off[b + 1] - e0;
-  // the wind step's inputs for this thread's first edge, loaded before the mass step so their latency overlaps it
-  // (they do not depend on it); further edges, if a patch has more than FBS, load in the loop below
-  const int q0 = threadIdx.x;
-  int e_ = 0, sl_ = 0;
-  Sub sbe{false, false, 0.0};
-  double v_[L], a_[L], tp_[L], rde_ = 0, G_ = 0;
-  if (q0 < ne) {
-    e_ = g.pe_edge[e0 + q0];
-    sl_ = g.pe_slot[e0 + q0];
-    sbe = sub_at(p, p.we, e_, stage, it, n, tau);
-    if (sbe.active) {
-      rde_ = dv.de[e_];
-      G_ = G[e_];
-#pragma unroll
-      for (int l = 0; l < L; l++) {
-        const size_t t = (size_t)l * E + e_;
-        v_[l] = uin[t];
-        a_[l] = it == 0 ? 0.0 : acc[t];
-        tp_[l] = Tp[t];
-      }
-    }
-  }
-  for (int s = threadIdx.x; s < nown + nh; s += FBS) {
-    const int i = s < nown ? c0 + s : g.ph_cell[h0 + s - nown];
-    const int slot = s < nown ? s : PC + (s - nown);
-    const Sub sb = sub_at(p, p.wc, i, stage, it, n, tau);
-    if (!sb.active) continue;
-    int e[6];
-    ring6(g.cellEdge, i, e);
-    double m1k[L], sak[L];
-#pragma unroll
-    for (int k = 0; k < L; k++) {
-      double c6[6];                                // (sign * l_e * h_e per slot, written with the stage's h_e)
-      load6(coef + ((size_t)k * N + i) * 6, c6);
-      const double* ul = uin + (size_t)k * E;
-      double t[6];
-#pragma unroll
-      for (int m = 0; m < 6; m++) t[m] = c6[m] * ul[ok0(e[m])];
-      double div = 0;
-#pragma unroll
-      for (int m = 0; m < 6; m++)
-        if (e[m] >= 0) div += t[m];
-      const double m0 = mu_src[(size_t)k * N + i];
-      const double m1 = m0 - DIVBY(sb.tau * div, dv.A[i]);
-      m1k[k] = m1;
-      sak[k] = m1 + p.div_damp * (m1 - m0);
-    }
-    double P[L], Sk[L];
-    double a = 0;
-#pragma unroll
-    for (int m = 0; m < L; m++) {
-      a += sak[m];
-      P[m] = a;
-      Sk[m] = S[(size_t)m * N + i];
-    }
-#pragma unroll
-    for (int k = 0; k < L; k++) {
-      double ph = 0;
-#pragma unroll
-      for (int m = L - 1; m >= k; m--) ph += Sk[m] * P[m];
-      sphi[k * PS + slot] = ph;
-      if (s < nown) mu_out[(size_t)k * N + i] = m1k[k];
-    }
-  }
-  __syncthreads();
-  if (q0 < ne && sbe.active) {
-    const int sI = sl_ & 0xffff, sJ = sl_ >> 16;
-    double* out = sbe.last ? un : uout;
-#pragma unroll
-    for (int l = 0; l < L; l++) {
-      const size_t t = (size_t)l * E + e_;
-      acc[t] = it == 0 ? 0.0 + v_[l] : a_[l] + v_[l];
-      out[t] = v_[l] + sbe.tau * (DIVBY(-(sphi[l * PS + sJ] - sphi[l * PS + sI]), rde_) + tp_[l] + G_);
-    }
-  }
-  for (int q = q0 + FBS; q < ne; q += FBS) {
-    const int e = g.pe_edge[e0 + q];
-    const Sub sb = sub_at(p, p.we, e, stage, it, n, tau);
-    if (!sb.active) continue;
-    const int sl = g.pe_slot[e0 + q];
-    const int sI = sl & 0xffff, sJ = sl >> 16;
-    const double rde = dv.de[e], Ge = G[e];
-    double* out = sb.last ? un : uout;
-#pragma unroll
-    for (int l = 0; l < L; l++) {
-      const size_t t = (size_t)l * E + e;
-      const double v = uin[t];
-      acc[t] = it == 0 ? 0.0 + v : acc[t] + v;
-      out[t] = v + sb.tau * (DIVBY(-(sphi[l * PS + sJ] - sphi[l * PS + sI]), rde) + Tp[t] + Ge);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------------------------
-// Ocean barotropic sub-steps (layers.cu:366-388) with the wall mask of the reference's lay_mask calls fused in.
-// ---------------------------------------------------------------------------------------------------------------
-// Two air fast sub-steps (it, it + 1) in one launch on the grid's patches (tables ph2_*, px_*, pc_*): A) the mass
-// step and Phi* of every cell of the patch's edges' cells' edges (patch, halo, the halo's halo); B) the wind of
-// sub-step it on every edge of patch and halo, in LDS; C) the mass step and Phi* of sub-step it + 1 on patch and
-// halo from B's winds; D) the wind of sub-step it + 1 on the patch's edges. Every value is computed as k_af_muphi and
-// k_af_u compute it, so the result is the same to the bit as two sub-steps of one launch each.
-// Latency: the kernel is a chain of dependent gathers (table -> edge -> value) between three barriers, with ~2.5
-// waves per SIMD at level 6, so only A gathers: thread q loads its own edge's inputs (B, D) and the q-th halo edge's
-// (B) before A, and A leaves each patch-and-halo cell's coefficients sign * l_e * h_e per layer in LDS (cf, L <= 4)
-// with its stiffness and area in registers (patch and halo come first in A's order, so thread q does cell q in both),
-// so that C reads no global memory. Halo edges past the block's FBS threads (a few at level 6) load as they go.
-template <int L>
-__global__ __launch_bounds__(FBS) void k_af_patch2(isw_grid g, LP p, Div dv, int stage, int it, int n, double tau,
-                                                   const fast* __restrict__ coef, const double* __restrict__ uin,
-                                                   const double* __restrict__ mu_src, double* __restrict__ mu_out,
-                                                   const double* __restrict__ S, const double* __restrict__ Tp,
-                                                   const double* __restrict__ G, double* __restrict__ acc,
-                                                   double* __restrict__ uout, double* __restrict__ un) {
-  constexpr bool CF = L <= 4;                      // C's coefficients from LDS (else C gathers them again)
   extern __shared__ double sm[];
-  const int N = g.N, E = g.E, PC = g.pcells, PS = g.pslots2, PE = g.pedges2, P1 = g.pslots;
-  double* phiA = sm;                               // [L][PS] Phi* of sub-step it
-  double* muA = phiA + L * PS;                     // [L][PS] the masses after it (patch and halo)
-  double* uB = muA + L * PS;                       // [L][PE] the winds after it
-  double* phiC = uB + L * PE;                      // [L][PS] Phi* of sub-step it + 1
-  double* cfs = phiC + L * PS;                     // [L][6][P1] (CF) the coefficients of patch and halo cells
-  const int b = xblock();
-  const int c0 = b * PC, nown = min(PC, N - c0);
-  const int h0 = g.ph_off[b], nh = g.ph_off[b + 1] - h0;
-  const int k0 = g.ph2_off[b], nk = g.ph2_off[b + 1] - k0;
-  const int e0 = g.pe_off[b], ne = g.pe_off[b + 1] - e0;
-  const int x0 = g.px_off[b], nx = g.px_off[b + 1] - x0;
-  const int nC = nown + nh;                        // <= P1 <= FBS (checked with the tables on the host)
-  const int q0 = threadIdx.x;
-  // this thread's own edge (if any): its inputs for B and D
-  int eo = 0, slo = 0;
-  Sub s1{false, false, 0.0}, s2{false, false, 0.0};
-  double v_[L], a_[L], tp_[L], rde_ = 0, G_ = 0;
-  if (q0 < ne) {
-    eo = g.pe_edge[e0 + q0];
-    slo = g.pe_slot[e0 + q0];
-    s1 = sub_at(p, p.we, eo, stage, it, n, tau);
-    s2 = sub_at(p, p.we, eo, stage, it + 1, n, tau);
-    if (s1.active) {
-      rde_ = dv.de[eo];
-      G_ = G[eo];
+  constexpr int PE = EPT * RBS + 2, PC = CPT * RBS;
+  const int N = g.N, E = g.E, t = (int)threadIdx.x;
+  double* F = sm;                                  // [L][PE] coef * u, the last but one 0
+  double* phi = sm + L * PE;                       // [L][PC] Phi*
+  const Ring r = ring_of(g);
+  bool last;
+  if (!ring_sub(p, g.rg_cell[r.c0], stage, it0, n, m, tau, last)) return;
+  const int ncm = r.cells(m), nem = r.edges(m), nem1 = r.edges(m - 1);
+  // the edges' state: the wind, its forcing Tp + G, the flux's coefficient l_e h_e, 1 / d_e (or d_e), both cells' places
+  double v[EPT][L], f[EPT][L], de[EPT], rde[EPT], a0[L];
+  fast cf[EPT][L];
+  int e_[EPT], ec[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < nem) e_[j] = g.rg_edge[r.e0 + q];
+    if (q < nem1) ec[j] = g.rg_ecell[r.e0 + q];
+  }
+  int c_[CPT];
+  RingCell rc[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ncm) {
+      c_[j] = g.rg_cell[r.c0 + q];
+      rc[j].set(g.rg_slot + 3 * (size_t)(r.c0 + q), PE - 2);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < nem) {
+      const int e = e_[j];
 #pragma unroll
       for (int l = 0; l < L; l++) {
-        const size_t t = (size_t)l * E + eo;
-        v_[l] = uin[t];
-        a_[l] = it == 0 ? 0.0 : acc[t];
-        tp_[l] = Tp[t];
+        v[j][l] = uin[(size_t)l * E + e];
+        cf[j][l] = coef[(size_t)l * E + e];
+      }
+      if (q < nem1) {
+        de[j] = dv.de[e];
+        rde[j] = recip(de[j]);
+        const double Ge = G[e];
+#pragma unroll
+        for (int l = 0; l < L; l++) f[j][l] = Tp[(size_t)l * E + e] + Ge;
       }
     }
   }
-  // the q-th halo edge of B: its inputs
-  int xsl = 0;
-  Sub sx{false, false, 0.0};
-  double xv_[L], xtp_[L], xrde = 0, xG = 0;
-  if (q0 < nx) {
-    const int xe = g.px_edge[x0 + q0];
-    xsl = g.px_slot[x0 + q0];
-    sx = sub_at(p, p.we, xe, stage, it, n, tau);
-    if (sx.active) {
-      xrde = dv.de[xe];
-      xG = G[xe];
+  if (t < r.own && it0 > 0) {
+#pragma unroll
+    for (int l = 0; l < L; l++) a0[l] = acc[(size_t)l * E + e_[0]];
+  } else {
+#pragma unroll
+    for (int l = 0; l < L; l++) a0[l] = 0.0;
+  }
+  double mu[CPT][L], Sk[CPT][L], A[CPT], rA[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; j++)
+    if (t + j * RBS < ncm) {
+      A[j] = dv.A[c_[j]];
+      rA[j] = recip(A[j]);
 #pragma unroll
       for (int l = 0; l < L; l++) {
-        const size_t t = (size_t)l * E + xe;
-        xv_[l] = uin[t];
-        xtp_[l] = Tp[t];
+        mu[j][l] = mu_src[(size_t)l * N + c_[j]];
+        Sk[j][l] = S[(size_t)l * N + c_[j]];
       }
     }
-  }
-  // the q-th patch-and-halo cell's edge slots in B's winds (0xffff: no edge)
-  int ces[6] = {0xffff, 0xffff, 0xffff, 0xffff, 0xffff, 0xffff};
-  if (q0 < nC) {
-    const int* ps_ = g.pc_eslot + 3 * g.pc_off[b] + 3 * q0;
-    // (unsigned: a missing edge's 0xffff in the high half makes the word negative as an int32)
-    const unsigned pa = (unsigned)ps_[0], pb2 = (unsigned)ps_[1], pcc = (unsigned)ps_[2];
-    ces[0] = (int)(pa & 0xffffu); ces[1] = (int)(pa >> 16); ces[2] = (int)(pb2 & 0xffffu);
-    ces[3] = (int)(pb2 >> 16); ces[4] = (int)(pcc & 0xffffu); ces[5] = (int)(pcc >> 16);
-  }
-  // A: masses and Phi* of sub-step it on patch, halo and second halo
-  int ci = 0, cslot = 0;                           // (thread q's cell q, for C)
-  Sub cc{false, false, 0.0};
-  double cS[L], cA = 0;
-  for (int s = q0; s < nown + nh + nk; s += FBS) {
-    const int i = s < nown ? c0 + s : s < nC ? g.ph_cell[h0 + s - nown] : g.ph2_cell[k0 + s - nC];
-    const int slot = s < nown ? s : PC + (s - nown);
-    const Sub sb = sub_at(p, p.wc, i, stage, it, n, tau);
-    if (s < nC) {
-      ci = i;
-      cslot = slot;
-      cc = sub_at(p, p.wc, i, stage, it + 1, n, tau);
-    }
-    if (!sb.active) continue;
-    int e[6];
-    ring6(g.cellEdge, i, e);
-    double sak[L], Sk[L];
 #pragma unroll
-    for (int k = 0; k < L; k++) {
-      double c6[6];                                // (sign * l_e * h_e per slot, written with the stage's h_e)
-      load6(coef + ((size_t)k * N + i) * 6, c6);
-      const double* ul = uin + (size_t)k * E;
-      double t[6];
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < nem)
 #pragma unroll
-      for (int m = 0; m < 6; m++) {
-        if (CF && s < nC) cfs[(k * 6 + m) * P1 + s] = c6[m];
-        t[m] = c6[m] * ul[ok0(e[m])];
+      for (int l = 0; l < L; l++) F[l * PE + q] = (double)cf[j][l] * v[j][l];
+  }
+  if (t < L) F[t * PE + PE - 2] = 0.0;
+  for (int it = 0; it < m; it++) {
+    const int nc = r.cells(m - it), ne = it + 1 < m ? r.edges(m - it - 1) : r.own;
+    __syncthreads();
+    // the masses of the rings this step still reaches, and Phi* from their forward-weighted sum
+#pragma unroll
+    for (int j = 0; j < CPT; j++) {
+      const int q = t + j * RBS;
+      if (q >= nc) continue;
+      double P[L], a = 0;
+#pragma unroll
+      for (int l = 0; l < L; l++) {
+        const double m0 = mu[j][l];
+        const double m1 = m0 - over(tau * rc[j].div(F + l * PE), A[j], rA[j]);
+        mu[j][l] = m1;
+        a += m1 + p.div_damp * (m1 - m0);
+        P[l] = a;
       }
-      double div = 0;
-#pragma unroll
-      for (int m = 0; m < 6; m++)
-        if (e[m] >= 0) div += t[m];
-      const double m0 = mu_src[(size_t)k * N + i];
-      const double m1 = m0 - DIVBY(sb.tau * div, dv.A[i]);
-      muA[k * PS + slot] = m1;
-      sak[k] = m1 + p.div_damp * (m1 - m0);
-      Sk[k] = S[(size_t)k * N + i];
-    }
-    if (s < nC) {
-#pragma unroll
-      for (int k = 0; k < L; k++) cS[k] = Sk[k];
-      cA = dv.A[i];
-    }
-    double P[L];
-    double a = 0;
-#pragma unroll
-    for (int m = 0; m < L; m++) {
-      a += sak[m];
-      P[m] = a;
-    }
-#pragma unroll
-    for (int k = 0; k < L; k++) {
       double ph = 0;
 #pragma unroll
-      for (int m = L - 1; m >= k; m--) ph += Sk[m] * P[m];
-      phiA[k * PS + slot] = ph;
+      for (int l = L - 1; l >= 0; l--) {
+        ph += Sk[j][l] * P[l];
+        phi[l * PC + q] = ph;
+      }
     }
-  }
-  __syncthreads();
-  // B: the winds of sub-step it on the patch's edges (registers) and the halo's
-  double u1_[L], acc1_[L];
-  if (q0 < ne && s1.active) {
-    const int sI = slo & 0xffff, sJ = slo >> 16;
+    __syncthreads();
+    // the winds of the edges inside those rings
 #pragma unroll
-    for (int l = 0; l < L; l++) {
-      acc1_[l] = it == 0 ? 0.0 + v_[l] : a_[l] + v_[l];
-      u1_[l] = v_[l] + s1.tau * (DIVBY(-(phiA[l * PS + sJ] - phiA[l * PS + sI]), rde_) + tp_[l] + G_);
-      uB[l * PE + q0] = u1_[l];
-    }
-    if (s1.last) {                                 // (a world whose last sub-step this is: done after B)
+    for (int j = 0; j < EPT; j++) {
+      const int q = t + j * RBS;
+      if (q >= ne) continue;
+      const int cI = ec[j] & 0xffff, cJ = ec[j] >> 16;
 #pragma unroll
       for (int l = 0; l < L; l++) {
-        const size_t t = (size_t)l * E + eo;
-        un[t] = u1_[l];
-        acc[t] = acc1_[l];
+        if (j == 0) a0[l] += v[j][l];
+        v[j][l] = v[j][l] + tau * (over(-(phi[l * PC + cJ] - phi[l * PC + cI]), de[j], rde[j]) + f[j][l]);
+        F[l * PE + q] = (double)cf[j][l] * v[j][l];
       }
     }
   }
-  if (q0 < nx && sx.active) {
-    const int sI = xsl & 0xffff, sJ = xsl >> 16;
-#pragma unroll
-    for (int l = 0; l < L; l++)
-      uB[l * PE + ne + q0] = xv_[l] + sx.tau * (DIVBY(-(phiA[l * PS + sJ] - phiA[l * PS + sI]), xrde) + xtp_[l] + xG);
-  }
-  for (int w = q0 + FBS; w < nx; w += FBS) {       // (halo edges past the block's threads)
-    const int e = g.px_edge[x0 + w];
-    const Sub sb = sub_at(p, p.we, e, stage, it, n, tau);
-    if (!sb.active) continue;
-    const int sl = g.px_slot[x0 + w];
-    const int sI = sl & 0xffff, sJ = sl >> 16;
-    const double rde = dv.de[e], Ge = G[e];
+  if (t < r.own) {
+    double* out = last ? un : uout;
 #pragma unroll
     for (int l = 0; l < L; l++) {
-      const size_t t = (size_t)l * E + e;
-      uB[l * PE + ne + w] =
-          uin[t] + sb.tau * (DIVBY(-(phiA[l * PS + sJ] - phiA[l * PS + sI]), rde) + Tp[t] + Ge);
+      acc[(size_t)l * E + e_[0]] = a0[l];
+      out[(size_t)l * E + e_[0]] = v[0][l];
     }
   }
-  __syncthreads();
-  // C: masses and Phi* of sub-step it + 1 on patch and halo (thread q's cell q), from B's winds
-  if (q0 < nC && cc.active) {
-    double cf[L][6];
-    if constexpr (CF) {
+  if (t < r.cells(0))
 #pragma unroll
-      for (int k = 0; k < L; k++)
-#pragma unroll
-        for (int m = 0; m < 6; m++) cf[k][m] = cfs[(k * 6 + m) * P1 + q0];
-    } else {
-#pragma unroll
-      for (int k = 0; k < L; k++) load6(coef + ((size_t)k * N + ci) * 6, cf[k]);
-    }
-    double m1k[L], sak[L];
-#pragma unroll
-    for (int k = 0; k < L; k++) {
-      double t[6];
-#pragma unroll
-      for (int m = 0; m < 6; m++) t[m] = cf[k][m] * uB[k * PE + (ces[m] != 0xffff ? ces[m] : 0)];
-      double div = 0;
-#pragma unroll
-      for (int m = 0; m < 6; m++)
-        if (ces[m] != 0xffff) div += t[m];
-      const double m0 = muA[k * PS + cslot];
-      const double m1 = m0 - DIVBY(cc.tau * div, cA);
-      m1k[k] = m1;
-      sak[k] = m1 + p.div_damp * (m1 - m0);
-    }
-    double P[L];
-    double a = 0;
-#pragma unroll
-    for (int m = 0; m < L; m++) {
-      a += sak[m];
-      P[m] = a;
-    }
-#pragma unroll
-    for (int k = 0; k < L; k++) {
-      double ph = 0;
-#pragma unroll
-      for (int m = L - 1; m >= k; m--) ph += cS[m] * P[m];
-      phiC[k * PS + cslot] = ph;
-      if (q0 < nown) mu_out[(size_t)k * N + ci] = m1k[k];
-    }
-  }
-  __syncthreads();
-  // D: the winds of sub-step it + 1 on the patch's edges
-  if (q0 < ne && s1.active && s2.active) {
-    const int sI = slo & 0xffff, sJ = slo >> 16;
-    double* out = s2.last ? un : uout;
-#pragma unroll
-    for (int l = 0; l < L; l++) {
-      const size_t t = (size_t)l * E + eo;
-      acc[t] = acc1_[l] + u1_[l];
-      out[t] = u1_[l] + s2.tau * (DIVBY(-(phiC[l * PS + sJ] - phiC[l * PS + sI]), rde_) + tp_[l] + G_);
-    }
-  }
+    for (int l = 0; l < L; l++) mu_out[(size_t)l * N + c_[0]] = mu[0][l];
 }
 
-// One barotropic sub-step in one launch on the grid's patches (as k_af_patch for the air): the surface height of
-// the patch's and halo cells, its potential Gc (eta + gamma (eta - eta_prev)) in LDS, then the barotropic wind on
-// the patch's edges. Heights alternate between eta and eta_prev, winds between ubb and ubc; an edge's last sub-step
-// writes ub (what the stage's update reads). Arithmetic as k_bt_eta's and k_bt_u's.
-__global__ __launch_bounds__(FBS) void k_bt_patch(isw_grid g, Div dv, LP p, int stage, int it, int n, double tau,
+// The ocean's barotropic sub-steps (layers.cu:366-388), the wall mask of the reference's lay_mask calls fused in: the
+// surface height of the rings' cells, its potential Gc (eta + gamma (eta - eta_prev)), the barotropic wind of their
+// edges. The last sub-step writes ub_fin (what the stage's update reads).
+template <int EPT, int CPT>
+__global__ __launch_bounds__(RBS) void k_bt_rings(isw_grid g, Div dv, LP p, int stage, int it0, int m, int n, double tau,
                                                   double gamma, const double* __restrict__ He,
-                                                  const double* __restrict__ ub_src,
-                                                  const double* __restrict__ eta_src, double* __restrict__ eta_out,
-                                                  const double* __restrict__ G, const double* __restrict__ Gc,
-                                                  const double* __restrict__ wall, double* __restrict__ acc,
-                                                  double* __restrict__ ub_out, double* __restrict__ ub_fin) {
-  extern __shared__ double sx[];                   // [pslots]
-  const int N = g.N, PC = g.pcells;
-  const int b = xblock();
-  const int c0 = b * PC, nown = min(PC, N - c0);
-  const int h0 = g.ph_off[b], nh = g.ph_off[b + 1] - h0;
-  const int e0 = g.pe_off[b], ne = g.pe_off[b + 1] - e0;
-  const int q0 = threadIdx.x;
-  int e_ = 0, sl_ = 0;
-  Sub sbe{false, false, 0.0};
-  double v_ = 0, a_ = 0, rde_ = 0, G_ = 0, w_ = 1;
-  if (q0 < ne) {
-    e_ = g.pe_edge[e0 + q0];
-    sl_ = g.pe_slot[e0 + q0];
-    sbe = sub_at(p, p.we, e_, stage, it, n, tau);
-    if (sbe.active) {
-      v_ = ub_src[e_];
-      a_ = it == 0 ? 0.0 : acc[e_];
-      rde_ = dv.de[e_];
-      G_ = G[e_];
-      if (wall) w_ = wall[e_];
-    }
-  }
-  for (int s = threadIdx.x; s < nown + nh; s += FBS) {
-    const int i = s < nown ? c0 + s : g.ph_cell[h0 + s - nown];
-    const int slot = s < nown ? s : PC + (s - nown);
-    const Sub sb = sub_at(p, p.wc, i, stage, it, n, tau);
-    if (!sb.active) continue;
-    const double et0 = eta_src[i];
-    int e[6];
-    ring6(g.cellEdge, i, e);
-    double t[6];
+                                                  const double* __restrict__ ub_src, const double* __restrict__ eta_src,
+                                                  double* __restrict__ eta_out, const double* __restrict__ G,
+                                                  const double* __restrict__ Gc, const double* __restrict__ wall,
+                                                  double* __restrict__ acc, double* __restrict__ ub_out,
+                                                  double* __restrict__ ub_fin) {
+  constexpr int PE = EPT * RBS + 2;
+  extern __shared__ double sm[];
+  const int t = (int)threadIdx.x;
+  double* F = sm;                                  // [PE] l_e H_e u, the last but one 0
+  double* x = sm + PE;                             // the potential
+  const Ring r = ring_of(g);
+  bool last;
+  if (!ring_sub(p, g.rg_cell[r.c0], stage, it0, n, m, tau, last)) return;
+  const int ncm = r.cells(m), nem = r.edges(m), nem1 = r.edges(m - 1);
+  double v[EPT], cf[EPT], f[EPT], de[EPT], rde[EPT], wl[EPT], a0 = 0;
+  int e_[EPT], ec[EPT], c_[CPT];
+  RingCell rc[CPT];
 #pragma unroll
-    for (int m = 0; m < 6; m++) {
-      const int ek = ok0(e[m]);
-      t[m] = (double)g.cellSign[i * 6 + m] * g.le[ek] * He[ek] * ub_src[ek];
-    }
-    double div = 0;
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < nem) e_[j] = g.rg_edge[r.e0 + q];
+    if (q < nem1) ec[j] = g.rg_ecell[r.e0 + q];
+  }
 #pragma unroll
-    for (int m = 0; m < 6; m++)
-      if (e[m] >= 0) div += t[m];
-    const double et = et0 - DIVBY(sb.tau * div, dv.A[i]);
-    sx[slot] = Gc[i] * (et + gamma * (et - et0));
-    if (s < nown) eta_out[i] = et;
-  }
-  __syncthreads();
-  for (int q = q0; q < ne; q += FBS) {
-    int e = e_, sl = sl_;
-    Sub sb = sbe;
-    double v = v_, a = a_, rde = rde_, Ge = G_, wl = w_;
-    if (q != q0) {                                 // (a patch with more edges than threads)
-      e = g.pe_edge[e0 + q];
-      sl = g.pe_slot[e0 + q];
-      sb = sub_at(p, p.we, e, stage, it, n, tau);
-      if (!sb.active) continue;
-      v = ub_src[e];
-      a = it == 0 ? 0.0 : acc[e];
-      rde = dv.de[e];
-      Ge = G[e];
-      wl = wall ? wall[e] : 1.0;
+  for (int j = 0; j < CPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ncm) {
+      c_[j] = g.rg_cell[r.c0 + q];
+      rc[j].set(g.rg_slot + 3 * (size_t)(r.c0 + q), PE - 2);
     }
-    if (!sb.active) continue;
-    double an = it == 0 ? 0.0 + v : a + v;
-    double un = v + sb.tau * (DIVBY(-(sx[sl >> 16] - sx[sl & 0xffff]), rde) + Ge);
-    if (wall && wl == 0) { un = 0; an = 0; }
-    (sb.last ? ub_fin : ub_out)[e] = un;
-    acc[e] = an;
   }
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < nem) {
+      const int e = e_[j];
+      v[j] = ub_src[e];
+      cf[j] = g.le[e] * He[e];
+      if (q < nem1) {
+        de[j] = dv.de[e];
+        rde[j] = recip(de[j]);
+        f[j] = G[e];
+        wl[j] = wall ? wall[e] : 1.0;
+      }
+    }
+  }
+  if (t < r.own && it0 > 0) a0 = acc[e_[0]];
+  double et[CPT], A[CPT], rA[CPT], gc[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; j++)
+    if (t + j * RBS < ncm) {
+      et[j] = eta_src[c_[j]];
+      A[j] = dv.A[c_[j]];
+      rA[j] = recip(A[j]);
+      gc[j] = Gc[c_[j]];
+    }
+#pragma unroll
+  for (int j = 0; j < EPT; j++)
+    if (t + j * RBS < nem) F[t + j * RBS] = cf[j] * v[j];
+  if (t == 0) F[PE - 2] = 0.0;
+  for (int it = 0; it < m; it++) {
+    const int nc = r.cells(m - it), ne = it + 1 < m ? r.edges(m - it - 1) : r.own;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < CPT; j++) {
+      const int q = t + j * RBS;
+      if (q >= nc) continue;
+      const double e0 = et[j], e1 = e0 - over(tau * rc[j].div(F), A[j], rA[j]);
+      x[q] = gc[j] * (e1 + gamma * (e1 - e0));
+      et[j] = e1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+      const int q = t + j * RBS;
+      if (q >= ne) continue;
+      if (j == 0) a0 += v[j];
+      v[j] = v[j] + tau * (over(-(x[ec[j] >> 16] - x[ec[j] & 0xffff]), de[j], rde[j]) + f[j]);
+      if (wl[j] == 0) {
+        v[j] = 0;
+        if (j == 0) a0 = 0;
+      }
+      F[q] = cf[j] * v[j];
+    }
+  }
+  if (t < r.own) {
+    (last ? ub_fin : ub_out)[e_[0]] = v[0];
+    acc[e_[0]] = a0;
+  }
+  if (t < r.cells(0)) eta_out[c_[0]] = et[0];
 }
 
 __global__ __launch_bounds__(BS) void k_bt_eta(isw_grid g, Div dv, LP p, int stage, int it, int n, double tau,
@@ -1790,6 +1655,38 @@ static void lap(const isw_grid* g, int L, const double* u, double* D1, double* Z
              k_edge_lap, g1((long)g->E * L), BS, *g, L, D1, Z1, out);
 }
 
+// The fast sub-steps that one launch takes on the grid's ring tables, for `rows` values per cell: as many as asked for
+// whose rings fit a block's threads (four edges and two cells each) and 64 KB of LDS; 0 without the tables.
+// (The kernels come with 2 or 3 edges and one cell to a thread, or 4 edges and two cells.)
+static int ring_cpt(const isw_grid* g, int m) { return g->rg_cells[m] > RBS || g->rg_edges[m] > 3 * RBS ? 2 : 1; }
+static int ring_ept(const isw_grid* g, int m) {
+  const int k = (g->rg_edges[m] + RBS - 1) / RBS, least = ring_cpt(g, m) == 2 ? 4 : 2;
+  return k < least ? least : k;
+}
+static size_t ring_lds(const isw_grid* g, int rows, int m) {
+  return (size_t)rows * (ring_ept(g, m) * RBS + 2 + ring_cpt(g, m) * RBS) * sizeof(double);
+}
+static int ring_most(const isw_grid* g, int rows, int want) {
+  if (!g->rg_head || g->rg_owned > RBS) return 0;
+  int m = want < g->rg_k ? want : g->rg_k;
+  while (m > 0 && (ring_ept(g, m) > 4 || g->rg_cells[m] > 2 * RBS || ring_lds(g, rows, m) > 65536)) m--;
+  return m;
+}
+// f(edges, cells per thread) as compile-time counts, for m sub-steps.
+template <class F>
+static void ring_launch(const isw_grid* g, int m, F&& f) {
+  using std::integral_constant;
+  const int e = ring_ept(g, m), c = ring_cpt(g, m);      // (e <= 4: ring_most)
+  if (c == 1 && e == 2) f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  else if (c == 1) f(integral_constant<int, 3>{}, integral_constant<int, 1>{});
+  else f(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+}
+// The next launch's share of `left` sub-steps: as few launches as there can be, as even as they can be.
+static int ring_steps(int left, int most) {
+  const int launches = (left + most - 1) / most;
+  return (left + launches - 1) / launches;
+}
+
 // Layers._stage (layers.py:255-309).
 static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div& dv, int si, const double* hs,
                   const double* us, const double* h0, const double* u0, double c, double dt, int nfast, double* hn,
@@ -1804,15 +1701,15 @@ static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div
 #if ISW_FORM_MIXED
   fast* pk = s->pkf;
   const fast* wf = g->wf;
-  // the air's fast sub-steps' coefficients per cell slot (FP32 in the mixed form)
-  fast* cf = s->air && g->ph_off ? s->cfcf : nullptr;
+  // the air's fast sub-steps' flux coefficients per edge (FP32 in the mixed form)
+  fast* cf = s->air && g->rg_head ? s->cfcf : nullptr;
 #else
   fast* pk = s->pk;
   const fast* wf = g->w;
-  fast* cf = s->air && g->ph_off ? s->cfc : nullptr;
+  fast* cf = s->air && g->rg_head ? s->cfc : nullptr;
 #endif
   ISW_LAUNCH("edge_hq", l_ * n_ * D + l_ * v_ * D + l_ * e_ * D + 4 * e_ * I + l_ * e_ * D + 3 * l_ * e_ * R +
-                            (cf ? 6 * l_ * n_ * sizeof(fast) + 2 * e_ + 6 * n_ + e_ * D : 0),
+                            (cf ? l_ * e_ * sizeof(fast) + e_ * D : 0),
              k_edge_hq, g1((long)E * L), BS, *g, L, s->shelf, hs, s->q, us, s->hedge, pk, cf);
   const double neoe = g->n_eoe;
   const double slow_bytes = 3 * l_ * e_ * R + neoe * (R + I) + (e_ + 1) * I + 2 * l_ * e_ * D + l_ * n_ * D +
@@ -1845,72 +1742,45 @@ static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div
     fs.we = s->batch->we;
     fs.winv = s->batch->inv_n;
   }
-  const size_t patch_lds = g->ph_off ? (size_t)L * g->pslots * sizeof(double) : 0;
-  if (s->air && g->ph_off && patch_lds <= 65536) {
-    // one launch per sub-step on the grid's patches; masses and winds alternate between (muf, mup) and (uf, ufb)
+  const int KR = s->air ? ring_most(g, L, AIR_STEPS) : ring_most(g, 1, SEA_STEPS);
+  if (s->air && KR) {
+    // several sub-steps per launch; masses and winds alternate between (muf, mup) and (uf, ufb)
     // the last stage steps the wind in place (un is u0): where a launch might both read u0 (its first sub-step's
-    // halo) and write un (an element's last sub-step), the sub-steps read a copy of u0 instead (s->F is free here)
+    // rings) and write un (a last sub-step), the sub-steps read a copy of u0 instead (s->F is free here)
     const double* uin = u0;
-    if (un == u0 && (s->batch || n <= 2)) {
+    if (un == u0 && (s->batch || n <= KR)) {
       ISW_LAUNCH("copy", 2 * l_ * e_ * D, k_copy, g1((long)E * L), BS, (long)E * L, u0, s->F);
       uin = s->F;
     }
     const double* mus = h0;
-    // LDS of the pair kernel: Phi* twice, masses and winds; with L <= 4 also its patch-and-halo cells' coefficients
-    const size_t pair_lds =
-        g->ph2_off ? (size_t)L * (3 * g->pslots2 + g->pedges2 + (L <= 4 ? 6 * g->pslots : 0)) * sizeof(double) : 0;
-    int it = 0;
     int flip = 0;
-    if (g->ph2_off && pair_lds <= 65536) {
-      // two sub-steps per launch while two remain; an odd one left runs alone below
-      for (; it + 1 < n; it += 2, flip ^= 1) {
-        double* uo = flip ? s->ufb : s->uf;
-        double* mo = flip ? s->mup : s->muf;
-        const double bytes = l_ * e_ * D + 6 * l_ * n_ * sizeof(fast) + 3 * l_ * n_ * D + l_ * e_ * D + e_ * D +
-                             (it == 0 ? 1 : 2) * l_ * e_ * D + l_ * e_ * D + 6 * n_ * I + n_ * D + e_ * D +
-                             2 * e_ * I;
-#define PAIR(LL)                                                                                                  \
-  ISW_LAUNCH_SHM("af_patch2", bytes, k_af_patch2<LL>, dim3((unsigned)g->npatch), dim3(FBS), pair_lds, *g, p, dv,  \
-                 si, it, n, tau, cf, uin, mus, mo, s->S, s->Tp, s->G, s->accL, uo, un)
-        switch (L) {
-          case 1: PAIR(1); break;
-          case 2: PAIR(2); break;
-          case 3: PAIR(3); break;
-          case 4: PAIR(4); break;
-          case 5: PAIR(5); break;
-          case 6: PAIR(6); break;
-          case 7: PAIR(7); break;
-          default: PAIR(8); break;
-        }
-#undef PAIR
-        uin = uo;
-        mus = mo;
-      }
-    }
-    for (; it < n; it++, flip ^= 1) {
+    for (int it = 0; it < n; flip ^= 1) {
+      const int m = ring_steps(n - it, KR);
       double* uo = flip ? s->ufb : s->uf;
       double* mo = flip ? s->mup : s->muf;
-      // (algorithmic bytes: uin, the cells' slot coefficients, mu in and out, S, Tp, G, acc, the wind out, the
-      // cell ring, 1/A, de, the patch's edge list and slots; the halo's re-reads and Phi* in LDS are free)
-      const double bytes = l_ * e_ * D + 6 * l_ * n_ * sizeof(fast) + 3 * l_ * n_ * D + l_ * e_ * D + e_ * D +
-                           (it == 0 ? 1 : 2) * l_ * e_ * D + l_ * e_ * D + 6 * n_ * I + n_ * D + e_ * D +
-                           2 * e_ * I;
-#define PATCH(LL)                                                                                                 \
-  ISW_LAUNCH_SHM("af_patch", bytes, k_af_patch<LL>, dim3((unsigned)g->npatch), dim3(FBS), patch_lds, *g, p, dv, si, \
-                 it, n, tau, cf, uin, mus, mo, s->S, s->Tp, s->G, s->accL, uo, un)
+      // (algorithmic bytes: uin, the coefficients, mu in and out, S, Tp, G, acc, the wind out, 1/A, de, the patches'
+      // cell and edge lists once each; the rings' re-reads and Phi* in LDS are free)
+      const double bytes = l_ * e_ * D + l_ * e_ * sizeof(fast) + 3 * l_ * n_ * D + l_ * e_ * D + e_ * D +
+                           (it == 0 ? 1 : 2) * l_ * e_ * D + l_ * e_ * D + n_ * D + e_ * D + 4 * n_ * I + 2 * e_ * I;
+#define RINGS(LL) ring_launch(g, m, [&](auto ept, auto cpt) {                              \
+    ISW_LAUNCH_SHM("af_rings", bytes, (k_af_rings<LL, decltype(ept)::value, decltype(cpt)::value>),                    \
+                   dim3((unsigned)g->rg_npatch), dim3(RBS), ring_lds(g, L, m), *g, p, dv, si, it, m, n, tau, cf, uin,  \
+                   mus, mo, s->S, s->Tp, s->G, s->accL, uo, un);                                                     \
+  })
       switch (L) {
-        case 1: PATCH(1); break;
-        case 2: PATCH(2); break;
-        case 3: PATCH(3); break;
-        case 4: PATCH(4); break;
-        case 5: PATCH(5); break;
-        case 6: PATCH(6); break;
-        case 7: PATCH(7); break;
-        default: PATCH(8); break;
+        case 1: RINGS(1); break;
+        case 2: RINGS(2); break;
+        case 3: RINGS(3); break;
+        case 4: RINGS(4); break;
+        case 5: RINGS(5); break;
+        case 6: RINGS(6); break;
+        case 7: RINGS(7); break;
+        default: RINGS(8); break;
       }
-#undef PATCH
+#undef RINGS
       uin = uo;
       mus = mo;
+      it += m;
     }
     fs.air = 1;
     fs.hedge = s->hedge;
@@ -1930,22 +1800,26 @@ static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div
     fs.hedge = s->hedge;
     fs.acc = s->accL;
   } else {
-    if (g->ph_off && s->ubc) {
-      // one launch per sub-step on the grid's patches: heights alternate between eta and eta_prev, winds between
-      // ubb and ubc, each edge's last sub-step writes ub
+    if (KR && s->ubc) {
+      // several sub-steps per launch: heights alternate between eta and eta_prev, winds between ubb and ubc, each
+      // edge's last sub-step writes ub
       const double* ubs_ = s->ub0;
       const double* ets = s->eta0;
-      for (int it = 0; it < n; it++) {
-        double* uo = (it & 1) ? s->ubc : s->ubb;
-        double* eo = (it & 1) ? s->eta_prev : s->eta;
-        ISW_LAUNCH_SHM("bt_patch", 2 * e_ * D + 6 * n_ * (I + C) + e_ * D + n_ * D + 2 * n_ * D + e_ * D + e_ * D +
-                                       n_ * D + (s->wall ? e_ * D : 0) + e_ * D + (it == 0 ? 1 : 2) * e_ * D +
-                                       2 * e_ * I,
-                       k_bt_patch, dim3((unsigned)g->npatch), dim3(FBS), (size_t)g->pslots * sizeof(double), *g, dv,
-                       p, si, it, n, tau, s->div_damp, s->He, ubs_, ets, eo, s->G, s->Gc, s->wall, s->acc, uo,
-                       s->ub);
+      int flip = 0;
+      for (int it = 0; it < n; flip ^= 1) {
+        const int m = ring_steps(n - it, KR);
+        double* uo = flip ? s->ubc : s->ubb;
+        double* eo = flip ? s->eta_prev : s->eta;
+        const double bytes = 3 * e_ * D + n_ * D + 3 * n_ * D + e_ * D + e_ * D + (s->wall ? e_ * D : 0) + e_ * D +
+                             (it == 0 ? 1 : 2) * e_ * D + 4 * n_ * I + 2 * e_ * I;
+        ring_launch(g, m, [&](auto ept, auto cpt) {
+          ISW_LAUNCH_SHM("bt_rings", bytes, (k_bt_rings<decltype(ept)::value, decltype(cpt)::value>),
+                         dim3((unsigned)g->rg_npatch), dim3(RBS), ring_lds(g, 1, m), *g, dv, p, si, it, m, n, tau,
+                         s->div_damp, s->He, ubs_, ets, eo, s->G, s->Gc, s->wall, s->acc, uo, s->ub);
+        });
         ubs_ = uo;
         ets = eo;
+        it += m;
       }
     } else
     for (int it = 0; it < n; it++) {

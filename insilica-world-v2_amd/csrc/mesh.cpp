@@ -504,4 +504,170 @@ int isw_mesh_weights(int64_t N, int64_t E, const uint8_t* deg, const int32_t* eI
   return 0;
 }
 
+// The patches of the fast sub-steps (isw_grid's rg_* tables): the cells split into npatch = ceil(N / pcells) compact
+// patches by recursive bisection across the longest principal axis, in the bisection's order, and each patch's K rings of
+// neighbour cells with the edges they touch. (Compact patches rather than runs of the cell numbering: the rings of a run
+// along the Hilbert curve hold a quarter more cells on average and twice as many at worst.)
+//
+// Per patch, head[16 * b ..]: its first entry in cell (and, times 3, in slot), its first entry in edge (and ecell), the
+// edges it owns (whose first cell is its own), then the cells within ring 0 .. K, then the edges touching those. cell: the
+// patch's cells ascending, then each ring's; edge: the owned edges ascending, the patch's others, then each ring's;
+// slot: per cell its six edges' places in the patch's edge list in cellEdge order, two to an int32, 0x8000 set where the
+// cell's sign on it is negative, 0x7fff for no edge; ecell: per edge the places of its first and second cell in the
+// patch's cell list (first | second << 16), 0 for edges that touch ring K only (their outer cell is not listed).
+// sizes (3 + 12): entries of cell, entries of edge, the most owned edges of a patch; then the most cells within ring
+// 0 .. K (six places) and the most edges touching those (six). Called twice, first with head NULL for the sizes. Returns -1 when an edge lacks a cell or a patch is too large for its slots.
+int isw_mesh_rings(int64_t N, int64_t E, int K, int64_t pcells, const double* pos, const int32_t* cellEdge,
+                   const int8_t* cellSign, const int32_t* eI, const int32_t* eJ, int64_t* sizes, int32_t* head,
+                   int32_t* cell, int32_t* slot, int32_t* edge, int32_t* ecell) {
+  if (K < 1 || K > 5 || pcells < 1 || N < 1) return -2;
+  for (int64_t e = 0; e < E; e++)
+    if (eI[e] < 0 || eJ[e] < 0 || eI[e] >= N || eJ[e] >= N) return -1;
+  const int64_t nb = (N + pcells - 1) / pcells;
+  std::vector<int32_t> order(N);
+  std::iota(order.begin(), order.end(), 0);
+  std::vector<int64_t> start(nb + 1, N);
+  struct Part { int64_t lo, hi, first, k; };
+  std::vector<Part> todo = {{0, N, 0, nb}};
+  std::vector<double> key(N);
+  while (!todo.empty()) {
+    const Part q = todo.back();
+    todo.pop_back();
+    if (q.k == 1) {
+      start[q.first] = q.lo;
+      std::sort(order.begin() + q.lo, order.begin() + q.hi);
+      continue;
+    }
+    V3 m = {0, 0, 0};
+    for (int64_t i = q.lo; i < q.hi; i++) m = add(m, get3(pos, order[i]));
+    m = scale(m, 1.0 / double(q.hi - q.lo));
+    double c[3][3] = {};
+    for (int64_t i = q.lo; i < q.hi; i++) {
+      const V3 d = sub(get3(pos, order[i]), m);
+      const double v[3] = {d.x, d.y, d.z};
+      for (int a = 0; a < 3; a++)
+        for (int b = 0; b < 3; b++) c[a][b] += v[a] * v[b];
+    }
+    double v[3] = {1.0, 0.9, 0.8};                       // the longest principal axis by power iteration
+    for (int it = 0; it < 50; it++) {
+      double w[3], s = 0;
+      for (int a = 0; a < 3; a++) {
+        w[a] = c[a][0] * v[0] + c[a][1] * v[1] + c[a][2] * v[2];
+        s += w[a] * w[a];
+      }
+      if (!(s > 0)) break;
+      for (int a = 0; a < 3; a++) v[a] = w[a] / std::sqrt(s);
+    }
+    for (int64_t i = q.lo; i < q.hi; i++) {
+      const V3 d = get3(pos, order[i]);
+      key[order[i]] = d.x * v[0] + d.y * v[1] + d.z * v[2];
+    }
+    const int64_t ka = q.k / 2, mid = q.lo + (q.hi - q.lo) * ka / q.k;
+    std::nth_element(order.begin() + q.lo, order.begin() + mid, order.begin() + q.hi,
+                     [&](int32_t a, int32_t b) { return key[a] != key[b] ? key[a] < key[b] : a < b; });
+    todo.push_back({mid, q.hi, q.first + ka, q.k - ka});
+    todo.push_back({q.lo, mid, q.first, ka});
+  }
+  std::vector<std::array<int32_t, 16>> heads(nb);
+  std::vector<std::vector<int32_t>> cells(nb), edges(nb);
+#pragma omp parallel
+  {
+    std::vector<int32_t> cmark(N, -1), emark(E, -1);      // the patch that listed a cell or an edge last
+#pragma omp for schedule(dynamic, 8)
+    for (int64_t b = 0; b < nb; b++) {
+      auto& C = cells[b];
+      auto& G = edges[b];
+      auto& H = heads[b];
+      H.fill(0);
+      C.assign(order.begin() + start[b], order.begin() + start[b + 1]);
+      for (int32_t c : C) cmark[c] = (int32_t)b;
+      // owned edges first, then the patch's others
+      for (int pass = 0; pass < 2; pass++) {
+        const size_t from = G.size();
+        for (int32_t c : C)
+          for (int k = 0; k < 6; k++) {
+            const int32_t e = cellEdge[6 * (int64_t)c + k];
+            if (e < 0 || emark[e] == b) continue;
+            const bool own = cmark[eI[e]] == b;
+            if (own != (pass == 0)) continue;
+            emark[e] = (int32_t)b;
+            G.push_back(e);
+          }
+        std::sort(G.begin() + from, G.end());
+        if (pass == 0) H[2] = (int32_t)G.size();
+      }
+      H[3] = (int32_t)C.size();
+      H[4 + K] = (int32_t)G.size();
+      for (int r = 1; r <= K; r++) {
+        const size_t from = C.size(), efrom = G.size();
+        for (size_t q = 0; q < efrom; q++)
+          for (int32_t c : {eI[G[q]], eJ[G[q]]})
+            if (cmark[c] != b) {
+              cmark[c] = (int32_t)b;
+              C.push_back(c);
+            }
+        std::sort(C.begin() + from, C.end());
+        for (size_t q = from; q < C.size(); q++)
+          for (int k = 0; k < 6; k++) {
+            const int32_t e = cellEdge[6 * (int64_t)C[q] + k];
+            if (e >= 0 && emark[e] != b) {
+              emark[e] = (int32_t)b;
+              G.push_back(e);
+            }
+          }
+        std::sort(G.begin() + efrom, G.end());
+        H[3 + r] = (int32_t)C.size();
+        H[4 + K + r] = (int32_t)G.size();
+      }
+    }
+  }
+  int64_t nc = 0, ne = 0;
+  int64_t out[15] = {};
+  for (int64_t b = 0; b < nb; b++) {
+    heads[b][0] = (int32_t)nc;
+    heads[b][1] = (int32_t)ne;
+    nc += (int64_t)cells[b].size();
+    ne += (int64_t)edges[b].size();
+    out[2] = std::max(out[2], (int64_t)heads[b][2]);
+    for (int r = 0; r <= K; r++) {
+      out[3 + r] = std::max(out[3 + r], (int64_t)heads[b][3 + r]);
+      out[9 + r] = std::max(out[9 + r], (int64_t)heads[b][4 + K + r]);
+    }
+  }
+  out[0] = nc;
+  out[1] = ne;
+  std::memcpy(sizes, out, sizeof out);
+  if (out[3 + K] >= 0x7fff || out[9 + K] >= 0x7fff) return -1;
+  if (!head) return 0;
+#pragma omp parallel
+  {
+    std::vector<int32_t> cat(N), eat(E), cm(N, -1);
+#pragma omp for schedule(dynamic, 8)
+    for (int64_t b = 0; b < nb; b++) {
+      const auto& C = cells[b];
+      const auto& G = edges[b];
+      std::memcpy(head + 16 * b, heads[b].data(), 16 * sizeof(int32_t));
+      for (size_t q = 0; q < C.size(); q++) { cat[C[q]] = (int32_t)q; cm[C[q]] = (int32_t)b; }
+      for (size_t q = 0; q < G.size(); q++) eat[G[q]] = (int32_t)q;
+      for (size_t q = 0; q < C.size(); q++) {
+        const int64_t o = heads[b][0] + (int64_t)q;
+        cell[o] = C[q];
+        uint32_t w[6];
+        for (int k = 0; k < 6; k++) {
+          const int32_t e = cellEdge[6 * (int64_t)C[q] + k];
+          w[k] = e < 0 ? 0x7fffu : (uint32_t)eat[e] | (cellSign[6 * (int64_t)C[q] + k] < 0 ? 0x8000u : 0u);
+        }
+        for (int k = 0; k < 3; k++) slot[3 * o + k] = (int32_t)(w[2 * k] | w[2 * k + 1] << 16);
+      }
+      for (size_t q = 0; q < G.size(); q++) {
+        const int64_t o = heads[b][1] + (int64_t)q;
+        const int32_t e = G[q], i = eI[e], j = eJ[e];
+        edge[o] = e;
+        ecell[o] = cm[i] == b && cm[j] == b ? (int32_t)((uint32_t)cat[i] | (uint32_t)cat[j] << 16) : 0;
+      }
+    }
+  }
+  return 0;
+}
+
 }  // extern "C"

@@ -29,7 +29,10 @@ class IswGrid(ctypes.Structure):
                 + [(k, _i32p) for k in ('ph2_off', 'ph2_cell', 'px_off', 'px_edge', 'px_slot', 'pc_off', 'pc_eslot')]
                 + [(k, ctypes.c_int32) for k in ('ptedges', 'pad3_')]
                 + [(k, _i32p) for k in ('pi_off', 'pi_edge', 'tc_slot')]
-                + [('eslot', _i8p)])
+                + [('eslot', _i8p)]
+                + [(k, ctypes.c_int32) for k in ('rg_k', 'rg_npatch', 'rg_owned', 'pad4_')]
+                + [(k, ctypes.c_int32 * 6) for k in ('rg_cells', 'rg_edges')]
+                + [(k, _i32p) for k in ('rg_head', 'rg_cell', 'rg_slot', 'rg_edge', 'rg_ecell')])
 
 
 LAYER_SCRATCH = ('B', 'q', 'Tp', 'F', 'scale', 'G', 'He', 'ubs', 'ub0', 'ub', 'acc', 'eta0', 'eta', 'eta_prev', 'h1',

@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from . import _hip
-from .grid import d2_stencil  # noqa: F401  (re-exported, as the reference's gpu.d2_stencil)
+from .grid import d2_stencil, rings  # noqa: F401  (d2_stencil re-exported, as the reference's gpu.d2_stencil)
 
 PRECISION = os.environ.get('INSILICA_PRECISION', 'mixed')
 
@@ -31,7 +31,7 @@ def device():
 
 
 PATCH_CELLS = 64
-PATCH_PAIRS = True          # the air's fast sub-steps two per launch where the patches' LDS allows
+RING_STEPS = 4              # the rings of the fast sub-steps' patches: the most of them that one launch takes
 
 
 def fast_patches(grid, pcells=64):
@@ -180,21 +180,21 @@ _PATCHES = {}
 
 
 def patch_tables(grid):
-    """fast_patches and fast_patches2 of a mesh, built once per mesh topology: meshes scaled to other planets share
-    their index arrays with the level's mesh, so they share these tables too. Host work only (safe to call from a
-    worker thread)."""
-    key = (id(grid.eI), int(grid.N), PATCH_CELLS, PATCH_PAIRS)
+    """The transport's patches (fast_patches, transport_patches) of a mesh, and its rings, built once per mesh topology:
+    meshes scaled to other planets share their index arrays with the level's mesh, so they share these tables too. Host
+    work only (safe to call from a worker thread)."""
+    rings(grid, RING_STEPS)
+    key = (id(grid.eI), int(grid.N), PATCH_CELLS)
     hit = _PATCHES.get(key)
     if hit is None or hit[0] is not grid.eI:
         pt = fast_patches(grid, PATCH_CELLS)
-        p2 = fast_patches2(grid, pt) if pt is not None and PATCH_PAIRS else None
         if pt is not None and pt['pcells'] == 64:
             pt.update(transport_patches(grid, pt))
-        hit = (grid.eI, pt, p2)
+        hit = (grid.eI, pt)
         if len(_PATCHES) > 16:
             _PATCHES.clear()
         _PATCHES[key] = hit
-    return hit[1], hit[2]
+    return hit[1]
 
 
 class DeviceGrid:
@@ -235,9 +235,9 @@ class DeviceGrid:
             setattr(s, k, ctypes.cast(getattr(self, k).data_ptr(), _hip._f64p))
         for k in ('wf', 'd2wtf'):
             setattr(s, k, ctypes.cast(getattr(self, k).data_ptr(), _hip._f32p))
-        pt, p2 = patch_tables(grid)
+        pt = patch_tables(grid)
         if pt is not None:
-            # each edge's slot in its two cells' rings (where the stage's coefficients of its cells are written)
+            # each edge's slot in its two cells' rings
             self.eslot = put(edge_slots(grid), np.int8)
             s.eslot = ctypes.cast(self.eslot.data_ptr(), _hip._i8p)
             s.npatch, s.pcells, s.pslots = pt['npatch'], pt['pcells'], pt['pslots']
@@ -250,11 +250,15 @@ class DeviceGrid:
                 for k in ('pi_off', 'pi_edge', 'tc_slot'):
                     setattr(self, k, put(pt[k], np.int32))
                     setattr(s, k, ctypes.cast(getattr(self, k).data_ptr(), _hip._i32p))
-            if p2 is not None:
-                s.pslots2, s.pedges2 = p2['pslots2'], p2['pedges2']
-                for k in ('ph2_off', 'ph2_cell', 'px_off', 'px_edge', 'px_slot', 'pc_off', 'pc_eslot'):
-                    setattr(self, k, put(p2[k], np.int32))
-                    setattr(s, k, ctypes.cast(getattr(self, k).data_ptr(), _hip._i32p))
+        rg = rings(grid, RING_STEPS)
+        if rg is not None:
+            s.rg_k, s.rg_npatch, s.rg_owned = RING_STEPS, len(rg['head']), int(rg['owned'])
+            for r in range(6):
+                s.rg_cells[r], s.rg_edges[r] = int(rg['cells'][r]), int(rg['edges'][r])
+            for k in ('head', 'cell', 'slot', 'edge', 'ecell'):
+                t = put(rg[k], np.int32)
+                setattr(self, 'rg_' + k, t)
+                setattr(s, 'rg_' + k, ctypes.cast(t.data_ptr(), _hip._i32p))
         self.s = s
         self.ref = ctypes.byref(s)
         self._sum_scratch = None

@@ -51,6 +51,7 @@ def _native():
             'isw_mesh_hilbert': [i64, vp, i32, vp],
             'isw_mesh_trisk': [i64, i64, i64] + [vp] * 25,
             'isw_mesh_weights': [i64, i64] + [vp] * 14,
+            'isw_mesh_rings': [i64, i64, i32, i64] + [vp] * 11,
         }.items():
             f = getattr(L, name)
             f.restype, f.argtypes = ctypes.c_int, args
@@ -237,6 +238,54 @@ def make(n, order=None, lloyd=None):
     return Grid(g), time.perf_counter() - t0
 
 
+def rings(g, depth, pcells=64):
+    """The patches of `g` with `depth` rings of neighbours (isw_grid's rg_* tables, see csrc/mesh.cpp): a dict of int32
+    arrays head, cell, slot, edge, ecell, the most edges a patch owns (owned) and, per ring, the most cells and edges a patch
+    has within it (cells, edges: six values); None for a mesh with an edge lacking a cell or without cell positions. A union of meshes (its `parts`) has its parts' patches, in turn."""
+    parts = getattr(g, 'parts', None)
+    if parts is not None:
+        each = [rings(p, depth, pcells) for p in parts]
+        if any(r is None for r in each):
+            return None
+        out = {k: [] for k in ('head', 'cell', 'slot', 'edge', 'ecell')}
+        nc = ne = 0
+        for r, c0, e0 in zip(each, g.cell0, g.edge0):
+            head = r['head'].copy()
+            head[:, 0] += nc
+            head[:, 1] += ne
+            nc, ne = nc + len(r['cell']), ne + len(r['edge'])
+            out['head'].append(head)
+            out['cell'].append(r['cell'] + np.int32(c0))
+            out['edge'].append(r['edge'] + np.int32(e0))
+            out['slot'].append(r['slot'])
+            out['ecell'].append(r['ecell'])
+        return dict({k: np.concatenate(v) for k, v in out.items()},
+                    **{k: np.max([r[k] for r in each], axis=0) for k in ('cells', 'edges', 'owned')})
+    key = (id(g.eI), depth, pcells)
+    hit = _rings.get(key)
+    if hit is not None and hit[0] is g.eI:               # (meshes scaled to other planets share their index arrays)
+        return hit[1]
+    out = None
+    if getattr(g, 'pos', None) is not None and g.E > 0:
+        i32 = lambda a: np.ascontiguousarray(a, np.int32)
+        args = (g.N, g.E, depth, pcells, np.ascontiguousarray(g.pos, np.float64), i32(g.cellEdge),
+                np.ascontiguousarray(g.cellSign, np.int8), i32(g.eI), i32(g.eJ))
+        sizes = np.zeros(15, np.int64)
+        fn = _native().isw_mesh_rings
+        at = lambda a: a.ctypes.data if isinstance(a, np.ndarray) else a
+        if fn(*map(at, args), at(sizes), None, None, None, None, None) == 0:
+            nc, ne = int(sizes[0]), int(sizes[1])
+            t = dict(head=np.zeros(((g.N + pcells - 1) // pcells, 16), np.int32), cell=np.zeros(nc, np.int32),
+                     slot=np.zeros(3 * nc, np.int32), edge=np.zeros(ne, np.int32), ecell=np.zeros(ne, np.int32))
+            _call('isw_mesh_rings', *args, sizes, *t.values())
+            out = dict(t, owned=int(sizes[2]), cells=sizes[3:9].copy(), edges=sizes[9:].copy())
+    if len(_rings) > 16:
+        _rings.clear()
+    _rings[key] = (g.eI, out)
+    return out
+
+
+_rings = {}
 _loaded = {}
 
 

@@ -94,3 +94,44 @@ def test_transport_tables(n):
         assert np.array_equal((tc[m] & 1) == 1, eI[asc[cells][m]] == np.repeat(cells, 6).reshape(-1, 6)[m])
         assert len(edges) <= r['ptedges']
     assert np.all((r['tc_slot'] < 0) == (asc < 0))
+
+
+@pytest.mark.parametrize('n,pc,union', [(3, 64, False), (4, 64, False), (4, 50, False), (3, 64, True)])
+def test_ring_tables(n, pc, union):
+    """The ring patches: every cell and every edge of the mesh is owned once; each ring is exactly the neighbours of what
+    is inside it, its edge list exactly the edges they touch; every slot names its cell's edge with its sign, every
+    edge's places name its cells, as far as the kernels read them; a union's patches stay inside its parts."""
+    from insilica.batch import UnionGrid
+    from insilica.grid import rings
+    K = 5
+    g = UnionGrid([gridmod.get(n), gridmod.get(n - 1), gridmod.get(n)]) if union else gridmod.get(n)
+    t = rings(g, K, pc)
+    eI, eJ, ce, sg = (np.asarray(getattr(g, k)).astype(np.int64) for k in ('eI', 'eJ', 'cellEdge', 'cellSign'))
+    cells_seen, edges_seen = [], []
+    for b, h in enumerate(t['head']):
+        nc, ne = h[3:4 + K], h[4 + K:5 + 2 * K]
+        C, G = t['cell'][h[0]:h[0] + nc[K]], t['edge'][h[1]:h[1] + ne[K]]
+        assert len(np.unique(C)) == len(C) and len(np.unique(G)) == len(G) and nc[0] <= pc
+        assert h[2] <= t['owned'] and np.all(nc <= t['cells'][:K + 1]) and np.all(ne <= t['edges'][:K + 1])
+        assert np.array_equal(np.sort(G[:h[2]]), np.flatnonzero(np.isin(eI, C[:nc[0]])))
+        for r in range(K + 1):
+            e = ce[C[:nc[r]]]
+            assert np.array_equal(np.sort(G[:ne[r]]), np.unique(e[e >= 0]))
+            if r:
+                inner = G[:ne[r - 1]]
+                assert np.array_equal(np.sort(C[:nc[r]]), np.unique(np.concatenate([eI[inner], eJ[inner]])))
+        s = t['slot'][3 * h[0]:3 * (h[0] + nc[K])].reshape(-1, 3).astype(np.int64) & 0xffffffff
+        s6 = np.stack([s & 0xffff, s >> 16], axis=2).reshape(-1, 6)
+        has = ce[C] >= 0
+        assert np.array_equal((s6 & 0x7fff) != 0x7fff, has)
+        assert np.array_equal(G[(s6 & 0x7fff)[has]], ce[C][has])
+        assert np.array_equal((s6[has] & 0x8000) != 0, sg[C][has] < 0)
+        read = slice(h[1], h[1] + ne[K - 1])
+        first, second = unpack(t['ecell'][read])
+        assert np.array_equal(C[first], eI[G[:ne[K - 1]]]) and np.array_equal(C[second], eJ[G[:ne[K - 1]]])
+        if union:
+            assert len(np.unique(g.world_cell[C])) == 1
+        cells_seen.append(C[:nc[0]])
+        edges_seen.append(G[:h[2]])
+    assert np.array_equal(np.sort(np.concatenate(cells_seen)), np.arange(g.N))
+    assert np.array_equal(np.sort(np.concatenate(edges_seen)), np.arange(g.E))
