@@ -614,6 +614,17 @@ struct RingCell {
     }
     return ((((t[0] + t[1]) + t[2]) + t[3]) + t[4]) + t[5];
   }
+  // What flows out of the cell.
+  __device__ __forceinline__ double out(const double* F) const {
+    double s = 0;
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      const double f = F[at[k]];
+      const double x = __hiloint2double((int)((unsigned)__double2hiint(f) ^ flip[k]), __double2loint(f));
+      if (x > 0) s += x;
+    }
+    return s;
+  }
 };
 // x / d with r = 1 / d at hand: the plain form's rounds as the division does (a quotient corrected by its exact
 // remainder), the mixed form's is the product (its Div holds reciprocals).
@@ -990,6 +1001,125 @@ __global__ __launch_bounds__(BS) void k_limit_h(isw_grid g, Div dv, FluxSrc fs, 
   }
   const double v0 = h0[t];
   hn[t] = v0 - DIVBY(cdt * div, dv.A[i]);
+}
+
+// The limiter and the update in one launch on the grid's ring patches (k_scale, k_limit_h and the ocean's k_lay_u): a
+// block leaves the stage's fluxes of its patch's and first ring's edges in LDS, each formed once (a pass over cells forms
+// every edge's twice, in each of two passes: at level 7, two layers, 31 + 41 us and 7 us for the winds), then the scales
+// of patch and ring, then limits its patch's edges and steps its cells. ring_h0: the step's starting thickness, read for
+// the ring's cells too (where the stage writes over it the copy `keep` that the first stage left). Bound by its chain of
+// loads at the smaller levels; the sums are in cellEdge order.
+template <int L>
+__global__ __launch_bounds__(RBS) void k_limit_rings(isw_grid g, Div dv, FluxSrc fs, double cdt, double dt, double floor_,
+                                                     const double* __restrict__ ring_h0, double* __restrict__ keep,
+                                                     double* __restrict__ hn, double* __restrict__ Fm,
+                                                     const double* u0, const double* __restrict__ Tp,
+                                                     const double* __restrict__ ub_end, const double* __restrict__ ub0,
+                                                     double* un) {
+  constexpr int EPT = 2, PE = EPT * RBS + 2, PC = RBS / 2;
+  extern __shared__ double sm[];
+  double* F = sm;                                  // [L][PE] l_e F, the last but one 0
+  double* sc = sm + L * PE;                        // [L][PC] the cells' scales
+  const int N = g.N, E = g.E, t = (int)threadIdx.x;
+  const Ring r = ring_of(g);
+  const int nc0 = r.cells(0), nc1 = r.cells(1), ne0 = r.edges(0), ne1 = r.edges(1);
+  int e_[EPT], ec[EPT];
+  double f[EPT][L], le[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ne1) e_[j] = g.rg_edge[r.e0 + q];
+    if (q < ne0) ec[j] = g.rg_ecell[r.e0 + q];
+  }
+  // two threads to a cell, each taking every other layer
+  const int cq = t >> 1, l0 = t & 1;
+  int ci = 0;
+  RingCell rc;
+  double A = 0, h0[(L + 1) / 2];
+  if (cq < nc1) {
+    ci = g.rg_cell[r.c0 + cq];
+    rc.set(g.rg_slot + 3 * (size_t)(r.c0 + cq), PE - 2);
+  }
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ne1) {
+      const int e = e_[j];
+      le[j] = g.le[e];
+      const double inv_n = fs.we ? fs.winv[fs.we[e] * 3 + fs.stage] : fs.inv_n;
+      const double ub = fs.air ? 0.0 : fs.ubs[e], ba = fs.air ? 0.0 : fs.bacc[e] * inv_n;
+      const bool wall = !fs.air && fs.wall && fs.wall[e] == 0;
+#pragma unroll
+      for (int l = 0; l < L; l++) {
+        const size_t o = (size_t)l * E + e;
+        const double he = fs.hedge[o];
+        f[j][l] = fs.air ? he * fs.acc[o] * inv_n : wall ? 0.0 : he * (fs.us[o] - ub) + he * ba;
+      }
+    }
+  }
+  if (cq < nc1) {
+    A = g.areaCell[ci];
+#pragma unroll
+    for (int k = 0; k < (L + 1) / 2; k++)
+      if (l0 + 2 * k < L) h0[k] = ring_h0[(size_t)(l0 + 2 * k) * N + ci];
+  }
+  // the ocean's winds, of the owned edges
+  if (un && t < r.own) {
+    const int e = e_[0];
+    const double db = ub_end[e] - ub0[e];
+    const bool wall = fs.wall && fs.wall[e] == 0;
+#pragma unroll
+    for (int l = 0; l < L; l++) {
+      const size_t o = (size_t)l * E + e;
+      un[o] = wall ? 0.0 : u0[o] + cdt * Tp[o] + db;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ne1)
+#pragma unroll
+      for (int l = 0; l < L; l++) F[l * PE + q] = f[j][l] * le[j];
+  }
+  if (t < L) F[t * PE + PE - 2] = 0.0;
+  __syncthreads();
+  if (cq < nc1) {
+#pragma unroll
+    for (int k = 0; k < (L + 1) / 2; k++) {
+      const int l = l0 + 2 * k;
+      if (l >= L) continue;
+      const double out = rc.out(F + l * PE) * cdt;
+      const double avail = h0[k] - floor_;
+      const double cap = (avail > 0 ? avail : 0.0) * A;
+      sc[l * PC + cq] = out > cap ? cap / out : 1.0;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int q = t + j * RBS;
+    if (q < ne0) {
+      const int cI = ec[j] & 0xffff, cJ = ec[j] >> 16;
+#pragma unroll
+      for (int l = 0; l < L; l++) {
+        const double fl = f[j][l] * sc[l * PC + (f[j][l] > 0 ? cI : cJ)], lf = le[j] * fl;
+        F[l * PE + q] = lf;
+        if (Fm && q < r.own) Fm[(size_t)l * E + e_[j]] = lf * dt;
+      }
+    }
+  }
+  __syncthreads();
+  if (cq < nc0) {
+    const double Ad = dv.A[ci], rA = recip(Ad);
+#pragma unroll
+    for (int k = 0; k < (L + 1) / 2; k++) {
+      const int l = l0 + 2 * k;
+      if (l >= L) continue;
+      const size_t o = (size_t)l * N + ci;
+      hn[o] = h0[k] - over(cdt * rc.div(F + l * PE), Ad, rA);
+      if (keep) keep[o] = h0[k];
+    }
+  }
 }
 
 __global__ __launch_bounds__(BS) void k_lay_u(int E, int L, double cdt, const double* u0, const double* __restrict__ Tp,
@@ -1840,6 +1970,30 @@ static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div
     fs.wall = s->wall;
   }
   const double fb = flux_bytes(fs, n_, e_, l_);
+  if (g->rg_head && g->rg_cells[1] <= RBS / 2 && g->rg_edges[1] <= 2 * RBS && g->rg_owned <= RBS) {
+    // one launch on the ring patches; the first stage keeps the starting thickness for the last, which writes over it
+    fs.hedge = s->hedge;
+    const bool over_h0 = hn == h0;
+#define LIMIT(LL)                                                                                                  \
+  ISW_LAUNCH_SHM("limit_rings", fb + 3 * l_ * n_ * D + n_ * D + e_ * D + 4 * n_ * I + 2 * e_ * I +                     \
+                                    (Fm ? l_ * e_ * D : 0) + (s->air ? 0 : 3 * l_ * e_ * D + 2 * e_ * D),            \
+                 k_limit_rings<LL>, dim3((unsigned)g->rg_npatch), dim3(RBS),                                        \
+                 (size_t)LL * (2 * RBS + 2 + RBS / 2) * sizeof(double), *g, dv, fs, c * dt, dt, s->floor_,            \
+                 over_h0 ? s->hold : h0, si == 0 ? s->hold : nullptr, hn, Fm, u0, s->Tp, s->ub, s->ub0,               \
+                 s->air ? nullptr : un)
+    switch (L) {
+      case 1: LIMIT(1); break;
+      case 2: LIMIT(2); break;
+      case 3: LIMIT(3); break;
+      case 4: LIMIT(4); break;
+      case 5: LIMIT(5); break;
+      case 6: LIMIT(6); break;
+      case 7: LIMIT(7); break;
+      default: LIMIT(8); break;
+    }
+#undef LIMIT
+    return;
+  }
   ISW_LAUNCH("scale", fb + 6 * n_ * I + 2 * e_ * I + e_ * D + l_ * n_ * D + n_ * D + l_ * n_ * D,
              k_scale, g1((long)N * L), BS, *g, fs, c * dt, s->floor_, h0, s->scale, L);
   ISW_LAUNCH("limit_h", fb + 6 * n_ * (I + C) + 2 * e_ * I + e_ * D + 3 * l_ * n_ * D + n_ * D +
