@@ -139,9 +139,12 @@ typedef struct isw_layers {
 } isw_layers;
 
 /* FCT transport scratch for up to rows_max rows (reference: src/insilica/transport.py:19-30 Transport.__init__).
- * (rows,N): td, p1, p2, Rp, Rm; (rows,E): Hf, A; pf: (rows,N) floats for the mixed form's stencil copy, else NULL. */
+ * (rows,N): td, p1, p2, Rp, Rm; (rows,E): Hf, A; pf: (rows,N) floats for the mixed form's stencil copy, else NULL;
+ * with rows_pad, of that many rows each, 16-byte aligned. */
 typedef struct isw_transport {
-  int32_t L, rows_max, prec, pad_;
+  int32_t L, rows_max, prec;
+  int32_t rows_pad; /* the rows every scratch array holds: at least the rows rounded up to a multiple of four lets the
+                     * passes keep them cell-major on the grid's patches; less (0) keeps them apart */
   double beta;
   double *td, *p1, *p2, *Rp, *Rm, *Hf, *A;
   float *pf;

@@ -1324,11 +1324,18 @@ __device__ __forceinline__ double upwind(const double* Fml, const double* p, con
 // stencil on `psf` (the field itself in the plain form, its FP32 copy in the mixed form) with weights wt.
 // The high-order flux of one edge from its stencil (eight cells ix with weights w, its two cells I, J), for the
 // tracer row ps (psf its stencil copy) and the edge's mass flux f.
+__device__ __forceinline__ double hoflux_of(double f, double pI, double pJ, const fast (&v)[8], const fast (&w)[8],
+                                            double beta) {
+  const fast a = w[0] * v[0] + w[1] * v[1] + w[2] * v[2] + w[3] * v[3];
+  const fast b = w[4] * v[4] + w[5] * v[5] + w[6] * v[6] + w[7] * v[7];
+  return f * (0.5 * (pI + pJ) - (double)(a + b)) + fabs(f) * ((double)(b - a) * beta);
+}
 __device__ __forceinline__ double hoflux_at(double f, const double* ps, const fast* psf, const int (&ix)[8],
                                             const fast (&w)[8], int I, int J, double beta) {
-  const fast a = w[0] * psf[ix[0]] + w[1] * psf[ix[1]] + w[2] * psf[ix[2]] + w[3] * psf[ix[3]];
-  const fast b = w[4] * psf[ix[4]] + w[5] * psf[ix[5]] + w[6] * psf[ix[6]] + w[7] * psf[ix[7]];
-  return f * (0.5 * (ps[I] + ps[J]) - (double)(a + b)) + fabs(f) * ((double)(b - a) * beta);
+  fast v[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) v[k] = psf[ix[k]];
+  return hoflux_of(f, ps[I], ps[J], v, w, beta);
 }
 __device__ __forceinline__ void stencil_at(const isw_grid& g, const fast* wt, int e, int (&ix)[8], fast (&w)[8]) {
   const int o = e * 8;
@@ -1416,69 +1423,298 @@ __global__ __launch_bounds__(BS) void k_tr_stage(isw_grid g, int Lm, int rows, d
   if (pf) pf[o] = (float)r;
 }
 
-// One RK stage of the transport in one launch on the grid's 64-cell patches (k_tr_hflux then k_tr_stage): block
-// (patch, four rows) first computes the third-order flux of every edge of its cells -- its own edges and those
-// whose second cell only is in the patch, the latter also computed by the neighbour that owns them, from the same
-// inputs, so every copy is the same to the bit -- into LDS, then steps its 64 cells x 4 rows from there. The flux
-// array's write and re-read (rows x E doubles each way) and one kernel boundary go away; the arithmetic and every
-// sum's order are k_tr_hflux's and k_tr_stage's. pfo: the output's FP32 copy (mixed form; the stencil reads srcf,
-// a different buffer, so no block overwrites what another still reads).
-__global__ __launch_bounds__(BS) void k_tr_hstage(isw_grid g, int Lm, int rows, double frac, double beta,
-                                                  const double* __restrict__ src, const fast* __restrict__ srcf,
-                                                  const fast* __restrict__ wt, const double* __restrict__ Fm,
-                                                  const double* __restrict__ M0, const double* __restrict__ psi,
-                                                  double* __restrict__ out, float* __restrict__ pfo) {
-  extern __shared__ double hs[];                   // [4][ptedges] the stage flux of the patch's edges, per row
-  const int PT = g.ptedges, N = g.N, E = g.E;
-  const int b = xblock();
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int y = blockIdx.y * 4 + ty;
-  const bool rowok = y < rows;
-  const int l = y % Lm;
-  const int e0 = g.pe_off[b], ne = g.pe_off[b + 1] - e0;
-  const int i0 = g.pi_off[b], ni = g.pi_off[b + 1] - i0;
-  // the stage flux of the patch's edges for the block's four rows: thread t takes edges t, t + BS, ..., each edge's
-  // stencil (its eight cells and weights, its two cells) loaded once for the four rows
-  const int y0 = blockIdx.y * 4, nq = ne + ni;
-  for (int q = ty * BS1 + tx; q < nq; q += BS) {
-    const int e = q < ne ? g.pe_edge[e0 + q] : g.pi_edge[i0 + q - ne];
-    int ix[8];
-    fast w[8];
-    stencil_at(g, wt, e, ix, w);
-    const int I = g.eI[e], J = g.eJ[e];
+// ---------------------------------------------------------------------------------------------------------------
+// The transport on the grid's 64-cell patches. Its scratch holds the rows cell-major, padded to RS, a multiple of four
+// (cell i's rows at i * RS ..), so that a stencil's gather of one cell brings four rows in one load: with the rows apart
+// (as psi is) each load of a wave touched seventeen lines for 64 values, and every pass was bound by that (15 rows at
+// level 6: tr_td 16.5, each stage 23, tr_aflux 14.4, tr_ratios 15.1, tr_apply 17.1 us). A block takes a patch and RC (4 or
+// 8) rows; a lane takes four rows of an edge, then two rows of a cell. Each pass forms the fluxes of every edge of its
+// cells -- the patch's own edges and those whose second cell only is in it, the latter also formed by the neighbour that
+// owns them, from the same inputs, so every copy is the same to the bit -- in LDS, then steps its cells from there (15 rows
+// at level 6, mixed: the stages 48.5 us for both, tr_limit 27.3, tr_correct 14.4, tr_turn 5.8: 1.6 to 2.7 TB/s of the bytes
+// each cannot do without; one row to a load was 105.4 for all, 120.6 with the rows apart). What is left is the latency of
+// the chain edge -> stencil -> eight gathers and the edges formed twice (a patch's rim, a sixth of its edges). The
+// arithmetic and every sum's order are k_tr_td's, k_tr_hflux's, k_tr_stage's, k_tr_aflux's, k_tr_ratios's and
+// k_tr_apply's; the padding rows hold zeros.
+// ---------------------------------------------------------------------------------------------------------------
+// A block's patch and rows: blocks run over a patch's row chunks first, so that one XCD's L2 serves them all.
+struct TrBlock {
+  int b, y0, e0, ne, i0, nq;
+  __device__ __forceinline__ int edge(const isw_grid& g, int q) const {
+    return q < ne ? g.pe_edge[e0 + q] : g.pi_edge[i0 + q - ne];
+  }
+};
+__device__ __forceinline__ TrBlock tr_block(const isw_grid& g, int chunks, int rc) {
+  TrBlock t;
+  const int x = xblock();
+  t.b = x / chunks;
+  t.y0 = (x - t.b * chunks) * rc;
+  t.e0 = g.pe_off[t.b];
+  t.ne = g.pe_off[t.b + 1] - t.e0;
+  t.i0 = g.pi_off[t.b];
+  t.nq = t.ne + g.pi_off[t.b + 1] - t.i0;
+  return t;
+}
+// Four (or two) rows of a cell or an edge, in 16-byte loads where the width allows.
+__device__ __forceinline__ void rows4(const double* p, double (&v)[4]) {
+  const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
+  v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+}
+__device__ __forceinline__ void rows4(const float* p, float (&v)[4]) {
+  const float4 a = *reinterpret_cast<const float4*>(p);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void put4(double* p, const double (&v)[4]) {
+  reinterpret_cast<double2*>(p)[0] = make_double2(v[0], v[1]);
+  reinterpret_cast<double2*>(p)[1] = make_double2(v[2], v[3]);
+}
+__device__ __forceinline__ double2 rows2(const double* p) { return *reinterpret_cast<const double2*>(p); }
+// The third-order fluxes of four rows of an edge with mass fluxes f, of the field whose rows at the edge's cells are pI,
+// pJ, its stencil copy psf.
+__device__ __forceinline__ void hoflux4(const fast* __restrict__ psf, const fast* __restrict__ wt, const isw_grid& g,
+                                        int RS, int e, int yr, const double (&f)[4], const double (&pI)[4],
+                                        const double (&pJ)[4], double beta, double (&h)[4]) {
+  int ix[8];
+  fast w[8], v[8][4];
+  stencil_at(g, wt, e, ix, w);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int yr = y0 + r;
-      if (yr < rows) {
-        const double f = Fm[(size_t)(yr % Lm) * E + e];
-        hs[r * PT + q] = frac * hoflux_at(f, src + (size_t)yr * N, srcf + (size_t)yr * N, ix, w, I, J, beta);
-      }
+  for (int k = 0; k < 8; k++) rows4(psf + (size_t)ix[k] * RS + yr, v[k]);
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const fast x[8] = {v[0][r], v[1][r], v[2][r], v[3][r], v[4][r], v[5][r], v[6][r], v[7][r]};
+    h[r] = hoflux_of(f[r], pI[r], pJ[r], x, w, beta);
+  }
+}
+// The mass fluxes of the rows' layers on an edge.
+__device__ __forceinline__ void tr_mass(const double* __restrict__ Fm, int E, int Lm, int e, int yr, double (&f)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; r++) f[r] = Fm[(size_t)((yr + r) % Lm) * E + e];
+}
+// Two rows of a cell moved by the fluxes in LDS (four rows to a place, from hs), in cellEdgeAsc order.
+template <int RC>
+__device__ __forceinline__ double2 tr_moved(double2 t, const double* hs, const int (&sl)[6]) {
+  double2 fv[6];
+#pragma unroll
+  for (int k = 0; k < 6; k++) fv[k] = rows2(hs + (sl[k] < 0 ? 0 : sl[k] >> 1) * RC);
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    if (sl[k] < 0) break;
+    if (sl[k] & 1) { t.x -= fv[k].x; t.y -= fv[k].y; } else { t.x += fv[k].x; t.y += fv[k].y; }
+  }
+  return t;
+}
+
+// psi (rows, N) cell-major, and its FP32 copy (mixed form): 64 cells x 16 rows through LDS.
+__global__ __launch_bounds__(BS) void k_tr_turn(int N, int rows, int RS, const double* __restrict__ psi,
+                                                double* __restrict__ out, float* __restrict__ pf) {
+  __shared__ double s[16][BS1 + 1];
+  const int i0 = xblock() * BS1, y0 = blockIdx.y * 16, t = (int)threadIdx.x;
+  for (int x = t; x < 16 * BS1; x += BS) {
+    const int y = x >> 6, c = x & 63;
+    s[y][c] = y0 + y < rows && i0 + c < N ? psi[(size_t)(y0 + y) * N + i0 + c] : 0.0;
+  }
+  __syncthreads();
+  const int nr = min(16, RS - y0);
+  for (int x = t; x < nr * BS1; x += BS) {
+    const int c = x / nr, y = x - c * nr;
+    if (i0 + c >= N) break;
+    const size_t o = (size_t)(i0 + c) * RS + y0 + y;
+    out[o] = s[y][c];
+    if (pf) pf[o] = (float)s[y][c];
+  }
+}
+
+// One RK stage: the third-order fluxes of src (cell-major, stencil copy srcf) and the step of psi by frac of them. The
+// first also steps psi upwind (td). pfo: the output's FP32 copy (the stencil reads srcf, a different buffer, so no block
+// overwrites what another still reads).
+template <int RC, bool TD>
+__global__ __launch_bounds__(BS) void k_tr_move(isw_grid g, int Lm, int RS, int chunks, double frac, double beta,
+                                                const double* __restrict__ src, const fast* __restrict__ srcf,
+                                                const fast* __restrict__ wt, const double* __restrict__ Fm,
+                                                const double* __restrict__ M0, const double* __restrict__ M1,
+                                                const double* __restrict__ psi, double* __restrict__ out,
+                                                float* __restrict__ pfo, double* __restrict__ td) {
+  extern __shared__ double sm[];
+  const int PT = g.ptedges, N = g.N;
+  double* hs = sm;                                 // [edge][RC] the stage's fluxes
+  double* us = hs + PT * RC;                       // [edge][RC] (TD) the upwind fluxes
+  const TrBlock t = tr_block(g, chunks, RC);
+  constexpr int Q = RC / 4, P = RC / 2;
+  for (int x = (int)threadIdx.x; x < t.nq * Q; x += BS) {
+    const int q = x / Q, y = (x - q * Q) * 4, yr = t.y0 + y;
+    if (yr >= RS) continue;
+    const int e = t.edge(g, q), I = g.eI[e], J = g.eJ[e];
+    double f[4], pI[4], pJ[4], h[4];
+    tr_mass(Fm, g.E, Lm, e, yr, f);
+    rows4(src + (size_t)I * RS + yr, pI);
+    rows4(src + (size_t)J * RS + yr, pJ);
+    hoflux4(srcf, wt, g, RS, e, yr, f, pI, pJ, beta, h);
+#pragma unroll
+    for (int r = 0; r < 4; r++) h[r] = frac * h[r];
+    put4(hs + q * RC + y, h);
+    if (TD) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) h[r] = f[r] * (f[r] >= 0 ? pI[r] : pJ[r]);
+      put4(us + q * RC + y, h);
     }
   }
   __syncthreads();
-  const int i = b * BS1 + tx;
-  if (!rowok || i >= N) return;
-  const size_t o = (size_t)y * N + i, om = (size_t)l * N + i;
-  const double* Fml = Fm + (size_t)l * E;
-  int e[6], sl[6];
-  ring6(g.cellEdgeAsc, i, e);
-  ring6(g.tc_slot, i, sl);
-  double fv[6], mv[6];
+  for (int x = (int)threadIdx.x; x < BS1 * P; x += BS) {
+    const int c = x / P, y = (x - c * P) * 2, yr = t.y0 + y, i = t.b * BS1 + c;
+    if (yr >= RS || i >= N) continue;
+    const size_t o = (size_t)i * RS + yr;
+    const int la = yr % Lm, lb = (yr + 1) % Lm;
+    int sl[6], e[6];
+    ring6(g.tc_slot, i, sl);
+    ring6(g.cellEdgeAsc, i, e);
+    double ma[6], mb[6];
 #pragma unroll
-  for (int k = 0; k < 6; k++) {
-    fv[k] = hs[ty * PT + (sl[k] < 0 ? 0 : sl[k] >> 1)];
-    mv[k] = frac * Fml[ok0(e[k])];
-  }
-  double t = M0[om] * psi[o];
-  double mx = M0[om];
+    for (int k = 0; k < 6; k++) {
+      ma[k] = frac * Fm[(size_t)la * g.E + ok0(e[k])];
+      mb[k] = frac * Fm[(size_t)lb * g.E + ok0(e[k])];
+    }
+    const double2 ps = rows2(psi + o), m0 = make_double2(M0[(size_t)la * N + i], M0[(size_t)lb * N + i]);
+    const double2 mp = make_double2(m0.x * ps.x, m0.y * ps.y);
+    double2 mx = m0;
 #pragma unroll
-  for (int k = 0; k < 6; k++) {
-    if (e[k] < 0) break;
-    if (sl[k] & 1) { t -= fv[k]; mx -= mv[k]; } else { t += fv[k]; mx += mv[k]; }
+    for (int k = 0; k < 6; k++) {
+      if (sl[k] < 0) break;
+      if (sl[k] & 1) { mx.x -= ma[k]; mx.y -= mb[k]; } else { mx.x += ma[k]; mx.y += mb[k]; }
+    }
+    double2 r = tr_moved<RC>(mp, hs + y, sl);
+    r.x /= mx.x;
+    r.y /= mx.y;
+    *reinterpret_cast<double2*>(out + o) = r;
+    if (pfo) *reinterpret_cast<float2*>(pfo + o) = make_float2((float)r.x, (float)r.y);
+    if (TD) {
+      r = tr_moved<RC>(mp, us + y, sl);
+      r.x /= M1[(size_t)la * N + i];
+      r.y /= M1[(size_t)lb * N + i];
+      *reinterpret_cast<double2*>(td + o) = r;
+    }
   }
-  const double r = t / mx;
-  out[o] = r;
-  if (pfo) pfo[o] = (float)r;
+}
+
+// The antidiffusive fluxes (the third-order ones of p2 less the upwind ones of psi; A, edge-major by rows, written by each
+// edge's first cell's patch) and the limiter's ratios.
+template <int RC>
+__global__ __launch_bounds__(BS) void k_tr_limit(isw_grid g, int Lm, int RS, int chunks, double beta,
+                                                 const double* __restrict__ psi, const double* __restrict__ p2,
+                                                 const fast* __restrict__ p2f, const fast* __restrict__ wt,
+                                                 const double* __restrict__ Fm, const double* __restrict__ td,
+                                                 const double* __restrict__ M1, double* __restrict__ A,
+                                                 double* __restrict__ Rp, double* __restrict__ Rm) {
+  extern __shared__ double sm[];
+  const int N = g.N;
+  double* as = sm;                                 // [edge][RC]
+  const TrBlock t = tr_block(g, chunks, RC);
+  constexpr int Q = RC / 4, P = RC / 2;
+  for (int x = (int)threadIdx.x; x < t.nq * Q; x += BS) {
+    const int q = x / Q, y = (x - q * Q) * 4, yr = t.y0 + y;
+    if (yr >= RS) continue;
+    const int e = t.edge(g, q), I = g.eI[e], J = g.eJ[e];
+    double f[4], pI[4], pJ[4], uI[4], uJ[4], h[4];
+    tr_mass(Fm, g.E, Lm, e, yr, f);
+    rows4(p2 + (size_t)I * RS + yr, pI);
+    rows4(p2 + (size_t)J * RS + yr, pJ);
+    rows4(psi + (size_t)I * RS + yr, uI);
+    rows4(psi + (size_t)J * RS + yr, uJ);
+    hoflux4(p2f, wt, g, RS, e, yr, f, pI, pJ, beta, h);
+#pragma unroll
+    for (int r = 0; r < 4; r++) h[r] -= f[r] * (f[r] >= 0 ? uI[r] : uJ[r]);
+    put4(as + q * RC + y, h);
+    if (q < t.ne) put4(A + (size_t)e * RS + yr, h);
+  }
+  __syncthreads();
+  for (int x = (int)threadIdx.x; x < BS1 * P; x += BS) {
+    const int c = x / P, y = (x - c * P) * 2, yr = t.y0 + y, i = t.b * BS1 + c;
+    if (yr >= RS || i >= N) continue;
+    const size_t o = (size_t)i * RS + yr;
+    int nb[6], sl[6];
+    ring6(g.nbr, i, nb);
+    ring6(g.tc_slot, i, sl);
+    double2 pv[6], tv[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      pv[k] = rows2(psi + (size_t)ok0(nb[k]) * RS + yr);
+      tv[k] = rows2(td + (size_t)ok0(nb[k]) * RS + yr);
+    }
+    const double2 pi = rows2(psi + o), ti = rows2(td + o);
+    double2 hi = make_double2(fmax(pi.x, ti.x), fmax(pi.y, ti.y)), lo = make_double2(fmin(pi.x, ti.x), fmin(pi.y, ti.y));
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      if (nb[k] < 0) break;
+      hi.x = fmax(hi.x, fmax(pv[k].x, tv[k].x));
+      hi.y = fmax(hi.y, fmax(pv[k].y, tv[k].y));
+      lo.x = fmin(lo.x, fmin(pv[k].x, tv[k].x));
+      lo.y = fmin(lo.y, fmin(pv[k].y, tv[k].y));
+    }
+    const double m1a = M1[(size_t)(yr % Lm) * N + i], m1b = M1[(size_t)((yr + 1) % Lm) * N + i];
+    double2 Pp = make_double2(0, 0), Pm = Pp;
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      if (sl[k] < 0) break;
+      const double2 a = rows2(as + (sl[k] >> 1) * RC + y);
+      if (sl[k] & 1) {
+        if (a.x > 0) Pm.x += a.x; else Pp.x -= a.x;
+        if (a.y > 0) Pm.y += a.y; else Pp.y -= a.y;
+      } else {
+        if (a.x > 0) Pp.x += a.x; else Pm.x -= a.x;
+        if (a.y > 0) Pp.y += a.y; else Pm.y -= a.y;
+      }
+    }
+    auto share = [](double room, double need) { return need > 0 ? fmin(1.0, room / need) : 0.0; };
+    *reinterpret_cast<double2*>(Rp + o) =
+        make_double2(share((hi.x - ti.x) * m1a, Pp.x), share((hi.y - ti.y) * m1b, Pp.y));
+    *reinterpret_cast<double2*>(Rm + o) =
+        make_double2(share((ti.x - lo.x) * m1a, Pm.x), share((ti.y - lo.y) * m1b, Pm.y));
+  }
+}
+
+// The upwind step corrected by the limited antidiffusive fluxes, back into psi's rows through LDS.
+template <int RC>
+__global__ __launch_bounds__(BS) void k_tr_correct(isw_grid g, int Lm, int rows, int RS, int chunks,
+                                                   const double* __restrict__ td, const double* __restrict__ M1,
+                                                   const double* __restrict__ A, const double* __restrict__ Rp,
+                                                   const double* __restrict__ Rm, double* __restrict__ out) {
+  extern __shared__ double sm[];
+  __shared__ double turn[RC][BS1 + 1];
+  double* as = sm;                                 // [edge][RC] the limited fluxes
+  const int N = g.N;
+  const TrBlock t = tr_block(g, chunks, RC);
+  constexpr int Q = RC / 4, P = RC / 2;
+  for (int x = (int)threadIdx.x; x < t.nq * Q; x += BS) {
+    const int q = x / Q, y = (x - q * Q) * 4, yr = t.y0 + y;
+    if (yr >= RS) continue;
+    const int e = t.edge(g, q);
+    const size_t oi = (size_t)g.eI[e] * RS + yr, oj = (size_t)g.eJ[e] * RS + yr;
+    double a[4], pi[4], pj[4], mi[4], mj[4];
+    rows4(A + (size_t)e * RS + yr, a);
+    rows4(Rp + oi, pi);
+    rows4(Rp + oj, pj);
+    rows4(Rm + oi, mi);
+    rows4(Rm + oj, mj);
+#pragma unroll
+    for (int r = 0; r < 4; r++) a[r] *= a[r] > 0 ? fmin(pj[r], mi[r]) : fmin(pi[r], mj[r]);
+    put4(as + q * RC + y, a);
+  }
+  __syncthreads();
+  for (int x = (int)threadIdx.x; x < BS1 * P; x += BS) {
+    const int c = x / P, y = (x - c * P) * 2, yr = t.y0 + y, i = t.b * BS1 + c;
+    if (yr >= RS || i >= N) continue;
+    int sl[6];
+    ring6(g.tc_slot, i, sl);
+    const double m1a = M1[(size_t)(yr % Lm) * N + i], m1b = M1[(size_t)((yr + 1) % Lm) * N + i];
+    const double2 ti = rows2(td + (size_t)i * RS + yr);
+    const double2 r = tr_moved<RC>(make_double2(ti.x * m1a, ti.y * m1b), as + y, sl);
+    turn[y][c] = r.x / m1a;
+    turn[y + 1][c] = r.y / m1b;
+  }
+  __syncthreads();
+  for (int x = (int)threadIdx.x; x < BS1 * RC; x += BS) {
+    const int y = x >> 6, c = x & 63;
+    if (t.y0 + y < rows && t.b * BS1 + c < N) out[(size_t)(t.y0 + y) * N + t.b * BS1 + c] = turn[y][c];
+  }
 }
 
 __global__ __launch_bounds__(BS) void k_tr_aflux(isw_grid g, int Lm, int rows, double beta, const double* __restrict__ psi,
@@ -2093,6 +2329,46 @@ int transport_step(const isw_grid* g, const isw_transport* tr, const double* M0,
   float* pf = nullptr;
   const fast* wt = g->d2wt;
 #endif
+  // On the patches with the rows cell-major, where the scratch holds them padded: psi's cell-major copy is in Hf, the FP32
+  // copies alternate between pf and pf2 (stage 1 writes p1's to pf2; stage 2 reads it and writes p2's to pf). Eight rows to
+  // a block share its edges' tables twice as often as four (15 rows at level 6: 96.1 us of kernels against 110.4); four
+  // where no more are there
+  const int RS = (rows + 3) / 4 * 4, RC = RS > 4 ? 8 : 4, chunks = (RS + RC - 1) / RC;
+  const size_t lds = (size_t)g->ptedges * RC * sizeof(double);
+  if (order == 3 && g->pi_off && g->pcells == BS1 && E >= N && RS <= tr->rows_pad && (!ISW_FORM_MIXED || tr->pf2) &&
+      2 * lds <= 65536) {
+    const double tabs = 2 * e_ * I + 6 * n_ * I, edge1 = 8 * e_ * (R + I) + l_ * e_ * D + 2 * e_ * I;
+    double* pc = tr->Hf;
+#if ISW_FORM_MIXED
+    float *pfa = tr->pf, *pfb = tr->pf2;
+    const fast *f0 = pfa, *f1 = pfb, *f2 = pfa;
+#else
+    float *pfa = nullptr, *pfb = nullptr;
+    const fast *f0 = pc, *f1 = tr->p1, *f2 = tr->p2;
+#endif
+    const dim3 gp((unsigned)(g->npatch * chunks));
+    ISW_LAUNCH("tr_turn", 2 * r_ * n_ * D + mixed * r_ * n_ * 4, k_tr_turn,
+               dim3((unsigned)((N + BS1 - 1) / BS1), (unsigned)((RS + 15) / 16)), BS, N, rows, RS, psi, pc, pfa);
+    const double mv = 3 * r_ * n_ * D + 2 * mixed * r_ * n_ * 4 + edge1 + l_ * n_ * D + tabs + 6 * n_ * I;
+#define TRANSPORT(C)                                                                                              \
+  ISW_LAUNCH_SHM("tr_move", mv + r_ * n_ * D + l_ * n_ * D, (k_tr_move<C, true>), gp, BS, 2 * lds, *g, Lm, RS, chunks, \
+                 1.0 / 3.0, tr->beta, pc, f0, wt, Fm, M0, M1, pc, tr->p1, pfb, tr->td);                              \
+  ISW_LAUNCH_SHM("tr_move", mv, (k_tr_move<C, false>), gp, BS, lds, *g, Lm, RS, chunks, 1.0 / 2.0, tr->beta, tr->p1,   \
+                 f1, wt, Fm, M0, M1, pc, tr->p2, pfa, nullptr);                                                     \
+  ISW_LAUNCH_SHM("tr_limit", 5 * r_ * n_ * D + mixed * r_ * n_ * 4 + edge1 + l_ * n_ * D + tabs + 6 * n_ * I +         \
+                                 r_ * e_ * D,                                                                     \
+                 k_tr_limit<C>, gp, BS, lds, *g, Lm, RS, chunks, tr->beta, pc, tr->p2, f2, wt, Fm, tr->td, M1,        \
+                 tr->A, tr->Rp, tr->Rm);                                                                          \
+  ISW_LAUNCH_SHM("tr_correct", 4 * r_ * n_ * D + r_ * e_ * D + l_ * n_ * D + 2 * e_ * I + tabs, k_tr_correct<C>, gp, BS, \
+                 lds, *g, Lm, rows, RS, chunks, tr->td, M1, tr->A, tr->Rp, tr->Rm, psi)
+    if (RC == 8) {
+      TRANSPORT(8);
+    } else {
+      TRANSPORT(4);
+    }
+#undef TRANSPORT
+    return (int)hipGetLastError();
+  }
   const double cellE = 6 * n_ * I + 2 * e_ * I;  // cellEdgeAsc, eI/eJ
   const double sten = 8 * e_ * (R + I) + l_ * e_ * D + 2 * e_ * I;
   ISW_LAUNCH("tr_td", 2 * l_ * n_ * D + r_ * n_ * D + l_ * e_ * D + cellE + r_ * n_ * D + mixed * r_ * n_ * 4,
@@ -2110,43 +2386,17 @@ int transport_step(const isw_grid* g, const isw_transport* tr, const double* M0,
   const fast* p1f = tr->p1;
   const fast* p2f = tr->p2;
 #endif
-  // (the flux of a patch's edges for four rows in LDS: at most 64 KiB)
-  const bool fused = g->pi_off && g->pcells == BS1 && (!ISW_FORM_MIXED || tr->pf2) &&
-                     (size_t)4 * g->ptedges * sizeof(double) <= 65536;
-  if (fused) {
-    // (algorithmic bytes: the stencil's field and its FP32 copy, the stencil and its weights, Fm, M0, psi, the
-    // output and its copy, the cell rings and the patch tables; the flux stays in LDS)
-    const double tabs = 6 * n_ * I + 2 * (n_ / BS1 + 1) * I + 2 * e_ * I + 6 * n_ * I;
-    const size_t shm = (size_t)4 * g->ptedges * sizeof(double);
-#if ISW_FORM_MIXED
-    float* pfb = tr->pf2;
-    const fast* p1s = tr->pf2;                     // (stage 1 writes p1's copy to pf2; stage 2 reads it, writes pf)
-#else
-    float* pfb = nullptr;
-    const fast* p1s = tr->p1;
-#endif
-    const dim3 gp((unsigned)g->npatch, (unsigned)((rows + 3) / 4));
-    ISW_LAUNCH_SHM("tr_hstage", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + l_ * n_ * D + r_ * n_ * D + tabs +
-                                    r_ * n_ * D + mixed * r_ * n_ * 4,
-                   k_tr_hstage, gp, dim3(BS1, 4), shm, *g, Lm, rows, 1.0 / 3.0, tr->beta, psi, psf, wt, Fm, M0, psi,
-                   tr->p1, pfb);
-    ISW_LAUNCH_SHM("tr_hstage", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + l_ * n_ * D + r_ * n_ * D + tabs +
-                                    r_ * n_ * D + mixed * r_ * n_ * 4,
-                   k_tr_hstage, gp, dim3(BS1, 4), shm, *g, Lm, rows, 1.0 / 2.0, tr->beta, tr->p1, p1s, wt, Fm, M0,
-                   psi, tr->p2, pf);
-  } else {
-    ISW_LAUNCH("tr_hflux", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + r_ * e_ * D,
-               k_tr_hflux, c4(E, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 3.0, tr->beta, psi, psf, wt, Fm, tr->Hf);
-    ISW_LAUNCH("tr_stage", l_ * n_ * D + r_ * n_ * D + r_ * e_ * D + l_ * e_ * D + cellE + r_ * n_ * D +
-                               mixed * r_ * n_ * 4,
-               k_tr_stage, c4(N, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 3.0, M0, psi, tr->Hf, Fm, tr->p1, pf);
-    ISW_LAUNCH("tr_hflux", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + r_ * e_ * D,
-               k_tr_hflux, c4(E, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 2.0, tr->beta, tr->p1, p1f, wt, Fm,
-               tr->Hf);
-    ISW_LAUNCH("tr_stage", l_ * n_ * D + r_ * n_ * D + r_ * e_ * D + l_ * e_ * D + cellE + r_ * n_ * D +
-                               mixed * r_ * n_ * 4,
-               k_tr_stage, c4(N, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 2.0, M0, psi, tr->Hf, Fm, tr->p2, pf);
-  }
+  ISW_LAUNCH("tr_hflux", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + r_ * e_ * D,
+             k_tr_hflux, c4(E, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 3.0, tr->beta, psi, psf, wt, Fm, tr->Hf);
+  ISW_LAUNCH("tr_stage", l_ * n_ * D + r_ * n_ * D + r_ * e_ * D + l_ * e_ * D + cellE + r_ * n_ * D +
+                             mixed * r_ * n_ * 4,
+             k_tr_stage, c4(N, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 3.0, M0, psi, tr->Hf, Fm, tr->p1, pf);
+  ISW_LAUNCH("tr_hflux", r_ * n_ * D + mixed * r_ * n_ * 4 + sten + r_ * e_ * D,
+             k_tr_hflux, c4(E, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 2.0, tr->beta, tr->p1, p1f, wt, Fm,
+             tr->Hf);
+  ISW_LAUNCH("tr_stage", l_ * n_ * D + r_ * n_ * D + r_ * e_ * D + l_ * e_ * D + cellE + r_ * n_ * D +
+                             mixed * r_ * n_ * 4,
+             k_tr_stage, c4(N, rows), dim3(BS1, 4), *g, Lm, rows, 1.0 / 2.0, M0, psi, tr->Hf, Fm, tr->p2, pf);
   ISW_LAUNCH("tr_aflux", 2 * r_ * n_ * D + mixed * r_ * n_ * 4 + sten + r_ * e_ * D,
              k_tr_aflux, dim3((unsigned)((E + BS - 1) / BS), (unsigned)((rows + 3) / 4)), dim3(BS1, 4), *g, Lm, rows,
              tr->beta, psi, tr->p2, p2f, wt, Fm, tr->A);

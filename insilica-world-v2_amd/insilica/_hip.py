@@ -65,7 +65,7 @@ class IswLayers(ctypes.Structure):
 
 
 class IswTransport(ctypes.Structure):
-    _fields_ = ([(k, ctypes.c_int32) for k in ('L', 'rows_max', 'prec', 'pad_')]
+    _fields_ = ([(k, ctypes.c_int32) for k in ('L', 'rows_max', 'prec', 'rows_pad')]
                 + [('beta', ctypes.c_double)]
                 + [(k, _f64p) for k in ('td', 'p1', 'p2', 'Rp', 'Rm', 'Hf', 'A')]
                 + [('pf', _f32p), ('pf2', _f32p)])

@@ -20,12 +20,13 @@ class Transport:
         N, E, R = dg.N, dg.E, tracers * layers
         z = dg.zeros
         self.psi = z(R, N)                           # the staging rows for tracers passed as separate arrays
-        self.td, self.p1, self.p2, self.Rp, self.Rm = (z(R, N) for _ in range(5))
-        self.Hf, self.A = z(R, E), z(R, E)
-        self.pf = z(R, N, dtype=torch.float32) if dg.mixed else None
-        self.pf2 = z(R, N, dtype=torch.float32) if dg.mixed else None
+        P = (R + 3) // 4 * 4                         # (the passes keep the rows cell-major, four to a load)
+        self.td, self.p1, self.p2, self.Rp, self.Rm = (z(P, N) for _ in range(5))
+        self.Hf, self.A = z(P, E), z(P, E)
+        self.pf = z(P, N, dtype=torch.float32) if dg.mixed else None
+        self.pf2 = z(P, N, dtype=torch.float32) if dg.mixed else None
         s = _hip.IswTransport()
-        s.L, s.rows_max, s.prec, s.beta = layers, R, dg.prec, beta
+        s.L, s.rows_max, s.rows_pad, s.prec, s.beta = layers, R, P, dg.prec, beta
         for k in ('td', 'p1', 'p2', 'Rp', 'Rm', 'Hf', 'A'):
             setattr(s, k, ctypes.cast(getattr(self, k).data_ptr(), _hip._f64p))
         s.pf = ctypes.cast(self.pf.data_ptr(), _hip._f32p) if self.pf is not None else None

@@ -1,0 +1,122 @@
+"""The passes that run on the 64-cell patches -- several fast sub-steps to a launch, the limiter with the thickness and wind
+update, the transport with its rows cell-major -- against the oracle where their shapes change: every remainder of the
+sub-steps over a launch's three (air) or four (ocean), one to eight layers (at which the rings are shallower, or absent, as
+LDS fills), row counts about the four to a load and the eight to a block, meshes whose last patch is part full (162, 642 and
+2,562 cells are 2.5, 10.03 and 40.03 patches), walls, and a floor that holds many cells' outflow back.
+
+Bars: the FP64 form, whose sums keep the oracle's order, to 1e-12 of the largest value after one step; the mixed form to
+1e-5, the figure it is held to over a day."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import relmax
+
+pytestmark = pytest.mark.gpu
+
+BARS = {'double': 1e-12, 'mixed': 1e-5}
+
+
+def _np(t):
+    return t.detach().cpu().numpy().copy()
+
+
+def _step(g, precision, kw, h, u, dt, nfast, theta=None):
+    """One step of the library and of the oracle: their largest differences by name."""
+    import oracle
+    from insilica.gpu import DeviceGrid
+    from insilica.layers import Layers
+    dg, og = DeviceGrid(g, precision), oracle.Grid(g)
+    lay, olay = Layers(dg, **kw), oracle.Layers(og, **kw)
+    hd, ud, Fd = dg.asarray(h), dg.asarray(u), dg.zeros(kw['layers'], g.E)
+    ho, uo, Fo = h.copy(), u.copy(), np.zeros((kw['layers'], g.E))
+    td = None if theta is None else dg.asarray(theta)
+    if theta is not None:
+        lay.update_gfast(hd, td)
+        olay.update_gfast(ho, theta)
+    lay.step(hd, ud, dt, nfast, Fd, theta=td)
+    olay.step(ho, uo, dt, nfast, Fo, theta=theta)
+    torch.cuda.synchronize()
+    return dict(h=relmax(_np(hd), ho), u=relmax(_np(ud), uo), Fm=relmax(_np(Fd), Fo))
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast', [(2, 3, 1), (3, 3, 2), (4, 3, 3), (4, 1, 4), (4, 2, 5), (4, 4, 7), (3, 5, 9),
+                                       (4, 6, 11), (4, 7, 8), (4, 8, 6)])
+def test_air(grids, n, L, nfast, precision):
+    from insilica import cases
+    from insilica.constants import CP_DRY, KAPPA, R_DRY
+    from insilica.ocean import visc4
+    print(f'case: air n={n} L={L} nfast={nfast} {precision}', flush=True)
+    g = grids(n)
+    st = cases.coupled_stack(g, seed=n + L, lmax=4)
+    at = np.linspace(0.0, 2.0, L) if L > 1 else np.array([1.0])
+    k, f = np.minimum(at.astype(int), 1), at - np.minimum(at.astype(int), 1)
+    theta, u = (np.ascontiguousarray((1 - f)[:, None] * st[x][k] + f[:, None] * st[x][k + 1]) for x in ('theta', 'u'))
+    h = np.repeat(st['h'].sum(0)[None] / L, L, 0)
+    kw = dict(layers=L, gprime=[0.0] * (L - 1), nu4=visc4(g, 15.0), floor=10.0,
+              air=dict(cp=CP_DRY, kappa=KAPPA, rd=R_DRY), thin_wind=100.0, stress=[0.0] * (L - 1) + [1e-2])
+    diff = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta)
+    assert max(diff.values()) <= BARS[precision], diff
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast,wall,floor', [(2, 2, 1, True, 1.0), (3, 1, 2, False, 1.0), (4, 2, 3, True, 1.0),
+                                                  (4, 2, 4, True, 0.995), (3, 3, 5, True, 0.995), (4, 2, 6, False, 0.995),
+                                                  (4, 5, 9, True, 0.999), (4, 8, 11, True, 0.995)])
+def test_ocean(grids, n, L, nfast, wall, floor, precision):
+    """floor below one: that share of the layers' mean thickness, which many cells start beneath."""
+    from insilica import cases
+    from insilica.ocean import visc4
+    print(f'case: ocean n={n} L={L} nfast={nfast} wall={wall} floor={floor} {precision}', flush=True)
+    g = grids(n)
+    h2, b, u2, gp = cases.phillips(g, 3.0)
+    rng = np.random.default_rng(n + L)
+    h = np.repeat(h2.sum(0)[None] / L, L, 0)
+    h = np.ascontiguousarray(h * (1 + rng.uniform(-0.01, 0.01, h.shape)))
+    u = np.ascontiguousarray(u2[np.arange(L) % 2] + rng.normal(0, 2.0, (L, g.E)))
+    kw = dict(layers=L, b=b, gprime=[gp / max(1, L - 1)] * (L - 1), stress=[0.0] * (L - 1) + [2.5e-4], nu4=visc4(g, 5.0),
+              floor=float(floor * h.mean()) if floor < 1 else floor, vmix=5e-4)
+    if wall:
+        land = rng.random(g.N) < 0.1
+        kw['wall'] = np.where(land[g.eI] | land[g.eJ], 0.0, 1.0)
+        u *= kw['wall'][None]
+    diff = _step(g, precision, kw, h, u, 100.0 * nfast, nfast)
+    assert max(diff.values()) <= BARS[precision], diff
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,K', [(4, 1, 1), (3, 3, 1), (4, 2, 2), (2, 5, 1), (4, 7, 1), (4, 2, 4), (3, 3, 3), (4, 4, 3),
+                                   (4, 3, 5), (4, 8, 2), (4, 1, 17)])
+def test_transport_rows(grids, n, L, K, precision):
+    """K tracers of L layers by unequal mass fluxes, steep rows among them, and the same rows where the scratch is not
+    padded (one row to a load): both against the oracle, the FP64 form's the same to the bit."""
+    import oracle
+    from insilica.gpu import DeviceGrid
+    from insilica.transport import Transport
+    print(f'case: transport n={n} L={L} K={K} {precision}', flush=True)
+    g = grids(n)
+    dg, og = DeviceGrid(g, precision), oracle.Grid(g)
+    rng = np.random.default_rng(10 * L + K)
+    area = g.areaCell
+    M = np.stack([(1 + 0.1 * l) * area for l in range(L)])
+    Fm = 0.03 * area.mean() * rng.normal(size=(L, g.E))
+    M1 = np.zeros_like(M)
+    oracle.mass_update(og, L, M, Fm, M1)
+    assert M1.min() > 0
+    rows = rng.random((L * K, g.N))
+    rows[::3] = (rows[::3] > 0.7).astype(float)
+    ro = rows.copy()
+    oracle.transport(og, L, M, M1, Fm, ro, order=3)
+    out = []
+    for padded in (True, False):
+        tr = Transport(dg, layers=L, tracers=K)
+        if not padded:
+            tr.s.rows_pad = 0
+        rd = dg.asarray(rows)
+        tr.step_rows(dg.asarray(M), dg.asarray(M1), dg.asarray(Fm), rd, 3)
+        torch.cuda.synchronize()
+        out.append(_np(rd))
+        assert relmax(out[-1], ro) <= BARS[precision], f'padded {padded}'
+    if precision == 'double':
+        assert np.array_equal(out[0], out[1])
