@@ -363,22 +363,29 @@ __global__ __launch_bounds__(BS) void k_edge_hq(isw_grid g, int L, double shelf,
 
 // Per stage, pass 3 (lay_slow, layers.cu:269-359): the slow momentum tendency of every layer of an edge (W-weight PV
 // flux with the thin-layer cap, -grad B, drag, exact-exponential stress, pibar grad theta for air, del^4), its
-// thickness-weighted column mean G, T' = T - G, H_e and the column wind. The ~10 eoe neighbours' indices and
-// weights are loaded before the sum so that their packed records are gathered together.
+// thickness-weighted column mean G, T' = T - G, H_e and the column wind. Bound by the latency of the chain edge -> ~10
+// neighbours -> their packed records: the indices and weights load first, then all of a layer's records whether or not
+// the edge has that many neighbours (a missing one repeats the first and is left out of the sum), so that no branch
+// stands between the loads (three layers at level 6, mixed: 16.0 -> 12.8 us; two at level 7 33.9 -> 27.1).
 // One thread per edge with the layers in registers (L a compile-time count): the edge's neighbour list and weights
-// load once for every layer, each neighbour's L packed records are one contiguous run, and the column's blend and
-// mean need no LDS; the column sums run in the reference's layer order.
-template <int L>
-__global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double dts, const fast* __restrict__ pk,
-                                               const fast* __restrict__ wf, const double* __restrict__ hedge,
-                                               const double* __restrict__ u, const double* __restrict__ B,
-                                               const double* __restrict__ lap4, const double* __restrict__ th,
-                                               const double* __restrict__ pibar, double* __restrict__ Tp,
-                                               double* __restrict__ G, double* __restrict__ He,
-                                               double* __restrict__ ubs) {
-  const int e = XTID;
-  if (e >= g.E) return;
+// load once for every layer and each neighbour's L packed records are one contiguous run. ROWS: a (64, L) block with a
+// thread per layer, for meshes too small to fill the card otherwise; the column's blend and mean then go through LDS.
+// The column sums run in the reference's layer order in both.
+template <int L, bool ROWS>
+__global__ __launch_bounds__(ROWS ? 64 * L : BS) void k_slow_e(isw_grid g, LP p, Div dv, double dts,
+                                                               const fast* __restrict__ pk, const fast* __restrict__ wf,
+                                                               const double* __restrict__ hedge,
+                                                               const double* __restrict__ u, const double* __restrict__ B,
+                                                               const double* __restrict__ lap4,
+                                                               const double* __restrict__ th,
+                                                               const double* __restrict__ pibar, double* __restrict__ Tp,
+                                                               double* __restrict__ G, double* __restrict__ He,
+                                                               double* __restrict__ ubs) {
   const int N = g.N, E = g.E;
+  const int at = ROWS ? xblock() * 64 + (int)threadIdx.x : XTID;
+  const bool live = at < E;
+  if (!ROWS && !live) return;
+  const int e = live ? at : 0;
   const int eI = g.eI[e], eJ = g.eJ[e];
   const int m0 = g.eoeStart[e], m1 = g.eoeStart[e + 1];
   constexpr int NB = 10;
@@ -392,22 +399,23 @@ __global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double 
   }
   const double rde = dv.de[e];
   const double nu4 = lap4 ? nu4_at(p, e) : 0.0;
-  double dk[L], hk[L], uk[L], sqk[L];
-#pragma unroll
-  for (int k = 0; k < L; k++) {
+  auto layer = [&](int k, double& dk, double& hk, double& uk, double& sqk) {
     const size_t o = (size_t)k * E + e;
     const double he = hedge[o];
     const double ue = u[o];
     const fast cap = (fast)(p.thin * he), qf = pk[((size_t)e * L + k) * 3 + 2];
+    fast hn[NB], un[NB], qn[NB];
+#pragma unroll
+    for (int m = 0; m < NB; m++) {
+      const fast* pp = pk + ((size_t)nb[m] * L + k) * 3;
+      hn[m] = pp[0]; un[m] = pp[1]; qn[m] = pp[2];
+    }
     fast Q = 0;
 #pragma unroll
     for (int m = 0; m < NB; m++) {
-      if (m0 + m >= m1) break;
-      const fast* pp = pk + ((size_t)nb[m] * L + k) * 3;
-      fast h2 = pp[0];
-      if (h2 > cap) h2 = cap;
-      const fast F2 = h2 * pp[1];
-      Q += w[m] * F2 * (fast)0.5 * (qf + pp[2]);
+      const fast F2 = (hn[m] > cap ? cap : hn[m]) * un[m];
+      const fast Qm = Q + w[m] * F2 * (fast)0.5 * (qf + qn[m]);
+      Q = m0 + m < m1 ? Qm : Q;
     }
     for (int m = m0 + NB; m < m1; m++) {           // (meshes with more neighbours per edge than 10)
       const fast* pp = pk + ((size_t)g.eoe[m] * L + k) * 3;
@@ -429,10 +437,7 @@ __global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double 
       if (p.cd_bot > 0) {
         fast vt = 0;
 #pragma unroll
-        for (int m = 0; m < NB; m++) {
-          if (m0 + m >= m1) break;
-          vt += w[m] * pk[((size_t)nb[m] * L + k) * 3 + 1];
-        }
+        for (int m = 0; m < NB; m++) vt = m0 + m < m1 ? vt + w[m] * un[m] : vt;
         for (int m = m0 + NB; m < m1; m++) vt += wf[m] * pk[((size_t)g.eoe[m] * L + k) * 3 + 1];
         ck += p.cd_bot * sqrt(ue * ue + (double)vt * (double)vt);
       }
@@ -448,10 +453,25 @@ __global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double 
       d = d + DIVBY(0.5 * (pl[eI] + pl[eJ]) * (tl[eJ] - tl[eI]), rde);
     }
     if (lap4) d = d - nu4 * lap4[o];
-    dk[k] = d;
-    hk[k] = he;
-    uk[k] = ue;
-    sqk[k] = sq0;
+    dk = d;
+    hk = he;
+    uk = ue;
+    sqk = sq0;
+  };
+  double dk[L], hk[L], uk[L], sqk[L];
+  if (ROWS) {
+    __shared__ double sc[4][L][64];
+    const int j = (int)threadIdx.x, y = (int)threadIdx.y;
+    double a, b, c, d;
+    layer(y, a, b, c, d);
+    sc[0][y][j] = a; sc[1][y][j] = b; sc[2][y][j] = c; sc[3][y][j] = d;
+    __syncthreads();
+    if (!live) return;
+#pragma unroll
+    for (int m = 0; m < L; m++) { dk[m] = sc[0][m][j]; hk[m] = sc[1][m][j]; uk[m] = sc[2][m][j]; sqk[m] = sc[3][m][j]; }
+  } else {
+#pragma unroll
+    for (int k = 0; k < L; k++) layer(k, dk[k], hk[k], uk[k], sqk[k]);
   }
   // the blend of a thin layer's tendency with its nearest thick neighbours' (shelf), then the column mean
   const bool blend = th && p.shelf > 0;
@@ -459,8 +479,13 @@ __global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double 
     double Tm = dk[m];
     if (blend && sqk[m] < 1) {
       double wgt = 0, s = 0;
-      for (int q2 = m - 1; q2 >= 0; q2--) if (sqk[q2] >= 1) { wgt += hk[q2]; s += hk[q2] * dk[q2]; break; }
-      for (int q2 = m + 1; q2 < L; q2++) if (sqk[q2] >= 1) { wgt += hk[q2]; s += hk[q2] * dk[q2]; break; }
+      bool up = true, down = true;
+#pragma unroll
+      for (int q = L - 1; q >= 0; q--)
+        if (q < m && up && sqk[q] >= 1) { wgt += hk[q]; s += hk[q] * dk[q]; up = false; }
+#pragma unroll
+      for (int q = 0; q < L; q++)
+        if (q > m && down && sqk[q] >= 1) { wgt += hk[q]; s += hk[q] * dk[q]; down = false; }
       if (wgt > 0) Tm = sqk[m] * dk[m] + (1 - sqk[m]) * s / wgt;
     }
     return Tm;
@@ -479,7 +504,8 @@ __global__ __launch_bounds__(BS) void k_slow_e(isw_grid g, LP p, Div dv, double 
   }
   const double gg = GT / H;
 #pragma unroll
-  for (int k = 0; k < L; k++) Tp[(size_t)k * E + e] = Tb[k] - gg;
+  for (int k = 0; k < L; k++) if (!ROWS || k == (int)threadIdx.y) Tp[(size_t)k * E + e] = Tb[k] - gg;
+  if (ROWS && threadIdx.y) return;
   G[e] = gg;
   He[e] = H;
   ubs[e] = U / H;
@@ -2081,10 +2107,19 @@ static void stage(const isw_grid* g, const isw_layers* s, const LP& p, const Div
   const double slow_bytes = 3 * l_ * e_ * R + neoe * (R + I) + (e_ + 1) * I + 2 * l_ * e_ * D + l_ * n_ * D +
                             2 * e_ * I + e_ * D + (s->nu4 != 0 ? l_ * e_ * D : 0) + air * 2 * l_ * n_ * D + l_ * e_ * D +
                             3 * e_ * D;
-#define SLOW(LL)                                                                                                   \
-  ISW_LAUNCH("slow", slow_bytes, k_slow_e<LL>, g1(E), BS, *g, p, dv, c * dt, pk, wf, s->hedge, us, s->B,             \
+  // A thread per layer while the edges alone give a SIMD at most one wave (256 CUs of four): three layers at level 5
+  // 10.4 -> 7.9 us, seven of FP64 at level 4 21.7 -> 8.4, at level 5 23.3 -> 14.6; beyond, a thread per edge: three
+  // layers at level 6 12.8 us against 15.9, seven of FP64 37.9 against 43.7
+#define SLOW_AS(LL, RW, GRID, BLOCK)                                                                               \
+  ISW_LAUNCH("slow", slow_bytes, (k_slow_e<LL, RW>), GRID, BLOCK, *g, p, dv, c * dt, pk, wf, s->hedge, us, s->B,     \
              s->nu4 != 0 ? s->L2 : nullptr, s->air ? theta : nullptr, s->air ? s->pibar : nullptr, s->Tp, s->G, s->He, \
              s->ubs)
+#define SLOW(LL)                                                                                                   \
+  if (LL > 1 && E <= 64 * 1024) {                                                                                    \
+    SLOW_AS(LL, true, dim3((unsigned)((E + 63) / 64)), dim3(64, LL));                                               \
+  } else {                                                                                                          \
+    SLOW_AS(LL, false, g1(E), BS);                                                                                  \
+  }
   switch (L) {
     case 1: SLOW(1); break;
     case 2: SLOW(2); break;
