@@ -64,9 +64,16 @@ __device__ __forceinline__ void layer_exner(const double* mu, const CP& P, doubl
   }
 }
 
-// theta* of interface j: the lowest is theta_star, the ones above from the list (from the top).
+// theta* of interface j: the lowest is theta_star, the ones above from the list (from the top; chosen by selects, as an
+// index known only at run time would put all of P in memory).
 template <int L>
-__device__ __forceinline__ double tstar(int j, const CP& P) { return j == L - 2 ? P.theta_star : P.ths[j]; }
+__device__ __forceinline__ double tstar(int j, const CP& P) {
+  double t = P.theta_star;
+#pragma unroll
+  for (int m = 0; m < ISW_LMAX; m++)
+    if (m != L - 2) t = j == m ? P.ths[m] : t;
+  return t;
+}
 
 // The shape s of a layer's truncated-exponential theta density between edges a < b with mean m (air.cu:245-270):
 // r(s) = 1 - 1/s + 1/(e^s - 1) = (m - a) / (b - a) by Newton's method kept inside a bracket.
@@ -140,6 +147,15 @@ struct AP {
   double cu_dth, cu_dp, cu_sub, cl_float, sub_mix;     // (the cumulus layer's)
 };
 
+// The kernel's copy of it, read where the launch put it (uniform, so through the scalar cache). As an ordinary by-value
+// argument whose address the column's functions take it was copied to every lane's private memory, 1.1 KB a column, and
+// read back from there: 7 cloudy layers at level 6 (mixed) 271 -> 254 us without that, 3 moist ones at level 5 (FP64)
+// 40.7 -> 33.2. The column is bound by its chain of dependent arithmetic and by what of its layers' arrays spills (one wave
+// per SIMD); so the functions that take those arrays by pointer and are called for every column (the crossing, the moves of
+// mass, the edges' vapor, the mixed layer's cloud) are inlined, for calls keep every array in private memory throughout:
+// 254 -> 210 us.
+using APk = const __attribute__((address_space(4))) AP;
+
 static AP make_ap(const double* a, const isw_air* air) {
   AP p;
   p.S0 = a[0]; p.asw = a[1]; p.tau0 = a[2]; p.mu_ref = a[3]; p.eps_s = a[4]; p.h_sens = a[5]; p.u0 = a[6];
@@ -181,13 +197,13 @@ __device__ __forceinline__ double fpow_(double x, double y) {
 }
 
 // The gray optical depth down to pressure p of a column with surface pressure ps (air.cu:853-856).
-__device__ __forceinline__ double tau_p(double p, double ps, const AP& A) {
+__device__ __forceinline__ double tau_p(double p, double ps, APk& A) {
   const double s = p / ps, s2 = s * s;
   return A.tau0 * (A.tau_lin * s + (1 - A.tau_lin) * s2 * s2);
 }
 
 // The sun's ecliptic longitude at t and its distance factor (air.cu:174-185): Kepler's equation, five Newton steps.
-__device__ double sun_lon_fd(double t, const AP& A, double* fd) {
+__device__ double sun_lon_fd(double t, APk& A, double* fd) {
   constexpr double PI_ = 3.14159265358979323846;
   if (!(A.ecc > 0)) {
     *fd = 1;
@@ -216,7 +232,7 @@ __device__ __forceinline__ F qsat_a(F T, F p, F eps, double ice) {
 
 // Saturation adjustment at Exner pib and pressure p in one Newton step (air.cu:190-198); returns the condensate.
 template <bool MIX>
-__device__ double condense(double& th, double& q, double pib, double p, const CP& P, const AP& A) {
+__device__ double condense(double& th, double& q, double pib, double p, const CP& P, APk& A) {
   using F = std::conditional_t<MIX, float, double>;
   const F T = (F)pib * (F)th / (F)P.cp, qs = qsat_a<F>(T, (F)p, (F)A.eps, A.ice_air);
   if (!(q > qs)) return 0;
@@ -246,7 +262,7 @@ __device__ __forceinline__ double spread_of(double m, double s, double es) {
 // uniform, or (spread) spread between its edges ea < eb by the truncated exponential of its mean (the mass share m
 // from its base at ea + (eb - ea) spread_of(m)). In the build's `fast` type, returned as such.
 template <bool MIX>
-__device__ __forceinline__ void layer_cap(double th, double pt, double pb, const CP& P, const AP& A,
+__device__ __forceinline__ void layer_cap(double th, double pt, double pb, const CP& P, APk& A,
                                           std::conditional_t<MIX, float, double>& qs,
                                           std::conditional_t<MIX, float, double>& dqs, bool spread = false,
                                           double ea = 0, double eb = 0) {
@@ -271,7 +287,7 @@ __device__ __forceinline__ void layer_cap(double th, double pt, double pb, const
 // Whether layer k's capacity has its theta spread between its edges (sat_prof: a middle layer below edge_k's
 // tropopause, colder than its top edge), and those edges.
 template <int L>
-__device__ __forceinline__ bool spread_layer(int k, double th, const CP& P, const AP& A, double& ea, double& eb) {
+__device__ __forceinline__ bool spread_layer(int k, double th, const CP& P, APk& A, double& ea, double& eb) {
   const bool sp = A.sat_prof > 0 && k >= (int)A.edge_k && k < L - 1 && th < tstar<L>(k - 1, P);
   ea = sp ? tstar<L>(k, P) : 0.0;
   eb = sp ? tstar<L>(k - 1, P) : 0.0;
@@ -280,7 +296,7 @@ __device__ __forceinline__ bool spread_layer(int k, double th, const CP& P, cons
 
 // Layer k's capacity (the spread one with sat_prof) over [pt, pb].
 template <int L, bool MIX>
-__device__ __forceinline__ void layer_cap_k(int k, double th, double pt, double pb, const CP& P, const AP& A,
+__device__ __forceinline__ void layer_cap_k(int k, double th, double pt, double pb, const CP& P, APk& A,
                                             std::conditional_t<MIX, float, double>& qs,
                                             std::conditional_t<MIX, float, double>& dqs) {
   double ea, eb;
@@ -291,7 +307,7 @@ __device__ __forceinline__ void layer_cap_k(int k, double th, double pt, double 
 // Saturation adjustment against the layer's capacity over [pt, pb] (air.cu:275-291; spread: condense_spread,
 // air.cu:292-315, the whole spread shifting with the mean): one Newton step.
 template <bool MIX>
-__device__ double condense_layer(double& th, double& q, double pib, double pt, double pb, const CP& P, const AP& A,
+__device__ double condense_layer(double& th, double& q, double pib, double pt, double pb, const CP& P, APk& A,
                                  bool spread = false, double ea = 0, double eb = 0) {
   using F = std::conditional_t<MIX, float, double>;
   F qs, dqs;
@@ -308,7 +324,7 @@ __device__ double condense_layer(double& th, double& q, double pib, double pt, d
 // at the pressure whose Exner function is the layer's. tk, qk: layer k's theta and vapor, updated.
 template <int L, bool MIX>
 __device__ double condense_at(int k, double& tk, double& qk, double pk, double pt, double mk, const CP& P,
-                              const AP& A) {
+                              APk& A) {
   if (A.sat_layer > 0) {
     double ea, eb;
     if (spread_layer<L>(k, tk, P, A, ea, eb))
@@ -325,7 +341,7 @@ __device__ double condense_at(int k, double& tk, double& qk, double pk, double p
 // condense_at for a runtime layer index: the layer's values go through selects.
 template <int L, bool MIX>
 __device__ double condense_k(int k, const double* mu, double* th, double* q, const double* pib, const CP& P,
-                             const AP& A) {
+                             APk& A) {
   double pt = 0, mk = 0, tk = 0, qk = 0, pk = 0;
 #pragma unroll
   for (int j = 0; j < L; j++) {
@@ -342,7 +358,7 @@ __device__ double condense_k(int k, const double* mu, double* th, double* q, con
 // The temperature at layer k's lower edge (pressure pb) (air.cu:476-482): its theta there, or for a spread middle
 // layer (sat_prof) its lower theta*.
 template <int L, bool MIX>
-__device__ __forceinline__ double base_T(int k, double th, double pb, const CP& P, const AP& A) {
+__device__ __forceinline__ double base_T(int k, double th, double pb, const CP& P, APk& A) {
   double ea, eb;
   return (spread_layer<L>(k, th, P, A, ea, eb) ? ea : th) * fpow_<MIX>(pb / P.p0, P.kappa);
 }
@@ -352,8 +368,8 @@ __device__ __forceinline__ double base_T(int k, double th, double pb, const CP& 
 // L >= 3) and, with bl_q, the mixed bottom layer keep their vapor even. Air of mass m leaving through that edge takes
 // the edge's vapor plus m's share of the way to the mean, at most the layer's whole vapor. k may be a runtime index.
 template <int L, bool MIX>
-__device__ double edge_q(int k, bool top, const double* mu, const double* th, const double* q, double m, const CP& P,
-                         const AP& A) {
+__device__ __forceinline__ double edge_q(int k, bool top, const double* mu, const double* th, const double* q,
+                                         double m, const CP& P, APk& A) {
   using F = std::conditional_t<MIX, float, double>;
   double mk = 0, tk = 0, qk = 0, pt = 0;
 #pragma unroll
@@ -378,7 +394,7 @@ __device__ double edge_q(int k, bool top, const double* mu, const double* th, co
 
 // A parcel (th, q) lifted to pressure p, condensing what it cannot hold (air.cu:468-473).
 template <bool MIX>
-__device__ __forceinline__ void parcel(double th, double q, double p, const CP& P, const AP& A, double& thp,
+__device__ __forceinline__ void parcel(double th, double q, double p, const CP& P, APk& A, double& thp,
                                        double& qp) {
   thp = th;
   qp = q;
@@ -403,7 +419,8 @@ __device__ __forceinline__ double column_energy(const double* mu, const double* 
 // (and vapor: it leaves with q_leave per kg and arrives with q_arrive) re-divided, the column's energy residual booked
 // into the receiver. CL: the air takes its cloud water cl along (the receiver's share re-divided).
 template <int L, bool MOIST = false, bool CL = false>
-__device__ void move_mass(const CP& P, double* mu, double* th, double* q, double* pib, int from, int to, double m,
+__device__ __forceinline__ void move_mass(const CP& P, double* mu, double* th, double* q, double* pib, int from,
+                                          int to, double m,
                           double th_leave, double th_arrive, double q_leave = 0, double q_arrive = 0,
                           double* cl = nullptr) {
   if (m == 0) return;
@@ -483,8 +500,8 @@ __device__ void move_mass(const CP& P, double* mu, double* th, double* q, double
 // the top layer's bottom-edge default its dth_up): always given, so every array stays in registers. CL: the crossing
 // air takes its cloud water cl along.
 template <int L, bool MOIST = false, bool CL = false, bool MIX = false>
-__device__ void crossing(const CP& P, double* mu, double* th, double* q, const double* dth, const double* et,
-                         const double* eb, double* pib, double* wxo, double* cl = nullptr, const AP* A = nullptr,
+__device__ __forceinline__ void crossing(const CP& P, double* mu, double* th, double* q, const double* dth,
+                         const double* et, const double* eb, double* pib, double* wxo, double* cl = nullptr, APk* A = nullptr,
                          double* gross = nullptr, size_t gstride = 0) {
 #pragma unroll
   for (int j = 0; j + 1 < L; j++) wxo[j] = 0;
@@ -811,7 +828,7 @@ __global__ void k_advance_time(double* t, double dt) { t[0] += dt; }
 
 // The cloud statistics (air.cu:383-388): total water qt spread evenly over +-(1 - rh_crit) qs about its mean; the
 // saturated share f and the mean condensate l there.
-__device__ __forceinline__ void cloud_pdf(double qt, double qs, const AP& A, double& l, double& f) {
+__device__ __forceinline__ void cloud_pdf(double qt, double qs, APk& A, double& l, double& f) {
   const double b = (1 - A.rh_crit) * qs, s = qt - qs;
   if (s <= -b) {
     l = 0;
@@ -826,7 +843,7 @@ __device__ __forceinline__ void cloud_pdf(double qt, double qs, const AP& A, dou
 }
 
 // The cover of cloud water cw spread at a cloud's typical water content by phase (air.cu:393-396).
-__device__ __forceinline__ double cover_of(double cw, double mu, double liq, const AP& A, double qs) {
+__device__ __forceinline__ double cover_of(double cw, double mu, double liq, APk& A, double qs) {
   const double s = A.cw_qs > 0 && qs > 0 ? fmin(1.0, A.cw_qs * qs / A.q_auto) : 1.0;
   return fmin(1.0, cw / (s * (liq * A.q_auto + (1 - liq) * A.l_ice)) * fmax(1.0, mu / A.mu_cloud));
 }
@@ -836,7 +853,7 @@ __device__ __forceinline__ double cover_of(double cw, double mu, double liq, con
 // dqf the condensate's fall per kelvin of warming; ml_clear (unless pdf): only air actually saturated condenses.
 // False for any other layer (or without bl_q).
 template <int L, bool MIX>
-__device__ bool mixed_cloud(int k, const double* mu, double th, double qt, const CP& P, const AP& A, double& l,
+__device__ __forceinline__ bool mixed_cloud(int k, const double* mu, double th, double qt, const CP& P, APk& A, double& l,
                             double& f, double& dqf, bool pdf) {
   using F = std::conditional_t<MIX, float, double>;
   if (!(A.bl_q > 0 && k == L - 1 && k > 0)) return false;
@@ -873,7 +890,7 @@ __device__ bool mixed_cloud(int k, const double* mu, double th, double qt, const
 // feedback on the capacity, or eroding over tau_erode (air.cu:438-450); returns the condensate.
 template <int L, bool MIX>
 __device__ double cloud_adjust_k(int k, const double* mu, double* th, double* q, double* cl, const double* pib,
-                                 double dt, const CP& P, const AP& A) {
+                                 double dt, const CP& P, APk& A) {
   using F = std::conditional_t<MIX, float, double>;
   double pt = 0, mk = 0, tk = 0, qk = 0, ck = 0, pk = 0;
 #pragma unroll
@@ -929,7 +946,7 @@ __device__ __forceinline__ double liq_of(double T) {
 // stop flag, so every per-layer value stays in registers.
 template <int L, bool MIX>
 __device__ void plume_ascent(const double* mu, const double* th, const double* q, double th0, double q0, double pi_,
-                             const CP& P, const AP& A, double& Ab, int& kd, double& thd, double& qd, double* qx,
+                             const CP& P, APk& A, double& Ab, int& kd, double& thd, double& qd, double* qx,
                              double* lt, double& G, double& FZ, double* Gl, bool shal = false) {
   constexpr int bot = L - 1, M = bot > 2 ? 3 : 8;
   const bool cu = A.cu_dth > 0;
@@ -1067,7 +1084,7 @@ __device__ void plume_ascent(const double* mu, const double* th, const double* q
 // updraft area storm_area rising at half sqrt(2 CAPE); only an updraft faster than graupel falls holds it up to
 // charge. Flashes per second per m^2.
 template <bool MIX>
-__device__ double storm_flashes(double mflux, const double* lt, const CP& P, const AP& A) {
+__device__ double storm_flashes(double mflux, const double* lt, const CP& P, APk& A) {
   const double qi = lt[0], w = 0.5 * sqrt(2 * fmax(0.0, lt[3])), gv = A.graupel_v;
   if (!(mflux > 0) || !(qi > 0) || !(w > gv)) return 0;
   const double rho = lt[1] / (A.rd * A.Tf), phi = rho * w * A.storm_area, lift = 1 - gv * gv / (w * w);
@@ -1081,7 +1098,7 @@ __device__ double storm_flashes(double mflux, const double* lt, const CP& P, con
 
 // Air (th, q) at pressure p evaporating water until saturated (air.cu:453-466): three Newton steps, Tetens' slope.
 template <bool MIX>
-__device__ void wet_bulb(double& th, double& q, double p, const CP& P, const AP& A) {
+__device__ void wet_bulb(double& th, double& q, double p, const CP& P, APk& A) {
   using F = std::conditional_t<MIX, float, double>;
   const double ex = fpow_<MIX>(p / P.p0, P.kappa);
   for (int it = 0; it < 3; it++) {
@@ -1100,7 +1117,7 @@ __device__ void wet_bulb(double& th, double& q, double p, const CP& P, const AP&
 // saturates (air.cu:1413-1421): 40 bisections in pressure; 0 if saturated at the ground, 1e30 if not even at a tenth of
 // the surface pressure.
 template <int L, bool MIX>
-__device__ double lcl_mass(const double* mu, double th, double q, const CP& P, const AP& A) {
+__device__ double lcl_mass(const double* mu, double th, double q, const CP& P, APk& A) {
   using F = std::conditional_t<MIX, float, double>;
   double ps_ = 0;
 #pragma unroll
@@ -1122,7 +1139,7 @@ __device__ double lcl_mass(const double* mu, double th, double q, const CP& P, c
 // cu_top (air.cu:668-680): the theta the bottom layer's air reaches lifted from its top by cu_dp (Pa), condensing on
 // the way, in eight equal steps (no higher than 1000 Pa).
 template <int L, bool MIX>
-__device__ double cu_top(const double* mu, const double* th, const double* q, const CP& P, const AP& A) {
+__device__ double cu_top(const double* mu, const double* th, const double* q, const CP& P, APk& A) {
   constexpr int bot = L - 1;
   double pb = 0;
 #pragma unroll
@@ -1140,7 +1157,7 @@ __device__ double cu_top(const double* mu, const double* th, const double* q, co
 // with cl_float the cloud layer's lower edge (interface L - 4) cl_float above cu_top where that is above its fixed
 // value ths_cl, below that layer's mean less 1 K and the edge above less 0.5 K.
 template <int L, bool MIX>
-__device__ void cu_edges(const double* mu, const double* th, const double* q, CP& P, const AP& A, double ths_cl) {
+__device__ void cu_edges(const double* mu, const double* th, const double* q, CP& P, APk& A, double ths_cl) {
   if constexpr (L > 4) {
     if (A.cl_float > 0 && A.cu_dth > 0 && A.cu_dp > 0)
       P.ths[L - 4] = fmax(ths_cl, fmin(cu_top<L, MIX>(mu, th, q, P, A) + A.cl_float,
@@ -1233,22 +1250,18 @@ struct AirIO {
 };
 
 template <int L, bool MIX, bool MOIST, bool CLOUD, bool FULL>
-__global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, const double* __restrict__ t,
+__global__ void __launch_bounds__(BS) k_air_column(AP, int N, CP P, int mode, const double* __restrict__ t,
                                                    const double* __restrict__ insol, const double* __restrict__ pos,
                                                    const double* __restrict__ uabs, const double* __restrict__ mu_in,
                                                    double dt,
                                                    const double* __restrict__ elev, const double* __restrict__ radf,
                                                    const double* __restrict__ swf, const double* __restrict__ ch,
                                                    AirIO o) {
+  APk& A = *(APk*)__builtin_amdgcn_kernarg_segment_ptr();      // (the first argument)
   const int i = XTID;
   if (i >= N) return;
-  if constexpr (!FULL) {
-    // (the plain column, launched only when all of these are off: their branches compile away, and the kernel keeps
-    // the registers they would take)
-    P.bl_mix = 0;
-    A.sat_prof = A.sat_base = A.edge_vap = A.freeze_dry = A.q_shape = A.plume_root = A.plume_deep = A.bl_q = 0;
-    A.cu_dth = A.cu_sub = 0;
-  }
+  if constexpr (!FULL) P.bl_mix = 0;   // (the plain column, launched only when all its options are off: their branches
+                                       // compile away, and the kernel keeps the registers they would take)
   if (elev && A.theta_rise > 0 && elev[i] > 0) P.theta_star += A.theta_rise * elev[i];
   const double ts_base = P.theta_star;
   P.bl_cap = omexp<MIX>(dt / 86400.0);                 // (the mixed layer takes in at most a day's share per step)
@@ -1326,7 +1339,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
     // cu_cloud (with ml_clear and bl_q): the mixed layer clear below its cloud base, the cloud its thermals make is
     // above it, in the layer above: the thermals' statistics at the mixed layer's levels give its cover there and its
     // water (cu_cloud 2: the cover alone), for the radiation
-    if (A.cu_cloud > 0 && A.ml_clear > 0 && A.bl_q > 0 && L > 2) {
+    if (A.cu_cloud > 0 && A.ml_clear > 0 && FULL && A.bl_q > 0 && L > 2) {
       double l_, f_, d_;
       if (mixed_cloud<L, MIX>(bot, mu, th[bot], q[bot] + cl[bot], P, A, l_, f_, d_, true) && f_ > 1e-6) {
         constexpr int kc = bot - 1;
@@ -1503,7 +1516,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
   // q_shape: the air at the surface holds the bottom layer's vapor at its relative humidity there (against the
   // layer's capacity), not the layer's mean; bl_q keeps the layer's vapor even
   double qa = qb;
-  if (MOIST && A.q_shape > 0 && !(A.bl_q > 0)) {
+  if (MOIST && FULL && A.q_shape > 0 && !(FULL && A.bl_q > 0)) {
     F qsl, dqsl;
     layer_cap_k<L, MIX>(bot, th[bot], pb[bot - 1], pb[bot], P, A, qsl, dqsl);
     const double qss = (double)qsat_a<F>((F)Tsa, (F)ps, (F)A.eps, 0.0);
@@ -1907,7 +1920,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
                                 fmax(0.0, mu_lcl - mu[bot]));
           if (m > 0) {
             const double fm = m / mu[k], thl = spread ? e + fm * D : th[k];
-            const double qx = A.edge_vap > 0 ? edge_q<L, MIX>(k, false, mu, th, q, m, P, A) : q[k];
+            const double qx = FULL && A.edge_vap > 0 ? edge_q<L, MIX>(k, false, mu, th, q, m, P, A) : q[k];
             move_mass<L, MOIST, CLOUD>(P, mu, th, q, pib, k, bot, m, thl, thl, qx, qx, cl);
 #pragma unroll
             for (int j = k; j < bot; j++) wxo[j] -= m;
@@ -1938,7 +1951,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
         const bool spread = ka >= 1 && thka < tska && thka > eka;
         const double fm = fmin(1.0, m / mka);
         const double thc = spread ? eka + fm * (thka - eka) : thka;
-        const double qx = MOIST && A.edge_vap > 0 ? edge_q<L, MIX>(ka, false, mu, th, q, m, P, A) : qka;
+        const double qx = MOIST && FULL && A.edge_vap > 0 ? edge_q<L, MIX>(ka, false, mu, th, q, m, P, A) : qka;
         move_mass<L, MOIST, CLOUD>(P, mu, th, q, pib, ka, bot, m, thc, thc, qx, qx, cl);
 #pragma unroll
         for (int j = 0; j < bot; j++)
@@ -1947,14 +1960,14 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
     }
     if (!(Bf > 0) && mu[bot] > A.mu_night) {
       const double m = fmin(-Bf * dt / (P.cp * jump), mu[bot] - A.mu_night);
-      const double qx = MOIST && A.edge_vap > 0 ? edge_q<L, MIX>(bot, true, mu, th, q, m, P, A) : q[bot];
+      const double qx = MOIST && FULL && A.edge_vap > 0 ? edge_q<L, MIX>(bot, true, mu, th, q, m, P, A) : q[bot];
       move_mass<L, MOIST, CLOUD>(P, mu, th, q, pib, bot, bot - 1, m, th[bot], th[bot], qx, qx, cl);
       wxo[bot - 1] += m;
     }
     if (A.bl_lcl > 0) {
       const double m = mu[bot] - fmax(lcl_mass<L, MIX>(mu, th[bot], q[bot], P, A), A.mu_night);
       if (m > 0) {
-        const double qx = MOIST && A.edge_vap > 0 ? edge_q<L, MIX>(bot, true, mu, th, q, m, P, A) : q[bot];
+        const double qx = MOIST && FULL && A.edge_vap > 0 ? edge_q<L, MIX>(bot, true, mu, th, q, m, P, A) : q[bot];
         move_mass<L, MOIST, CLOUD>(P, mu, th, q, pib, bot, bot - 1, m, th[bot], th[bot], qx, qx, cl);
         wxo[bot - 1] += m;
       }
@@ -1973,7 +1986,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
     for (int k = 0; k < bot; k++) pi_ += P.grav * mu[k];
     const double th0 = th[bot];
     double q0 = q[bot];
-    if (A.plume_root > 0) {
+    if (FULL && A.plume_root > 0) {
       // plume_root: plumes root in the air at the surface, the layer's vapor at its relative humidity there (edge_q
       // at its bottom edge); root_q: plus the thermals' excess b E / (rho w_m), b = 8.5, w_m = (u*^3 + 0.28 w*^3)^(1/3)
       // (Holtslag & Boville 1993), up to the surface air's saturation; else with clouds its moistest part by the
@@ -2002,7 +2015,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
       q0 = fmax(q0, fmin((double)qs, q0 + (1 - A.rh_crit) * qs));
     }
     double thp, qc, thp2, qc2;
-    if (A.plume_deep > 0 && bot >= 2) {
+    if (FULL && A.plume_deep > 0 && bot >= 2) {
       // the deep plume: its full ascent against the layers' spread air, mixing and entraining; the air it rises
       // through sinks to make room, warming each level by the theta it had below, so the mass that removes its
       // buoyancy is A / (theta_d - theta*), relaxed over tau_conv; it takes in the cloud layer's air it entrained (me),
@@ -2016,10 +2029,10 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
       if (kd >= 0 && Ab > 0) {
         const double rise = thp - tstar<L>(bot - 1, P);
         mc = fmin(Ab / (rise > 1 ? rise : 1.0), mu[bot] - P.floor_) * omexp<MIX>(dt / A.tau_conv);
-        if (A.plume_root > 0 && q0 > 0) mc = fmin(mc, mu[bot] * q[bot] / q0);
+        if (FULL && A.plume_root > 0 && q0 > 0) mc = fmin(mc, mu[bot] * q[bot] / q0);
         // the mixed boundary layer (bl_q): plumes leave it through the clouds at its top, at most rho a w* with a
         // their share there and w* the free convection's velocity scale (Neggers, Stevens & Neelin 2006)
-        if (blm && A.bl_q > 0) {
+        if (blm && FULL && A.bl_q > 0) {
           double l_, f_, d_;
           if (mixed_cloud<L, MIX>(bot, mu, th[bot], q[bot] + (CLOUD ? cl[bot] : 0.0), P, A, l_, f_, d_,
                                   A.cu_cloud > 0)) {
@@ -2032,7 +2045,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
         // cu_dth: through the cumulus and cloud layers, the air it took in from each (the layer it stops in included)
         // moved by plume_out
         double cond_cu = 0, det_cu = 0, G_cu = 1;
-        const bool cu = A.cu_dth > 0;
+        const bool cu = FULL && A.cu_dth > 0;
         if (mc > 0 && cu)
           plume_out<L, CLOUD>(P, mu, th, q, pib, cl, kd, mc, th0, q0, thp, qc, Gl, qx, wxo, A.l_det, cond_cu, det_cu,
                               G_cu);
@@ -2209,7 +2222,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
     // root_q), entraining twice the deep one's with ent_ifs, stopping in the cloud layer and leaving its air there;
     // its base mass flux Grant (2001)'s rho a w* (a = shallow), cut to the air and vapor the layers hold. Its
     // condensate leaves as the deep plume's: l_det as cloud, the rest rains, its frozen share as snow
-    if (A.shallow > 0 && A.plume_deep > 0 && bot >= 2 && ex_r >= 0 && ws_r > 0) {
+    if (A.shallow > 0 && FULL && A.plume_deep > 0 && bot >= 2 && ex_r >= 0 && ws_r > 0) {
       constexpr int ks = bot >= 1 ? bot - 1 : 0;
       double pis = 0;
 #pragma unroll
@@ -2222,7 +2235,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
       plume_ascent<L, MIX>(mu, th, q, ths0, qs0, pis, P, A, As, kds, thps, qcs, qxs, lts, Gs, FZs, Gls, true);
 #pragma unroll
       for (int k = 0; k <= bot; k++) xss += qxs[k];
-      if (A.cu_dth > 0) {
+      if (FULL && A.cu_dth > 0) {
         // cu_dth: through the cumulus layer and into the cloud layer above it, stopping in either; what it took in
         // from each moved by plume_out; with buoy_v only through the cloud at the mixed layer's top, its share there
         // at most
@@ -2325,7 +2338,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
     // sinking between the clouds, up to the condensation level: the slice from that layer's bottom edge, its theta
     // and vapor as the mixed layer's entrainment's; sub_mix stirs it toward the cumulus layer's mean
     if constexpr (L >= 3) {
-      if (A.cu_sub > 0 && A.bl_lcl > 0 && blm) {
+      if (FULL && A.cu_sub > 0 && A.bl_lcl > 0 && blm) {
         constexpr int ka = bot - 1;
         const double m = fmin(fmin(mu_pre - mu[bot], lcl_mass<L, MIX>(mu, th[bot], q[bot], P, A) - mu[bot]),
                               mu[ka] - P.floor_);
@@ -2333,7 +2346,7 @@ __global__ void __launch_bounds__(BS) k_air_column(int N, CP P, AP A, int mode, 
           const double e = tstar<L>(ka, P), fm = fmin(1.0, m / mu[ka]);
           const bool spread = th[ka] < tstar<L>(ka - 1, P) && th[ka] > e;
           double thc = spread ? e + fm * (th[ka] - e) : th[ka];
-          double qx = A.edge_vap > 0 ? edge_q<L, MIX>(ka, false, mu, th, q, m, P, A) : q[ka];
+          double qx = FULL && A.edge_vap > 0 ? edge_q<L, MIX>(ka, false, mu, th, q, m, P, A) : q[ka];
           if (A.sub_mix > 0) {
             thc += A.sub_mix * (th[ka] - thc);
             qx += A.sub_mix * (q[ka] - qx);
@@ -2522,7 +2535,7 @@ int air_column_cloudy(int N, int L, int mixed, bool full, const CP& P, const AP&
     else LAUNCHC(LL, false, false);                                                                                  \
   }
 #define LAUNCHC(LL, MX, FU)                                                                                          \
-  ISW_LAUNCH("air_column", bytes, (k_air_column<LL, MX, true, true, FU>), grid1(N), dim3(BS), N, P, A, mode, t,      \
+  ISW_LAUNCH("air_column", bytes, (k_air_column<LL, MX, true, true, FU>), grid1(N), dim3(BS), A, N, P, mode, t,      \
              insol, pos, uabs, mu, dt, elev, radf, swf, ch, o)
   ISW_BY_L(CALL)
 #undef CALL
@@ -2567,7 +2580,7 @@ int air_column(int N, int L, const double* par, const isw_air* air, int mode, co
                const double* ch, const double* lc, double* firn, double* cloudw, double* cloudo, double* xfer,
                double* dgo, int mixed, hipStream_t st) {
   const CP P = make_cp(par);
-  const AP A = make_ap(par, air);
+  AP A = make_ap(par, air);
   const bool moist = P.moist > 0, cloudy = moist && par[55] > 0 && cloudw;
   if (!moist) land = nullptr;                          // (the dry column has no land)
   const AirIO o{theta, qv, Ts, ice, wx, olr, sw_abs, stored, rain, evap, conv, tsurf, rainp, qocean, qsw, flash,
@@ -2585,11 +2598,14 @@ int air_column(int N, int L, const double* par, const isw_air* air, int mode, co
   // kernel (FULL false), their code compiled away (the dry column is always the full one: bl_mix acts there too)
   const bool full = land || P.bl_mix > 0 || par[51] > 0 || par[53] > 0 || par[86] > 0 || par[85] > 0 ||
                     par[83] > 0 || par[88] > 0 || par[47] > 0 || par[89] > 0 || par[111] > 0 || par[114] > 0;
+  if (!full && moist)
+    A.sat_prof = A.sat_base = A.edge_vap = A.freeze_dry = A.q_shape = A.plume_root = A.plume_deep = A.bl_q = A.cu_dth =
+        A.cu_sub = 0;
   if (cloudy)
     return air_column_cloudy(N, L, mixed, full, P, A, mode, t, insol, pos, uabs, mu, dt, elev, radf, swf, ch, o,
                              bytes, st);
 #define LAUNCH(LL, MX, MO, FU)                                                                                     \
-  ISW_LAUNCH("air_column", bytes, (k_air_column<LL, MX, MO, false, FU>), grid1(N), dim3(BS), N, P, A, mode, t,     \
+  ISW_LAUNCH("air_column", bytes, (k_air_column<LL, MX, MO, false, FU>), grid1(N), dim3(BS), A, N, P, mode, t,     \
              insol, pos, uabs, mu, dt, elev, radf, swf, ch, o)
 #define CALL(LL)                                    \
   if (mixed) {                                      \
