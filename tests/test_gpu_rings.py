@@ -90,8 +90,8 @@ def test_ocean(grids, n, L, nfast, wall, floor, precision):
 @pytest.mark.parametrize('n,L,K', [(4, 1, 1), (3, 3, 1), (4, 2, 2), (2, 5, 1), (4, 7, 1), (4, 2, 4), (3, 3, 3), (4, 4, 3),
                                    (4, 3, 5), (4, 8, 2), (4, 1, 17)])
 def test_transport_rows(grids, n, L, K, precision):
-    """K tracers of L layers by unequal mass fluxes, steep rows among them, and the same rows where the scratch is not
-    padded (one row to a load): both against the oracle, the FP64 form's the same to the bit."""
+    """K tracers of L layers by unequal mass fluxes, steep rows among them (row counts that fill three quarters of their
+    blocks, and ones that do not and are kept apart), and the same rows where the scratch is not padded: both against the oracle, the FP64 form's the same to the bit."""
     import oracle
     from insilica.gpu import DeviceGrid
     from insilica.transport import Transport
