@@ -7,7 +7,7 @@
 // in float, as the reference's MIXED build; every g-point sum stays FP64).
 //
 // Design (MI355X): a 64-aligned block takes columns in turn, one thread per g-point, the column's sub-level properties
-// staged once in LDS as what the walk needs (table offsets, bilinear weights, amounts). Kernels are instantiated per
+// staged once in LDS as what the walk needs (table offsets and shares, amounts). Kernels are instantiated per
 // layer count so that every per-g-point array has a compile-time size and stays in VGPRs, and each walks the sub-levels
 // once: what the walk back needs is kept as small linear maps per layer instead of being computed again. A column's table
 // rows are the same for all its g-points, so their bases are scalar and the lanes differ by g alone. Per-g results go to
@@ -264,22 +264,6 @@ __device__ __forceinline__ tabp row_at(const float* tab, size_t off) {
 // of the column and keeps its operands, two to three times as many, in registers instead.
 __device__ __forceinline__ void pin(fast& x) { asm volatile("" : "+v"(x)); }
 
-// A sub-level's place in the ln k tables: the element offset of its (log p, T) cell and the four corners' bilinear
-// weights. In the mixed form the weights carry log2 e, so that exp(ln k) is the hardware's 2^x of the weighted sum.
-struct Cell {
-  fast w00, w10, w01, w11;
-};
-__device__ __forceinline__ Cell cell_weights(fast fp, fast ft) {
-  const double s = ISW_FORM_MIXED ? 1.4426950408889634 : 1.0, p = fp, t = ft;
-  return Cell{(fast)((1 - p) * (1 - t) * s), (fast)(p * (1 - t) * s), (fast)((1 - p) * t * s), (fast)(p * t * s)};
-}
-__device__ __forceinline__ fast kexp(fast x) {
-#if ISW_FORM_MIXED
-  return __builtin_amdgcn_exp2f(x);
-#else
-  return exp(x);
-#endif
-}
 // One float at a 32-bit byte offset beside a scalar base: no 64-bit lane address.
 __device__ __forceinline__ float at(tabp p, unsigned o) {
   asm("" : "+v"(o));
@@ -300,15 +284,21 @@ struct Corners {
       for (int m = 0; m < 4; m++) v[c][m] = at(K, o[m]);
     }
   }
-  __device__ __forceinline__ fast depth(const Cell& q, const fast* a) const {
+  // ln k is interpolated by its differences on the cell, which are small where ln k is not: by the corners' weights (with
+  // log2 e in them, four operations for seven) each weight's rounding took its share of the whole of ln k, and the
+  // longwave's error against 64 bits was 1.6% larger on average, 4.5% at most, over 24 sets of columns and tables; so it is
+  // 1.0% smaller on average than with one depth at a time, never larger (lw_column at 40,962 x 7 x 256: 1.38 -> 1.44 ms).
+  __device__ __forceinline__ fast depth(fast fp, fast ft, const fast* a) const {
+    const fast fpt = fp * ft;
     fast tau = 0;
 #pragma unroll
-    for (int c = 0; c < NCOMP; c++)
-      tau += a[c] * kexp(q.w00 * (fast)v[c][0] + q.w10 * (fast)v[c][1] + q.w01 * (fast)v[c][2] + q.w11 * (fast)v[c][3]);
+    for (int c = 0; c < NCOMP; c++) {
+      const fast v00 = v[c][0], v10 = v[c][1], v01 = v[c][2], v11 = v[c][3];
+      tau += a[c] * fexp(v00 + (v10 - v00) * fp + (v01 - v00) * ft + (v00 - v01 - v10 + v11) * fpt);
+    }
     return fmax((fast)0, tau);
   }
-  // The same by the differences of ln k on the cell, water's two tables blended by fh: each operation's rounding then as
-  // the layer optics' comment asks.
+  // The same with water's two tables blended by fh: each operation's rounding then as the layer optics' comment asks.
   __device__ __forceinline__ fast blend(fast fp, fast ft, const fast* u, fast fh) const {
     fast lk[NCOMP];
 #pragma unroll
@@ -377,8 +367,7 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
   constexpr int NSS = NSUB * L, RW = L + 1, E0 = 3 * RW + 3;
   using R = LwRows<L>;
   extern __shared__ float red[];                       // R::S per g-point
-  __shared__ Cell sq[NSS];
-  __shared__ fast sa[NSS][6], scl[NSS], sft[NSS], scia[NSS], sfc[L];   // (amounts; cloud; T share; CIA; cover)
+  __shared__ fast sa[NSS][6], scl[NSS], sfp[NSS], sft[NSS], scia[NSS], sfc[L];   // (amounts; cloud; T share; CIA; cover)
   __shared__ fast spt[NSS + 1], spb[NSS];              // Planck table shares (the last: the surface's)
   __shared__ int so[NSS], sit[NSS], sjt[NSS + 1], sjb[NSS];
   const unsigned g = threadIdx.x, NG = t.NG, row = (unsigned)(t.NT * t.NG);
@@ -400,7 +389,7 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
       so[s] = (ip * t.NT + it) * t.NG;
       sit[s] = it * t.NG;
       sft[s] = y - (fast)it;
-      sq[s] = cell_weights(x - (fast)ip, y - (fast)it);
+      sfp[s] = x - (fast)ip;
       const fast u0 = R_(4), fh = R_(9), df = (fast)1.66;
       sa[s][0] = df * (u0 * (1 - fh));                 // (water's two tables blended by its share; diffusivity 1.66)
       sa[s][1] = df * (u0 * fh);
@@ -453,7 +442,7 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
           const int s = k * NSUB + j;
           __builtin_amdgcn_sched_barrier(0);           // (sub-level by sub-level, or the registers run out)
           load(s);
-          fast x = row_s.k.depth(sq[s], sa[s]);          // (1.66 times the optical depth)
+          fast x = row_s.k.depth(sfp[s], sft[s], sa[s]);          // (1.66 times the optical depth)
           if (t.cia) {
             const tabp C = row_at(t.cia, uni(sit[s]));
             x += scia[s] * ((fast)at(C, o4[0]) + ((fast)at(C, o4[2]) - (fast)at(C, o4[0])) * sft[s]);

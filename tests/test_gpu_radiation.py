@@ -180,3 +180,29 @@ def test_columns_at_the_edges(N, L, lwb, swb):
         e_sw = np.max(np.abs(swf - osw))
         print(f'{prec}: lw {e_lw:.2e} sw {e_sw:.2e}', flush=True)
         assert e_lw <= tol and e_sw <= tol
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('L', [2, 7])
+def test_longwave_of_constant_tables(L, precision):
+    """Where ln k is the same at every pressure and temperature, a gas's depth does not depend on where in the tables a
+    sub-level lies: columns that differ in that alone have the same fluxes to the bit. (ln k interpolated by the corners'
+    weights takes the weights' rounding times all of ln k with it and fails here in the mixed form.)"""
+    from insilica.ktables import synthetic_lw
+    from insilica.radiation import Longwave
+    N = 64
+    print(f'case: longwave, constant tables, L={L} {precision}', flush=True)
+    c, _, par = case(N, L, 31)
+    lwk = synthetic_lw(bands=4, seed=L)
+    lwk['logk'] = np.broadcast_to(np.median(lwk['logk'], axis=(1, 2), keepdims=True), lwk['logk'].shape).copy()
+    lw = Longwave(N, L, par, tables=lwk, precision=precision)
+    mu, th, q, co = (_dev(np.repeat(c[k][:, :1], N, 1)) for k in ('mu', 'theta', 'q', 'cloudo'))
+    lw.setup(mu, th, q, co)
+    sub = lw.sub.view(4 * L, 15, N)
+    rng = np.random.default_rng(L)
+    for row, size in ((2, lwk['logk'].shape[1]), (3, lwk['logk'].shape[2])):
+        sub[:, row] = torch.as_tensor(rng.uniform(0, size - 1.01, (4 * L, N)).astype(np.float32), device='cuda')
+    lw.column(_dev(np.full(N, c['Ts'][0])))
+    torch.cuda.synchronize()
+    radf = _np(lw.radf)
+    assert np.all(np.isfinite(radf)) and np.array_equal(radf, np.repeat(radf[:, :1], N, 1))
