@@ -72,7 +72,10 @@ __device__ __forceinline__ fast fquot(fast a, fast b) {
 // The shortwave's layer optics divide by 1 - (k mu0)^2, which passes through zero where the beam and the diffuse light
 // decay alike: what they lose to rounding there is a thousand times larger, so their quotients and square root are
 // rounded as IEEE's are: one Newton step on the hardware's reciprocal (or reciprocal root), then one on the residual, and
-// the fix-up for zeros and infinities. Six instructions besides the reciprocal where the compiler's division takes ten.
+// the fix-up for zeros and infinities. Six instructions besides the reciprocal where the compiler's division takes ten, for
+// it does not scale: where b is denormal its reciprocal is infinite and the Newton step not a number, so what may vanish
+// is divided by only above TINY.
+constexpr fast TINY = ISW_FORM_MIXED ? (fast)1.17549435e-38f : (fast)0;
 __device__ __forceinline__ fast fdiv(fast a, fast b) {
 #if ISW_FORM_MIXED
   float y = __builtin_amdgcn_rcpf(b);
@@ -716,8 +719,8 @@ __global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int
         // the sub-level's optics: molecules, haze and gas (air.cu:2440-2458), with the cloud's share mixed in
         const fast trs = ray * sr[s] * (fast)air.ray, ths = (fast)t.tau550 * hzf * sh[s];
         const fast tt = tg + trs + ths, sc = trs + (fast)t.hssa * ths;
-        const fast ssa = tt > 0 ? fmin(fdiv(sc, tt), (fast)(1 - 1e-6)) : (fast)0;
-        const fast ga = sc > 0 ? fdiv((fast)t.hg * (fast)t.hssa * ths, sc) : (fast)0;
+        const fast ssa = tt > TINY ? fmin(fdiv(sc, tt), (fast)(1 - 1e-6)) : (fast)0;
+        const fast ga = sc > TINY ? fdiv((fast)t.hg * (fast)t.hssa * ths, sc) : (fast)0;
         fast cRd, cTd, cRs, cTs, cTdd;
         sw_layer(tt, ssa, ga, mu0, cRd, cTd, cRs, cTs, cTdd);
         fast rd = cRd, td = cTd, rs = cRs, ts = cTs, tdd = cTdd;
@@ -728,12 +731,12 @@ __global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int
           if (t.cssa_i) {
             const fast sl = sli[s], wl = sl * cssa, wi = (1 - sl) * cssa_i;
             cw = wl + wi;
-            cg = cw > 0 ? fdiv(wl * (fast)P.cloud_g + wi * g_i, cw) : cg;
+            cg = cw > TINY ? fdiv(wl * (fast)P.cloud_g + wi * g_i, cw) : cg;
           }
           const fast sc2 = sc + cw * tc;
-          const fast g2 = fdiv(ga * sc + cg * cw * tc, sc2);
+          const fast g2 = sc2 > TINY ? fdiv(ga * sc + cg * cw * tc, sc2) : (fast)0;
           fast r1, t1, r2, t3, d1;
-          sw_layer(t2, fmin(fdiv(sc2, t2), (fast)(1 - 1e-6)), g2, mu0, r1, t1, r2, t3, d1);
+          sw_layer(t2, t2 > TINY ? fmin(fdiv(sc2, t2), (fast)(1 - 1e-6)) : (fast)0, g2, mu0, r1, t1, r2, t3, d1);
           rd = (1 - f) * cRd + f * r1;
           td = (1 - f) * cTd + f * t1;
           rs = (1 - f) * cRs + f * r2;

@@ -206,3 +206,27 @@ def test_longwave_of_constant_tables(L, precision):
     torch.cuda.synchronize()
     radf = _np(lw.radf)
     assert np.all(np.isfinite(radf)) and np.array_equal(radf, np.repeat(radf[:, :1], N, 1))
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('ray,haze', [(1e-41, 0.0), (0.0, 1e-41), (1e-41, 1e-41)])
+def test_shortwave_of_vanishing_depths(ray, haze, precision):
+    """Gases that absorb nothing, and molecules and haze whose depths are denormal in the mixed form: the light passes as
+    if they were not there (nothing is divided by a denormal depth)."""
+    from insilica.ktables import synthetic_lw, synthetic_sw
+    from insilica.radiation import Longwave, Shortwave
+    N, L = 64, 3
+    print(f'case: shortwave, vanishing depths, ray {ray} haze {haze} {precision}', flush=True)
+    c, pos, par = case(N, L, 33)
+    swk = synthetic_sw(bands=4, seed=2)
+    swk['logk'] = np.full_like(swk['logk'], -1000.0)
+    out = []
+    for r, h in ((ray, haze), (0.0, 0.0)):
+        lw = Longwave(N, L, par, tables=synthetic_lw(bands=4, seed=1), precision=precision)
+        swk['haze_par'] = np.concatenate([[h], swk['haze_par'][1:]])
+        sw = Shortwave(N, L, par, lw, tables=swk, air=dict(ray=r), precision=precision)
+        lw.setup(*(_dev(c[k]) for k in ('mu', 'theta', 'q')), None)
+        sw(0, _dev([3.0e6]), 3600.0, _dev(pos), _dev(c['alb']), None)
+        torch.cuda.synchronize()
+        out.append(_np(sw.swf))
+    assert np.all(np.isfinite(out[0])) and np.max(np.abs(out[0] - out[1])) <= 1e-6
