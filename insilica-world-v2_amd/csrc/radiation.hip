@@ -318,19 +318,23 @@ struct Corners {
 // Per-g float values in LDS summed over the g-points: g-point m's values at red[m * S ..], S odd, so that a wave's writes
 // fall on different banks and every value's address is the lane's own plus a constant (with rows g-points long, their
 // run-time length cost a register per row for the addresses). Eight lanes per row, each adding every eighth g-point in
-// FP64, then three exchanges: a fixed order, so results repeat bit for bit. Lane 0 of the eight gets the row's sum.
-template <int ROWS, int S, class F>
-__device__ __forceinline__ void g_sums(const float* red, int NG, F&& put) {
+// FP64, then three exchanges: a fixed order, so results repeat bit for bit. Lane 0 of the eight gets the row's sum. slot(r):
+// where row r's values are.
+template <int ROWS, int S, class At, class F>
+__device__ __forceinline__ void g_sums(const float* red, int NG, At&& slot, F&& put) {
   static_assert(S % 2 == 1 && ROWS <= S, "odd stride");
   const int part = (int)threadIdx.x & 7, nr = (int)blockDim.x >> 3;
   for (int r = (int)threadIdx.x >> 3; r < ROWS; r += nr) {
+    const int at = slot(r);
     double v = 0;
-    for (int m = part; m < NG; m += 8) v += (double)red[m * S + r];
+    for (int m = part; m < NG; m += 8) v += (double)red[m * S + at];
 #pragma unroll
     for (int o = 4; o >= 1; o >>= 1) v += __shfl_xor(v, o);
     if (part == 0) put(r, v);
   }
 }
+
+__device__ __forceinline__ int same(int r) { return r; }
 
 // f(S), f(S - 1), .., f(0), each with its own constant.
 template <int S, class F>
@@ -502,7 +506,7 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
     }
     // the sums of the way down: radf's rows RW + k + 1 and the layers' inner edges
     auto sums_down = [&]() {
-      g_sums<R::NDN, R::S>(red + R::DN0, (int)NG, [&](int q, double w) {
+      g_sums<R::NDN, R::S>(red + R::DN0, (int)NG, same, [&](int q, double w) {
         const int k = q / 3, m = q - 3 * k;
         radf[(size_t)(m == 0 ? RW + k + 1 : E0 + 6 * k + (m == 1 ? 1 : 4)) * N + i] = w;
       });
@@ -543,7 +547,7 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
       for (int m = (int)threadIdx.x & 63; m < (int)NG; m += 64) bsum += (double)red[m * R::S + 3];
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) bsum += __shfl_xor(bsum, o);
-      g_sums<R::NUP, R::S>(red, (int)NG, [&](int q, double w) {
+      g_sums<R::NUP, R::S>(red, (int)NG, same, [&](int q, double w) {
         int r;
         bool over = false;
         if (q < 4) {
@@ -708,7 +712,7 @@ __global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int
       // 1 - As there
       fast md[L][3], ma[L][3], mc[L][3], nd[L][3], ns[L][3];
       auto walk = [&](int s) __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_barrier(0);             // (sub-level by sub-level: see ISW_RAD_WAVES)
+        __builtin_amdgcn_sched_barrier(0);             // (sub-level by sub-level, or the registers run out)
         Corners<7> row_s;
         row_s.load(t.logk, (size_t)uni(so[s]), cs, o4);
         fast tg = row_s.blend(sfp[s], sft[s], su[s], sfh[s]);
@@ -809,10 +813,15 @@ __global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int
       slot[3] = (float)(wg * cAs);
     }
     __syncthreads();
-    g_sums<6 * L, S>(red, (int)NG, [&](int q, double v) {
-      const int k = q / 6, m = q - 6 * k;              // (layer, slot: 0 the top sub-level's, 4 the bottom's, 5 its own)
-      const int r = m == 0 ? L + 2 + 2 * k : m == 4 ? L + 3 + 2 * k : m == 5 ? k : k == 0 && m >= 2 ? L + m - 2 : -1;
-      if (r >= 0) swf[(size_t)r * N + i] = v;
+    // the rows' slots: the layers' absorption, top and bottom sub-level's, then the surface's two
+    g_sums<3 * L + 2, S>(red, (int)NG, [](int r) {
+      if (r >= 3 * L) return r - 3 * L + 2;
+      const int k = r / 3, m = r - 3 * k;
+      return 6 * k + (m == 0 ? 5 : m == 1 ? 0 : 4);
+    }, [&](int r, double v) {
+      const int k = r / 3, m = r - 3 * k;
+      const int row = r >= 3 * L ? L + r - 3 * L : m == 0 ? k : L + 1 + 2 * k + m;
+      swf[(size_t)row * N + i] = v;
     });
     if (i + 1 < i1) stage(i + 1);
     __syncthreads();
