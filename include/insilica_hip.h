@@ -154,7 +154,9 @@ typedef struct isw_transport {
 
 /* Layers.step (reference: src/insilica/layers.py:311-338; kernels/layers.cu): one time-split RK3 step in place on
  * h (L,N) and u (L,E); theta (L,N) for air, else NULL; Fm (L,E, nullable) receives the last stage's l*dt*F.
- * Stage s takes ceil(c_s * nfast) fast sub-steps (c = 1/3, 1/2, 1). Then the interfacial stress (vmix). */
+ * Stage s takes ceil(c_s * nfast) fast sub-steps (c = 1/3, 1/2, 1). Then the interfacial stress (vmix). lay->F (L,E) is
+ * scratch of the air's last stage with rg_* tables and a batch, or sub-steps that fit one launch (rg_k at most);
+ * refused (ISW_EBADARG) when it is needed and NULL. */
 int32_t isw_layers_step(const isw_grid* g, const isw_layers* lay, double* h, double* u, double* theta, double* Fm,
                         double dt, int32_t nfast, void* stream);
 

@@ -2346,6 +2346,9 @@ int layers_step(const isw_grid* g, const isw_layers* s, double* h, double* u, do
   const Div dv = divs(g);
   const int N = g->N, L = s->L;
   const double n_ = N, e_ = g->E, l_ = L;
+  // (the last stage's copy of u, where one launch takes all of its sub-steps)
+  const int KR = s->air ? ring_most(g, L, AIR_STEPS) : 0;
+  if (KR && !s->F && (s->batch || nfast <= KR)) return ISW_EBADARG;
   if (s->air) {
     ISW_LAUNCH("air_stiff", 3 * l_ * n_ * D, k_air_stiff, c1(N), BS1, N, p, h, theta, s->S);
   } else {

@@ -172,6 +172,54 @@ def test_grid_check_pair_tables():
     assert lib.isw_grid_check(None) == E
 
 
+def _grid(n=642, patches=False, rings=False):
+    """A mesh struct whose tables are host buffers that the host checks do not look into."""
+    g = _hip.IswGrid()
+    g.N, g.E, g.NV = n, 3 * (n - 2), 2 * (n - 2)
+    p32 = ctypes.cast((ctypes.c_int32 * 8)(), _hip._i32p)
+    for k in ('eI', 'eJ', 'cellEdge', 'cellEdgeAsc'):
+        setattr(g, k, p32)
+    g.cellSign = ctypes.cast((ctypes.c_int8 * 8)(), _hip._i8p)
+    g.le = g.de = g.areaCell = g.rA = g.rde = g.rAV = ctypes.cast((ctypes.c_double * 8)(), _hip._f64p)
+    g.wf = g.d2wtf = ctypes.cast((ctypes.c_float * 8)(), _hip._f32p)
+    if patches:
+        g.npatch, g.pcells, g.pslots, g.pown, g.ptedges = (n + 63) // 64, 64, 120, 200, 230
+        g.eslot = g.cellSign
+        for k in ('ph_off', 'ph_cell', 'pe_off', 'pe_edge', 'pe_slot', 'pi_off', 'pi_edge', 'tc_slot'):
+            setattr(g, k, p32)
+    if rings:
+        g.rg_k, g.rg_npatch, g.rg_owned = 4, (n + 63) // 64, 190
+        for r in range(6):
+            g.rg_cells[r], g.rg_edges[r] = 64 + 40 * r, 220 + 120 * r
+        for k in ('head', 'cell', 'slot', 'edge', 'ecell'):
+            setattr(g, 'rg_' + k, p32)
+    return g
+
+
+def test_air_step_refused_without_its_scratch():
+    """The air's last stage reads a copy of the winds in F where one launch takes all of its sub-steps, and always in a
+    batch: refused without F, before any launch."""
+    lib = _hip.lib()
+    g = _grid(rings=True)
+    one = ctypes.cast((ctypes.c_double * 8)(), _hip._f64p)
+    lay = _hip.IswLayers()
+    lay.L, lay.air, lay.prec = 3, 1, _hip.ISW_FP64
+    for k in _hip.LAYER_SCRATCH + ('fV', 'b', 'Gc', 'cfc'):
+        setattr(lay, k, one)
+    lay.F = None
+    step = lambda nfast: lib.isw_layers_step(ctypes.byref(g), ctypes.byref(lay), one, one, one, None, 900.0, nfast, None)
+    assert step(1) == _hip.ISW_EBADARG and step(3) == _hip.ISW_EBADARG
+    b = _hip.IswBatch()
+    b.nworlds = 1
+    p32 = ctypes.cast((ctypes.c_int32 * 8)(), _hip._i32p)
+    b.wc = b.we = b.nsub = p32
+    b.grav = b.nu4 = b.tau = b.inv_n = one
+    for k in range(3):
+        b.nmax[k] = 12
+    lay.batch = ctypes.pointer(b)
+    assert step(12) == _hip.ISW_EBADARG
+
+
 def test_ocean_column_refusals():
     """The ocean's column entry points refuse bad sizes and settings on the host (no launch)."""
     lib = _hip.lib()
