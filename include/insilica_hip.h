@@ -140,11 +140,11 @@ typedef struct isw_layers {
 
 /* FCT transport scratch for up to rows_max rows (reference: src/insilica/transport.py:19-30 Transport.__init__).
  * (rows,N): td, p1, p2, Rp, Rm; (rows,E): Hf, A; pf: (rows,N) floats for the mixed form's stencil copy, else NULL;
- * with rows_pad, of that many rows each, 16-byte aligned. */
+ * with rows_pad, of that many rows each, 16-byte aligned (else the rows are kept apart). */
 typedef struct isw_transport {
   int32_t L, rows_max, prec;
-  int32_t rows_pad; /* the rows every scratch array holds: at least the rows rounded up to a multiple of four lets the
-                     * passes keep them cell-major on the grid's patches; less (0) keeps them apart */
+  int32_t rows_pad; /* the rows every scratch array holds: rows_max or more, and at least the rows rounded up to a multiple
+                     * of four, lets the passes keep them cell-major on the grid's patches; less (0) keeps them apart */
   double beta;
   double *td, *p1, *p2, *Rp, *Rm, *Hf, *A;
   float *pf;
@@ -504,6 +504,9 @@ const char* isw_version(void);
  * consistent, at most ISW_PAIR_THREADS owned edges and patch-and-halo cells per patch for the two-sub-step tables). isw_air_column_options:
  * the column options (par in PAR_ORDER, host) that isw_air_column does not carry for L layers. */
 int32_t isw_grid_check(const isw_grid* g);
+/* The rows to a block (4 or 8) that isw_transport_step takes for this many rows at order 3, 0 where it keeps the rows
+ * apart, ISW_EBADARG for a refused grid or row count (host only, as the checks above). */
+int32_t isw_transport_shape(const isw_grid* g, const isw_transport* tr, int32_t rows);
 int32_t isw_air_column_options(int32_t L, const double* par);
 
 /* The mountains' drag on the air (reference: OroDrag.apply, orodrag.py:62-68; kernels/drag.cu:40-193, Lott & Miller

@@ -23,6 +23,7 @@
                       double*, int, double, hipStream_t);                                                            \
   int vmix_heat(const isw_grid*, const isw_layers*, const double*, const double*, double*, hipStream_t);            \
   int mass_update(const isw_grid*, int, const double*, const double*, double*, hipStream_t);                        \
+  int transport_shape(const isw_grid*, const isw_transport*, int);                                                  \
   int transport_step(const isw_grid*, const isw_transport*, const double*, const double*, const double*, double*,   \
                      int, int, hipStream_t);                                                                         \
   int swe_step(const isw_grid*, const isw_layers*, double*, double*, double*, double, hipStream_t);                 \
@@ -401,6 +402,11 @@ int32_t isw_ice_flow(const isw_grid* g, const double* b, const double* land, dou
 const char* isw_version(void) { return "insilica_hip 0.1 gfx950"; }
 
 int32_t isw_grid_check(const isw_grid* g) { return grid_ok(g) ? 0 : ISW_EBADARG; }
+
+int32_t isw_transport_shape(const isw_grid* g, const isw_transport* tr, int32_t rows) {
+  if (!grid_ok(g) || !tr || rows < 1 || rows > tr->rows_max || !prec_ok(tr->prec)) return ISW_EBADARG;
+  return DISPATCH(tr->prec, transport_shape(g, tr, rows));
+}
 
 int32_t isw_air_column_options(int32_t L, const double* par) {
   if (L < 2 || L > ISW_LMAX || !par) return ISW_EBADARG;

@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <type_traits>
 
@@ -2420,6 +2421,24 @@ int mass_update(const isw_grid* g, int L, const double* M0, const double* Fm, do
   return (int)hipGetLastError();
 }
 
+// The rows to a block of the passes that keep the rows cell-major on the patches (4 or 8), 0 for those that keep them apart.
+// They need the patches, the scratch's rows padded to a multiple of four (rows_pad at least rows_max: a smaller one is
+// taken as not given) and every array of it where 16 bytes are loaded at once.
+int transport_shape(const isw_grid* g, const isw_transport* tr, int rows) {
+  const int RS = (rows + 3) / 4 * 4, RC = RS > 4 ? 8 : 4, chunks = (RS + RC - 1) / RC;
+  if (!g->pi_off || g->pcells != BS1 || g->E < g->N || RS > tr->rows_pad || tr->rows_max > tr->rows_pad) return 0;
+  if (ISW_FORM_MIXED && !tr->pf2) return 0;
+  const void* at[] = {tr->td, tr->p1, tr->p2, tr->Rp, tr->Rm, tr->Hf, tr->A, tr->pf, tr->pf2};
+  for (const void* p : at)
+    if (reinterpret_cast<uintptr_t>(p) & 15) return 0;
+  // Eight rows to a block share its edges' tables twice as often as four (15 rows at level 6: 96.1 us of kernels against
+  // 110.4); four where no more are there. Only where at least three in four of the blocks' rows are real, for the others
+  // cost as much: 9 and 10 rows of 16 at level 6 81 and 88 us with the rows apart against 88 and 92, 5 of 8 (FP64) 63
+  // against 65, but 12 of 16 (FP64) 108 against 103, 20 of 24 153 against 129, 3 of 4 44 against 41
+  if (4 * rows < 3 * RC * chunks || (size_t)g->ptedges * RC * 2 * sizeof(double) > 65536) return 0;
+  return RC;
+}
+
 // Transport.step_many (transport.py:40-71) on rows stacked in psi; the result is written back into psi.
 int transport_step(const isw_grid* g, const isw_transport* tr, const double* M0, const double* M1, const double* Fm,
                    double* psi, int rows, int order, hipStream_t st) {
@@ -2432,16 +2451,12 @@ int transport_step(const isw_grid* g, const isw_transport* tr, const double* M0,
   float* pf = nullptr;
   const fast* wt = g->d2wt;
 #endif
-  // On the patches with the rows cell-major, where the scratch holds them padded: psi's cell-major copy is in Hf, the FP32
-  // copies alternate between pf and pf2 (stage 1 writes p1's to pf2; stage 2 reads it and writes p2's to pf). Eight rows to
-  // a block share its edges' tables twice as often as four (15 rows at level 6: 96.1 us of kernels against 110.4); four
-  // where no more are there. Only where at least three in four of the blocks' rows are real, for the others cost as much:
-  // 9 and 10 rows of 16 at level 6 81 and 88 us with the rows apart against 88 and 92, 5 of 8 (FP64) 63 against 65, but
-  // 12 of 16 (FP64) 108 against 103, 20 of 24 153 against 129, 3 of 4 44 against 41
-  const int RS = (rows + 3) / 4 * 4, RC = RS > 4 ? 8 : 4, chunks = (RS + RC - 1) / RC;
-  const size_t lds = (size_t)g->ptedges * RC * sizeof(double);
-  if (order == 3 && 4 * rows >= 3 * RC * chunks && g->pi_off && g->pcells == BS1 && E >= N && RS <= tr->rows_pad && (!ISW_FORM_MIXED || tr->pf2) &&
-      2 * lds <= 65536) {
+  // On the patches with the rows cell-major: psi's cell-major copy is in Hf, the FP32 copies alternate between pf and pf2
+  // (stage 1 writes p1's to pf2; stage 2 reads it and writes p2's to pf).
+  const int RC = order == 3 ? transport_shape(g, tr, rows) : 0;
+  if (RC) {
+    const int RS = (rows + 3) / 4 * 4, chunks = (RS + RC - 1) / RC;
+    const size_t lds = (size_t)g->ptedges * RC * sizeof(double);
     const double tabs = 2 * e_ * I + 6 * n_ * I, edge1 = 8 * e_ * (R + I) + l_ * e_ * D + 2 * e_ * I;
     double* pc = tr->Hf;
 #if ISW_FORM_MIXED

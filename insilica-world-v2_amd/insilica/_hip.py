@@ -161,6 +161,7 @@ def lib():
             'isw_ocn_fresh': [i32, vp, vp, vp, vp, vp, vp, vp, d, vp, vp, vp, vp, vp, vp, vp],
             'isw_ocn_diffuse': [vp, i32, vp, vp, vp, vp, vp, vp, d, d, vp],
             'isw_grid_check': [vp],
+            'isw_transport_shape': [vp, vp, i32],
             'isw_air_column_options': [i32, vp],
             'isw_oro_drag': [vp, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, d, vp, vp],
             'isw_wave_drag': [vp, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, d, vp, vp],
@@ -183,7 +184,7 @@ EXPORTS = ('isw_layers_step', 'isw_layers_lap', 'isw_layers_gfast', 'isw_layers_
            'isw_ocn_cap', 'isw_dsum', 'isw_csum', 'isw_dsum_noalloc', 'isw_fill', 'isw_lw_setup', 'isw_lw_column', 'isw_sw_column',
            'isw_hs_column', 'isw_surface_layer', 'isw_cell_speed', 'isw_cell_speed_perot', 'isw_gas_src',
            'isw_advance_time', 'isw_air_column', 'isw_timing_start', 'isw_timing_stop', 'isw_version',
-           'isw_grid_check', 'isw_air_column_options', 'isw_ocn_overturn', 'isw_ocn_forcing', 'isw_ocn_column',
+           'isw_grid_check', 'isw_transport_shape', 'isw_air_column_options', 'isw_ocn_overturn', 'isw_ocn_forcing', 'isw_ocn_column',
            'isw_ocn_xch_salt', 'isw_ocn_pen', 'isw_ocn_fresh', 'isw_ocn_diffuse', 'isw_mesh_lloyd_device',
            'isw_land_route', 'isw_ice_flow', 'isw_oro_drag', 'isw_wave_drag', 'isw_tide_pot',
            'isw_tide_itd', 'isw_tide_mix')

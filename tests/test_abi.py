@@ -4,6 +4,8 @@ import ctypes
 import re
 from pathlib import Path
 
+import pytest
+
 from insilica import _hip
 
 HEADER = Path(__file__).resolve().parent.parent / 'include' / 'insilica_hip.h'
@@ -218,6 +220,34 @@ def test_air_step_refused_without_its_scratch():
         b.nmax[k] = 12
     lay.batch = ctypes.pointer(b)
     assert step(12) == _hip.ISW_EBADARG
+
+
+@pytest.mark.parametrize('prec', [_hip.ISW_FP64, _hip.ISW_MIXED])
+def test_transport_keeps_rows_apart(prec):
+    """The transport's passes that load 16 bytes at once run only where every scratch array is aligned for it and is said to
+    hold the rows padded, and at least as many as rows_max."""
+    lib = _hip.lib()
+    g = _grid(n=40962, patches=True)
+    tr = _hip.IswTransport()
+    tr.L, tr.rows_max, tr.rows_pad, tr.prec = 3, 15, 16, prec
+    arrays = [k for k, _ in _hip.IswTransport._fields_ if k not in ('L', 'rows_max', 'rows_pad', 'prec', 'beta')]
+    put = lambda k, at: setattr(tr, k, ctypes.cast(ctypes.c_void_p(at), dict(_hip.IswTransport._fields_)[k]))
+    for k in arrays:
+        put(k, 1 << 20)
+    shape = lambda rows: lib.isw_transport_shape(ctypes.byref(g), ctypes.byref(tr), rows)
+    assert shape(15) == 8 and shape(3) == 4
+    for k in arrays:
+        put(k, (1 << 20) + 8)
+        assert shape(15) == 0 and shape(3) == 0, k
+        put(k, 1 << 20)
+    for pad in (0, -16, 12, 14):
+        tr.rows_pad = pad
+        assert shape(15) == 0 and shape(3) == 0, pad
+    tr.rows_pad = 15                                                   # 12 rows fit, 15 padded do not
+    assert shape(15) == 0 and shape(12) > 0
+    assert shape(16) == _hip.ISW_EBADARG and shape(0) == _hip.ISW_EBADARG
+    tr.prec = 7
+    assert shape(15) == _hip.ISW_EBADARG
 
 
 def test_ocean_column_refusals():
