@@ -2125,7 +2125,7 @@ static size_t ring_lds(const isw_grid* g, int rows, int m) {
   return (size_t)rows * (ring_ept(g, m) * RBS + 2 + ring_cpt(g, m) * RBS) * sizeof(double);
 }
 static int ring_most(const isw_grid* g, int rows, int want) {
-  if (!g->rg_head || g->rg_owned > RBS) return 0;
+  if (!g->rg_head || g->rg_owned > RBS || g->rg_cells[0] > RBS) return 0;   // (each on a thread of its own)
   int m = want < g->rg_k ? want : g->rg_k;
   while (m > 0 && (ring_ept(g, m) > 4 || g->rg_cells[m] > 2 * RBS || ring_lds(g, rows, m) > 65536)) m--;
   return m;

@@ -198,6 +198,33 @@ def _grid(n=642, patches=False, rings=False):
     return g
 
 
+def test_grid_check_ring_tables():
+    """The ring tables are refused without one of them, with a depth the patch records do not hold, without patches, with
+    fewer edges than a patch owns, and where a ring's places do not fit their slots."""
+    lib = _hip.lib()
+    check = lambda g: lib.isw_grid_check(ctypes.byref(g))
+    assert check(_grid(rings=True)) == 0
+    for k in ('cell', 'slot', 'edge', 'ecell'):
+        g = _grid(rings=True)
+        setattr(g, 'rg_' + k, None)
+        assert check(g) == _hip.ISW_EBADARG, k
+    for k, bad in (('rg_k', 0), ('rg_k', 6), ('rg_npatch', 0), ('rg_owned', 0)):
+        g = _grid(rings=True)
+        setattr(g, k, bad)
+        assert check(g) == _hip.ISW_EBADARG, (k, bad)
+    for r in range(5):
+        for k, bad in (('rg_edges', 189), ('rg_cells', 0), ('rg_edges', 0x7fff), ('rg_cells', 0x7fff)):
+            g = _grid(rings=True)
+            getattr(g, k)[r] = bad
+            assert check(g) == _hip.ISW_EBADARG, (k, r, bad)
+    g = _grid(rings=True)
+    g.rg_cells[5] = g.rg_edges[5] = 0                                  # (beyond the depth: not read)
+    assert check(g) == 0
+    g.rg_head = None                                                   # without the tables nothing of them is looked at
+    g.rg_k = 0
+    assert check(g) == 0
+
+
 def test_air_step_refused_without_its_scratch():
     """The air's last stage reads a copy of the winds in F where one launch takes all of its sub-steps, and always in a
     batch: refused without F, before any launch."""

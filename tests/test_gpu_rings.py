@@ -22,12 +22,16 @@ def _np(t):
     return t.detach().cpu().numpy().copy()
 
 
-def _step(g, precision, kw, h, u, dt, nfast, theta=None):
-    """One step of the library and of the oracle: their largest differences by name."""
+def _step(g, precision, kw, h, u, dt, nfast, theta=None, edit=None):
+    """One step of the library and of the oracle: their largest differences by name. With edit, a change of the mesh struct,
+    the same step on the changed mesh instead, and the names of the kernels that it launched."""
     import oracle
+    from insilica import _hip
     from insilica.gpu import DeviceGrid
     from insilica.layers import Layers
     dg, og = DeviceGrid(g, precision), oracle.Grid(g)
+    if edit:
+        edit(dg.s)
     lay, olay = Layers(dg, **kw), oracle.Layers(og, **kw)
     hd, ud, Fd = dg.asarray(h), dg.asarray(u), dg.zeros(kw['layers'], g.E)
     ho, uo, Fo = h.copy(), u.copy(), np.zeros((kw['layers'], g.E))
@@ -35,42 +39,35 @@ def _step(g, precision, kw, h, u, dt, nfast, theta=None):
     if theta is not None:
         lay.update_gfast(hd, td)
         olay.update_gfast(ho, theta)
+    if edit:
+        torch.cuda.synchronize()
+        _hip.timing_start()
     lay.step(hd, ud, dt, nfast, Fd, theta=td)
     olay.step(ho, uo, dt, nfast, Fo, theta=theta)
     torch.cuda.synchronize()
-    return dict(h=relmax(_np(hd), ho), u=relmax(_np(ud), uo), Fm=relmax(_np(Fd), Fo))
+    diff = dict(h=relmax(_np(hd), ho), u=relmax(_np(ud), uo), Fm=relmax(_np(Fd), Fo))
+    print(diff, flush=True)
+    return (diff, set(_hip.timing_stop())) if edit else diff
 
 
-@pytest.mark.parametrize('precision', ['double', 'mixed'])
-@pytest.mark.parametrize('n,L,nfast', [(6, 2, 3), (6, 8, 1), (2, 3, 1), (3, 3, 2), (4, 3, 3), (4, 1, 4), (4, 2, 5), (4, 4, 7), (3, 5, 9),
-                                       (4, 6, 11), (4, 7, 8), (4, 8, 6)])
-def test_air(grids, n, L, nfast, precision):
+def _air(g, n, L):
+    """An air stack of L layers: settings, thickness, wind, theta."""
     from insilica import cases
     from insilica.constants import CP_DRY, KAPPA, R_DRY
     from insilica.ocean import visc4
-    print(f'case: air n={n} L={L} nfast={nfast} {precision}', flush=True)
-    g = grids(n)
     st = cases.coupled_stack(g, seed=n + L, lmax=4)
     at = np.linspace(0.0, 2.0, L) if L > 1 else np.array([1.0])
     k, f = np.minimum(at.astype(int), 1), at - np.minimum(at.astype(int), 1)
     theta, u = (np.ascontiguousarray((1 - f)[:, None] * st[x][k] + f[:, None] * st[x][k + 1]) for x in ('theta', 'u'))
     h = np.repeat(st['h'].sum(0)[None] / L, L, 0)
-    kw = dict(layers=L, gprime=[0.0] * (L - 1), nu4=visc4(g, 15.0), floor=10.0,
-              air=dict(cp=CP_DRY, kappa=KAPPA, rd=R_DRY), thin_wind=100.0, stress=[0.0] * (L - 1) + [1e-2])
-    diff = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta)
-    assert max(diff.values()) <= BARS[precision], diff
+    return dict(layers=L, gprime=[0.0] * (L - 1), nu4=visc4(g, 15.0), floor=10.0,
+                air=dict(cp=CP_DRY, kappa=KAPPA, rd=R_DRY), thin_wind=100.0, stress=[0.0] * (L - 1) + [1e-2]), h, u, theta
 
 
-@pytest.mark.parametrize('precision', ['double', 'mixed'])
-@pytest.mark.parametrize('n,L,nfast,wall,floor', [(6, 4, 5, True, 0.995), (2, 2, 1, True, 1.0), (3, 1, 2, False, 1.0), (4, 2, 3, True, 1.0),
-                                                  (4, 2, 4, True, 0.995), (3, 3, 5, True, 0.995), (4, 2, 6, False, 0.995),
-                                                  (4, 5, 9, True, 0.999), (4, 8, 11, True, 0.995)])
-def test_ocean(grids, n, L, nfast, wall, floor, precision):
-    """floor below one: that share of the layers' mean thickness, which many cells start beneath."""
+def _ocean(g, n, L, wall, floor):
+    """An ocean stack of L layers: settings, thickness, wind. floor below one: that share of the mean thickness."""
     from insilica import cases
     from insilica.ocean import visc4
-    print(f'case: ocean n={n} L={L} nfast={nfast} wall={wall} floor={floor} {precision}', flush=True)
-    g = grids(n)
     h2, b, u2, gp = cases.phillips(g, 3.0)
     rng = np.random.default_rng(n + L)
     h = np.repeat(h2.sum(0)[None] / L, L, 0)
@@ -82,8 +79,78 @@ def test_ocean(grids, n, L, nfast, wall, floor, precision):
         land = rng.random(g.N) < 0.1
         kw['wall'] = np.where(land[g.eI] | land[g.eJ], 0.0, 1.0)
         u *= kw['wall'][None]
+    return kw, h, u
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast', [(6, 2, 3), (6, 8, 1), (2, 3, 1), (3, 3, 2), (4, 3, 3), (4, 1, 4), (4, 2, 5), (4, 4, 7), (3, 5, 9),
+                                       (4, 6, 11), (4, 7, 8), (4, 8, 6)])
+def test_air(grids, n, L, nfast, precision):
+    print(f'case: air n={n} L={L} nfast={nfast} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u, theta = _air(g, n, L)
+    diff = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta)
+    assert max(diff.values()) <= BARS[precision], diff
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast,wall,floor', [(6, 4, 5, True, 0.995), (2, 2, 1, True, 1.0), (3, 1, 2, False, 1.0), (4, 2, 3, True, 1.0),
+                                                  (4, 2, 4, True, 0.995), (3, 3, 5, True, 0.995), (4, 2, 6, False, 0.995),
+                                                  (4, 5, 9, True, 0.999), (4, 8, 11, True, 0.995)])
+def test_ocean(grids, n, L, nfast, wall, floor, precision):
+    """floor below one: that share of the layers' mean thickness, which many cells start beneath."""
+    print(f'case: ocean n={n} L={L} nfast={nfast} wall={wall} floor={floor} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u = _ocean(g, n, L, wall, floor)
     diff = _step(g, precision, kw, h, u, 100.0 * nfast, nfast)
     assert max(diff.values()) <= BARS[precision], diff
+
+
+def _no_rings(s):
+    s.rg_head = None
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast', [(2, 3, 1), (4, 1, 4), (4, 3, 5), (3, 8, 3)])
+def test_air_without_rings(grids, n, L, nfast, precision):
+    """The passes of a mesh without the ring tables (one sub-step to a launch, the limiter apart from the update)."""
+    print(f'case: air without rings n={n} L={L} nfast={nfast} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u, theta = _air(g, n, L)
+    diff, ran = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta, _no_rings)
+    assert max(diff.values()) <= BARS[precision], diff
+    assert {'af_muphi', 'af_u', 'scale', 'limit_h'} <= ran and not {'af_rings', 'limit_rings'} & ran, ran
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast,wall,floor', [(2, 2, 1, True, 1.0), (4, 1, 3, False, 1.0), (4, 2, 5, True, 0.995),
+                                                  (3, 8, 4, True, 0.999)])
+def test_ocean_without_rings(grids, n, L, nfast, wall, floor, precision):
+    print(f'case: ocean without rings n={n} L={L} nfast={nfast} wall={wall} floor={floor} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u = _ocean(g, n, L, wall, floor)
+    diff, ran = _step(g, precision, kw, h, u, 100.0 * nfast, nfast, edit=_no_rings)
+    assert max(diff.values()) <= BARS[precision], diff
+    assert {'bt_eta', 'bt_u', 'scale', 'limit_h', 'lay_u'} <= ran and not {'bt_rings', 'limit_rings'} & ran, ran
+
+
+@pytest.mark.parametrize('air', [True, False])
+def test_patches_too_large_for_a_block(grids, air):
+    """Patches said to hold more cells of their own than a block has threads (each steps on one) are not stepped in rings."""
+    print(f'case: patches too large, air={air}', flush=True)
+    g = grids(3)
+
+    def large(s):
+        for r in range(6):
+            s.rg_cells[r] = max(s.rg_cells[r], 300)
+    if air:
+        kw, h, u, theta = _air(g, 3, 3)
+        diff, ran = _step(g, 'double', kw, h, u, 360.0, 3, theta, large)
+    else:
+        kw, h, u = _ocean(g, 3, 2, True, 1.0)
+        diff, ran = _step(g, 'double', kw, h, u, 300.0, 3, edit=large)
+    assert max(diff.values()) <= BARS['double'], diff
+    assert not {'af_rings', 'bt_rings', 'limit_rings'} & ran, ran
 
 
 @pytest.mark.parametrize('precision', ['double', 'mixed'])
