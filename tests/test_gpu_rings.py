@@ -1,12 +1,17 @@
 """The passes that run on the 64-cell patches -- several fast sub-steps to a launch, the limiter with the thickness and wind
 update, the transport with its rows cell-major -- and the slow tendency against the oracle where their shapes change: every
 remainder of the sub-steps over a launch's three (air) or four (ocean), one to eight layers (at which the rings are
-shallower, or absent, as LDS fills), a thread to an edge's layer (levels to 5) or to all of them (level 6), row counts about
-the four to a load and the eight to a block, meshes whose last patch is part full (162, 642 and 2,562 cells are 2.5, 10.03
-and 40.03 patches), walls, and a floor that holds many cells' outflow back.
+shallower as LDS fills), the ring kernels' three shapes of threads, meshes without ring tables, a thread to an edge's layer
+(levels to 5) or to all of them (level 6), row counts about the four to a load and the eight to a block, meshes whose last
+patch is part full (162, 642 and 2,562 cells are 2.5, 10.03 and 40.03 patches), walls, and a floor that holds many cells'
+outflow back.
 
-Bars: the FP64 form, whose sums keep the oracle's order, to 1e-12 of the largest value after one step; the mixed form to
-1e-5, the figure it is held to over a day."""
+Bars, after one step, of the largest value: the FP64 form, whose sums keep the oracle's terms (the forcing Tp + G is added up
+first and a cell's outflow is summed in its edges' table order, so the last digits differ), to 1e-12. The mixed form holds
+the flux coefficients and the Coriolis term's operands in FP32: a step changes a wind by less than the largest wind, so by
+those roundings of 6e-8 it and the fluxes differ by less than 2e-7 of theirs, and a thickness, which a step changes by less
+than a hundredth, by less than 2e-9 (measured: 4.3e-8, 1.4e-8 and 5.6e-10 at most); a row, of which a step moves less than a
+fifth, with the stencil's values and weights in FP32, by less than 2e-8 (measured: 3.8e-9)."""
 import numpy as np
 import pytest
 import torch
@@ -15,7 +20,11 @@ from conftest import relmax
 
 pytestmark = pytest.mark.gpu
 
-BARS = {'double': 1e-12, 'mixed': 1e-5}
+BARS = {'double': dict(h=1e-12, u=1e-12, Fm=1e-12, rows=1e-12), 'mixed': dict(h=2e-9, u=2e-7, Fm=2e-7, rows=2e-8)}
+
+
+def _within(diff, precision):
+    assert all(v <= BARS[precision][k] for k, v in diff.items()), diff
 
 
 def _np(t):
@@ -90,7 +99,7 @@ def test_air(grids, n, L, nfast, precision):
     g = grids(n)
     kw, h, u, theta = _air(g, n, L)
     diff = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta)
-    assert max(diff.values()) <= BARS[precision], diff
+    _within(diff, precision)
 
 
 @pytest.mark.parametrize('precision', ['double', 'mixed'])
@@ -103,7 +112,36 @@ def test_ocean(grids, n, L, nfast, wall, floor, precision):
     g = grids(n)
     kw, h, u = _ocean(g, n, L, wall, floor)
     diff = _step(g, precision, kw, h, u, 100.0 * nfast, nfast)
-    assert max(diff.values()) <= BARS[precision], diff
+    _within(diff, precision)
+
+
+def _wide(s):
+    """Three rings said to touch more edges than three to a thread: as the level-7 mesh's largest patch does."""
+    for r in range(3, 6):
+        s.rg_edges[r] = max(s.rg_edges[r], 771)
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,nfast', [(3, 1, 3), (4, 2, 4), (4, 3, 6), (4, 4, 9), (4, 5, 7), (4, 6, 3), (3, 8, 3)])
+def test_air_wide_patches(grids, n, L, nfast, precision):
+    """The shape with four edges and two cells to a thread, which level 7 runs (from six layers on LDS takes a ring less)."""
+    print(f'case: air wide n={n} L={L} nfast={nfast} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u, theta = _air(g, n, L)
+    diff, ran = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta, _wide)
+    _within(diff, precision)
+    assert 'af_rings' in ran and 'limit_rings' in ran, ran
+
+
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+def test_level_7(grids, precision):
+    """One step of three air layers and of two ocean layers on the largest mesh that is served."""
+    print(f'case: level 7 {precision}', flush=True)
+    g = grids(7)
+    kw, h, u, theta = _air(g, 7, 3)
+    _within(_step(g, precision, kw, h, u, 180.0, 3, theta), precision)
+    kw, h, u = _ocean(g, 7, 2, True, 0.995)
+    _within(_step(g, precision, kw, h, u, 400.0, 8), precision)
 
 
 def _no_rings(s):
@@ -118,7 +156,7 @@ def test_air_without_rings(grids, n, L, nfast, precision):
     g = grids(n)
     kw, h, u, theta = _air(g, n, L)
     diff, ran = _step(g, precision, kw, h, u, 120.0 * nfast, nfast, theta, _no_rings)
-    assert max(diff.values()) <= BARS[precision], diff
+    _within(diff, precision)
     assert {'af_muphi', 'af_u', 'scale', 'limit_h'} <= ran and not {'af_rings', 'limit_rings'} & ran, ran
 
 
@@ -130,7 +168,7 @@ def test_ocean_without_rings(grids, n, L, nfast, wall, floor, precision):
     g = grids(n)
     kw, h, u = _ocean(g, n, L, wall, floor)
     diff, ran = _step(g, precision, kw, h, u, 100.0 * nfast, nfast, edit=_no_rings)
-    assert max(diff.values()) <= BARS[precision], diff
+    _within(diff, precision)
     assert {'bt_eta', 'bt_u', 'scale', 'limit_h', 'lay_u'} <= ran and not {'bt_rings', 'limit_rings'} & ran, ran
 
 
@@ -149,7 +187,7 @@ def test_patches_too_large_for_a_block(grids, air):
     else:
         kw, h, u = _ocean(g, 3, 2, True, 1.0)
         diff, ran = _step(g, 'double', kw, h, u, 300.0, 3, edit=large)
-    assert max(diff.values()) <= BARS['double'], diff
+    _within(diff, 'double')
     assert not {'af_rings', 'bt_rings', 'limit_rings'} & ran, ran
 
 
@@ -185,6 +223,7 @@ def test_transport_rows(grids, n, L, K, precision):
         tr.step_rows(dg.asarray(M), dg.asarray(M1), dg.asarray(Fm), rd, 3)
         torch.cuda.synchronize()
         out.append(_np(rd))
-        assert relmax(out[-1], ro) <= BARS[precision], f'padded {padded}'
+        print('rows', relmax(out[-1], ro), flush=True)
+        _within(dict(rows=relmax(out[-1], ro)), precision)
     if precision == 'double':
         assert np.array_equal(out[0], out[1])
