@@ -2425,18 +2425,32 @@ int mass_update(const isw_grid* g, int L, const double* M0, const double* Fm, do
 // They need the patches, the scratch's rows padded to a multiple of four (rows_pad at least rows_max: a smaller one is
 // taken as not given) and every array of it where 16 bytes are loaded at once.
 int transport_shape(const isw_grid* g, const isw_transport* tr, int rows) {
-  const int RS = (rows + 3) / 4 * 4, RC = RS > 4 ? 8 : 4, chunks = (RS + RC - 1) / RC;
+  constexpr int CUS = 256;
+  const int RS = (rows + 3) / 4 * 4, c4 = RS / 4, c8 = (RS + 7) / 8;
   if (!g->pi_off || g->pcells != BS1 || g->E < g->N || RS > tr->rows_pad || tr->rows_max > tr->rows_pad) return 0;
   if (ISW_FORM_MIXED && !tr->pf2) return 0;
   const void* at[] = {tr->td, tr->p1, tr->p2, tr->Rp, tr->Rm, tr->Hf, tr->A, tr->pf, tr->pf2};
   for (const void* p : at)
     if (reinterpret_cast<uintptr_t>(p) & 15) return 0;
-  // Eight rows to a block share its edges' tables twice as often as four (15 rows at level 6: 96.1 us of kernels against
-  // 110.4); four where no more are there. Only where at least three in four of the blocks' rows are real, for the others
-  // cost as much: 9 and 10 rows of 16 at level 6 81 and 88 us with the rows apart against 88 and 92, 5 of 8 (FP64) 63
-  // against 65, but 12 of 16 (FP64) 108 against 103, 20 of 24 153 against 129, 3 of 4 44 against 41
-  if (4 * rows < 3 * RC * chunks || (size_t)g->ptedges * RC * 2 * sizeof(double) > 65536) return 0;
-  return RC;
+  const long b4 = (long)g->npatch * c4, b8 = (long)g->npatch * c8;
+  auto fits = [&](int rc) { return (size_t)g->ptedges * rc * 2 * sizeof(double) <= 65536 ? rc : 0; };
+  if (rows < 3) return 0;                          // (2 rows at level 6, FP64: 38 us apart, 43 with two of padding)
+  // Four rows to a block: where no more are there, and on meshes so small that every block has a CU of its own (the mixed
+  // form: a third of one), for then a pass takes as long as its blocks do, which is less for smaller ones, and padding is
+  // free (level 4, 15 rows, FP64: 35.1 us apart, 37.3 eight to a block, 34.0 four; 5 rows 34.1, 35.3, 30.5; level 5, mixed,
+  // 15 rows 47.7, 45.0, 43.4; FP64, at two blocks to a CU, 50.1, 49.1, 53.0); and for ten to twelve, which eight to a
+  // block would pad to sixteen (12 rows: level 5, FP64, 44.5 us, 47.0, 38.5; level 6, mixed, 100.5, 87.8, 76.5)
+  if (c4 == 1 || (c4 == 3 && rows > 9) || b4 <= (ISW_FORM_MIXED ? 3 : 1) * CUS) return fits(4);
+  // Eight: they share the edges' tables twice as often (15 rows at level 6: 96.1 us of kernels against 110.4), but cost as
+  // much for a padded row as for a real one: with three in four of their rows real or more (9 of 16 at level 6 81 us apart,
+  // 88 so; 5 of 8, FP64, 63 and 65, but at level 5, a CU to a block, 37.7 and 36.4; 20 of 24 at level 6 151 and 123), and,
+  // of more than one chunk, with five in nine of what the chip could hold in the rounds that its CUs take blocks in (FP64,
+  // level 5: 14 rows of seven layers, 0.55 of two rounds, 48.8 us apart and 50.4 so; 15 rows, 0.59, 50.1 and 49.2; level 4:
+  // 25 rows, 0.50, 37.4 and 37.8; 28, 0.56, 40.7 and 37.7)
+  const long rounds = (b8 + CUS - 1) / CUS;
+  const bool real = rows * 4 >= 3 * 8 * c8 || (c8 == 1 && b8 <= CUS);
+  const bool held = c8 == 1 || 9l * rows * g->npatch >= 5 * 8 * CUS * rounds;
+  return real && held ? fits(8) : 0;
 }
 
 // Transport.step_many (transport.py:40-71) on rows stacked in psi; the result is written back into psi.

@@ -277,6 +277,28 @@ def test_transport_keeps_rows_apart(prec):
     assert shape(15) == _hip.ISW_EBADARG
 
 
+@pytest.mark.parametrize('level,layers,rows,fp64,mixed', [
+    (2, 1, 1, 0, 0), (6, 1, 2, 0, 0), (6, 3, 3, 4, 4), (7, 1, 4, 4, 4),                     # a block's four rows
+    (4, 5, 5, 4, 4), (4, 3, 15, 4, 4), (4, 3, 24, 4, 4), (3, 5, 40, 4, 4),                  # a CU for every block
+    (5, 5, 5, 8, 4), (5, 3, 6, 8, 4), (5, 7, 14, 0, 4), (5, 3, 15, 8, 4), (5, 5, 20, 8, 8),
+    (4, 5, 25, 0, 4), (4, 7, 28, 8, 4), (4, 7, 35, 8, 4), (5, 5, 25, 8, 8), (5, 7, 35, 8, 8),
+    (6, 5, 5, 0, 0), (6, 3, 6, 8, 8), (6, 3, 9, 0, 0), (6, 5, 10, 4, 4), (6, 3, 12, 4, 4),
+    (6, 7, 14, 8, 8), (6, 3, 15, 8, 8), (6, 1, 17, 0, 0), (6, 5, 20, 8, 8), (7, 3, 15, 8, 8)])
+def test_transport_shape_by_size(level, layers, rows, fp64, mixed):
+    """The transport's rows to a block by the mesh's and the rows' number, where each was measured no slower than the rows
+    apart (15 rows of a level-4 mesh went eight to a block: 82 blocks for 256 CUs)."""
+    lib = _hip.lib()
+    g = _grid(n=10 * 4 ** level + 2, patches=True)
+    tr = _hip.IswTransport()
+    for k, t in _hip.IswTransport._fields_[5:]:
+        setattr(tr, k, ctypes.cast(ctypes.c_void_p(1 << 20), t))
+    tr.L, tr.rows_max, tr.rows_pad = layers, rows, (rows + 3) // 4 * 4
+    got = []
+    for tr.prec in (_hip.ISW_FP64, _hip.ISW_MIXED):
+        got.append(lib.isw_transport_shape(ctypes.byref(g), ctypes.byref(tr), rows))
+    assert got == [fp64, mixed]
+
+
 def test_ocean_column_refusals():
     """The ocean's column entry points refuse bad sizes and settings on the host (no launch)."""
     lib = _hip.lib()

@@ -12,6 +12,8 @@ the flux coefficients and the Coriolis term's operands in FP32: a step changes a
 those roundings of 6e-8 it and the fluxes differ by less than 2e-7 of theirs, and a thickness, which a step changes by less
 than a hundredth, by less than 2e-9 (measured: 4.3e-8, 1.4e-8 and 5.6e-10 at most); a row, of which a step moves less than a
 fifth, with the stencil's values and weights in FP32, by less than 2e-8 (measured: 3.8e-9)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -195,9 +197,26 @@ def test_patches_too_large_for_a_block(grids, air):
 @pytest.mark.parametrize('n,L,K', [(4, 1, 1), (3, 3, 1), (4, 2, 2), (2, 5, 1), (4, 7, 1), (4, 2, 4), (3, 3, 3), (4, 4, 3),
                                    (4, 3, 5), (4, 8, 2), (4, 1, 17)])
 def test_transport_rows(grids, n, L, K, precision):
-    """K tracers of L layers by unequal mass fluxes, steep rows among them (row counts that fill three quarters of their
-    blocks, and ones that do not and are kept apart), and the same rows where the scratch is not padded: both against the oracle, the FP64 form's the same to the bit."""
+    """K tracers of L layers by unequal mass fluxes, steep rows among them (row counts that fill their blocks, ones that do
+    not, and ones that are kept apart), and the same rows where the scratch is not padded: both against the oracle, the FP64
+    form's the same to the bit."""
+    _transport(grids, n, L, K, precision)
+
+
+@pytest.mark.parametrize('n,L,K,shapes', [(5, 3, 2, (8, 4)), (5, 5, 4, (8, 8)), (4, 7, 5, (8, 4)), (5, 3, 4, (4, 4)),
+                                          (5, 7, 2, (0, 4)), (5, 5, 1, (8, 4)), (6, 3, 5, (8, 8)), (6, 1, 11, (4, 4)),
+                                          (6, 3, 3, (0, 0)), (4, 5, 5, (0, 4)), (4, 4, 7, (8, 4))])
+def test_transport_shapes(grids, n, L, K, shapes):
+    """The same with four rows to a block, eight, and apart, in the FP64 and the mixed form, at the lines of the rule that
+    chooses them."""
+    for precision, rows in zip(('double', 'mixed'), shapes):
+        assert _transport(grids, n, L, K, precision) == rows
+
+
+def _transport(grids, n, L, K, precision):
+    """Compares one step with the oracle; the rows to a block that it took, 0 for rows kept apart."""
     import oracle
+    from insilica import _hip
     from insilica.gpu import DeviceGrid
     from insilica.transport import Transport
     print(f'case: transport n={n} L={L} K={K} {precision}', flush=True)
@@ -227,3 +246,5 @@ def test_transport_rows(grids, n, L, K, precision):
         _within(dict(rows=relmax(out[-1], ro)), precision)
     if precision == 'double':
         assert np.array_equal(out[0], out[1])
+    tr.s.rows_pad = (L * K + 3) // 4 * 4
+    return _hip.lib().isw_transport_shape(dg.ref, ctypes.byref(tr.s), L * K)
