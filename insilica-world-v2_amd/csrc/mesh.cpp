@@ -516,13 +516,17 @@ int isw_mesh_weights(int64_t N, int64_t E, const uint8_t* deg, const int32_t* eI
 // cell's sign on it is negative, 0x7fff for no edge; ecell: per edge the places of its first and second cell in the
 // patch's cell list (first | second << 16), 0 for edges that touch ring K only (their outer cell is not listed).
 // sizes (3 + 12): entries of cell, entries of edge, the most owned edges of a patch; then the most cells within ring
-// 0 .. K (six places) and the most edges touching those (six). Called twice, first with head NULL for the sizes. Returns -1 when an edge lacks a cell or a patch is too large for its slots.
+// 0 .. K (six places) and the most edges touching those (six). Called twice, first with head NULL for the sizes. Returns -1
+// when an edge lacks a cell, a cell's position is not finite (the bisection orders cells by it) or a patch is too large for
+// its slots.
 int isw_mesh_rings(int64_t N, int64_t E, int K, int64_t pcells, const double* pos, const int32_t* cellEdge,
                    const int8_t* cellSign, const int32_t* eI, const int32_t* eJ, int64_t* sizes, int32_t* head,
                    int32_t* cell, int32_t* slot, int32_t* edge, int32_t* ecell) {
   if (K < 1 || K > 5 || pcells < 1 || N < 1) return -2;
   for (int64_t e = 0; e < E; e++)
     if (eI[e] < 0 || eJ[e] < 0 || eI[e] >= N || eJ[e] >= N) return -1;
+  for (int64_t k = 0; k < 3 * N; k++)
+    if (!std::isfinite(pos[k])) return -1;
   const int64_t nb = (N + pcells - 1) / pcells;
   std::vector<int32_t> order(N);
   std::iota(order.begin(), order.end(), 0);

@@ -241,7 +241,8 @@ def make(n, order=None, lloyd=None):
 def rings(g, depth, pcells=64):
     """The patches of `g` with `depth` rings of neighbours (isw_grid's rg_* tables, see csrc/mesh.cpp): a dict of int32
     arrays head, cell, slot, edge, ecell, the most edges a patch owns (owned) and, per ring, the most cells and edges a patch
-    has within it (cells, edges: six values); None for a mesh with an edge lacking a cell or without cell positions. A union of meshes (its `parts`) has its parts' patches, in turn."""
+    has within it (cells, edges: six values); None for a mesh with an edge lacking a cell or without finite cell positions. A
+    union of meshes (its `parts`) has its parts' patches, in turn."""
     parts = getattr(g, 'parts', None)
     if parts is not None:
         each = [rings(p, depth, pcells) for p in parts]

@@ -135,3 +135,22 @@ def test_ring_tables(n, pc, union):
         edges_seen.append(G[:h[2]])
     assert np.array_equal(np.sort(np.concatenate(cells_seen)), np.arange(g.N))
     assert np.array_equal(np.sort(np.concatenate(edges_seen)), np.arange(g.E))
+
+
+def test_ring_tables_refused():
+    """A mesh with an edge lacking a cell, or whose positions cannot be ordered, has no rings (and steps without them)."""
+    import types
+    from insilica.grid import rings
+    g = gridmod.get(3)
+
+    def like(**change):
+        m = types.SimpleNamespace(N=g.N, E=g.E, pos=g.pos, cellEdge=g.cellEdge, cellSign=g.cellSign, eI=g.eI.copy(), eJ=g.eJ)
+        for k, v in change.items():
+            setattr(m, k, v)
+        return m
+    assert rings(like(), 4) is not None
+    pos = np.array(g.pos)
+    pos[7, 1] = np.nan
+    lacking = np.array(g.eJ)
+    lacking[11] = -1
+    assert rings(like(pos=pos), 4) is None and rings(like(pos=None), 4) is None and rings(like(eJ=lacking), 4) is None
