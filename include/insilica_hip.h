@@ -58,8 +58,9 @@ typedef struct isw_grid {
   int32_t npatch, pcells, pslots, pown;
   const int32_t *ph_off, *ph_cell, *pe_off, *pe_edge, *pe_slot;
   /* Two air fast sub-steps per launch on the same patches (optional; checked when given, but no kernel reads these
-   * tables now: the rg_* tables below take their place). The first sub-step's cells: patch, halo and the halo's halo ph2_cell[ph2_off[b] ..] (slots after the halo's); its winds on
-   * every edge of patch and halo: the patch's edges (slots 0 .. ne - 1) and px_edge[px_off[b] ..] (slots from ne),
+   * tables now, and no other of the ph_* than the transport's edge lists: the rg_* tables below take their place, and a
+   * mesh without those steps one sub-step in two launches). The first sub-step's cells: patch, halo and the halo's halo
+   * ph2_cell[ph2_off[b] ..] (slots after the halo's); its winds on every edge of patch and halo: the patch's edges (slots 0 .. ne - 1) and px_edge[px_off[b] ..] (slots from ne),
    * with their cells' slots px_slot (as pe_slot); pc_eslot[3 pc_off[b] ..]: each patch-then-halo cell's six edge
    * slots, two per int32 (0xffff: no edge); pslots2, pedges2: the most cell and edge slots a patch uses. Refused
    * (ISW_EBADARG) when a patch owns more than 256 edges (pown > 256) or its patch and halo hold more than 256 cells
@@ -501,8 +502,8 @@ const char* isw_version(void);
 /* Host-only argument checks (no counterpart in the reference, whose kernels check nothing): each returns 0 where the
  * entry points above would accept the argument and ISW_EBADARG where they refuse it, and launches nothing.
  * isw_grid_check: the mesh struct every grid-taking entry point checks first (tables present, patch tables
- * consistent, at most ISW_PAIR_THREADS owned edges and patch-and-halo cells per patch for the two-sub-step tables). isw_air_column_options:
- * the column options (par in PAR_ORDER, host) that isw_air_column does not carry for L layers. */
+ * consistent, at most ISW_PAIR_THREADS owned edges and patch-and-halo cells per patch for the two-sub-step tables).
+ * isw_air_column_options: the column options (par in PAR_ORDER, host) that isw_air_column does not carry for L layers. */
 int32_t isw_grid_check(const isw_grid* g);
 /* The rows to a block (4 or 8) that isw_transport_step takes for this many rows at order 3, 0 where it keeps the rows
  * apart, ISW_EBADARG for a refused grid or row count (host only, as the checks above). */

@@ -12,8 +12,11 @@
 // read the stage's start state directly (no copies) and keep it in registers and LDS between them; the stage flux
 // F = h_e * mean(u) is recomputed inside the limiter and the divergence instead of being stored, the limited
 // flux's volume Fm is written by each edge's eI cell, and the wall mask is applied inside the kernels that write.
-// Every sum keeps the reference's order (a cell's edges in cellEdge or cellEdgeAsc order, a vertex's three in table
-// order, an edge's eoe neighbours ascending), so the FP64 form matches the reference's double path value for value.
+// Sums keep the reference's order (a cell's edges in cellEdge or cellEdgeAsc order, a vertex's three in table order, an
+// edge's eoe neighbours ascending) but for two on the ring patches: a fast sub-step adds the wind's forcing Tp + G before
+// the gradient (the reference adds them to it one by one), and the limiter sums a cell's outflow in cellEdge order and
+// scales the sum by the step (the reference in cellEdgeAsc order, each term scaled). So the FP64 form matches the
+// reference's double path to rounding: within 1e-12 of the largest value after a step.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -583,8 +586,9 @@ __global__ __launch_bounds__(BS) void k_af_u(isw_grid g, int L, Div dv, LP p, in
 // the bit. Between the steps only LDS is touched: the edges' threads leave each flux coef * u there, the cells' threads
 // leave each potential. So a launch pays its chain of dependent loads (arguments, the patch's record, the index lists,
 // the values) once for m steps, about 6 us of it before the first step at level 6 (three layers, mixed: 7.7 us for one
-// step, 9.4 for two, 11.2 for three); what bounds each further step is LDS: six fluxes per cell, two potentials per edge. Two buffers alternate for masses and winds, as a neighbour block may still read a launch's
-// inputs. A patch's cells are of one world, so a batch's counts and lengths are the block's.
+// step, 9.4 for two, 11.2 for three); what bounds each further step is LDS: six fluxes per cell, two potentials per edge.
+// Two buffers alternate for masses and winds, as a neighbour block may still read a launch's inputs. A patch's cells are of
+// one world, so a batch's counts and lengths are the block's.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int RBS = 256;
 // The sub-steps a launch takes. Air: 3 (level 6, three layers, nfast 15, the 28 sub-steps of a step: 216 us at one per
@@ -2115,7 +2119,8 @@ static void lap(const isw_grid* g, int L, const double* u, double* D1, double* Z
 
 // The fast sub-steps that one launch takes on the grid's ring tables, for `rows` values per cell: as many as asked for
 // whose rings fit a block's threads (four edges and two cells each) and 64 KB of LDS; 0 without the tables.
-// (The kernels come with 2 or 3 edges and one cell to a thread, or 4 edges and two cells.)
+// (The kernels come with 2 or 3 edges and one cell to a thread, or 4 edges and two cells; the mesh's largest patch decides
+// for all: at level 7 one of 2,561 touches 771 edges within three rings, three more than 3 to a thread.)
 static int ring_cpt(const isw_grid* g, int m) { return g->rg_cells[m] > RBS || g->rg_edges[m] > 3 * RBS ? 2 : 1; }
 static int ring_ept(const isw_grid* g, int m) {
   const int k = (g->rg_edges[m] + RBS - 1) / RBS, least = ring_cpt(g, m) == 2 ? 4 : 2;

@@ -14,7 +14,7 @@
 // LDS as float32 (the reference's red[][] width) and are summed in FP64 in a fixed order, so results repeat bit for bit.
 // Blocks are renumbered so that each XCD takes a contiguous range of columns (the sub-level reads of neighbouring columns
 // share cache lines). Measured at 40,962 columns x 7 layers, mixed: lw_column (256 g-points) 3.72 -> 1.44 ms, sw_column
-// (224) 6.86 -> 2.21 ms; FP64 at 2,562 x 3 (144 / 112): 192 -> 109 us and 273 -> 113 us.
+// (224) 6.86 -> 2.18 ms; FP64 at 2,562 x 3 (144 / 112): 192 -> 109 us and 273 -> 113 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -54,7 +54,8 @@ __device__ __forceinline__ double FPOWd(double x, double y) {
 }
 // The column passes' exp and quotient: FP64 in the plain form (the reference's operations); in the mixed form the
 // hardware's: exp as 2^(x log2 e) (v_exp_f32) and a / b as a times the hardware reciprocal, each within a few float
-// steps (the mixed form's bar against FP64 is 1e-4 of the fluxes).
+// steps (the mixed form's bar against FP64 is 1e-4 of the fluxes). fquot stands in the longwave's emission and in the two
+// denominators of the shortwave's adding, where an IEEE quotient was no closer to 64 bits.
 __device__ __forceinline__ fast fexp(fast x) {
 #if ISW_FORM_MIXED
   return __expf(x);
@@ -70,9 +71,10 @@ __device__ __forceinline__ fast fquot(fast a, fast b) {
 #endif
 }
 // The shortwave's layer optics divide by 1 - (k mu0)^2, which passes through zero where the beam and the diffuse light
-// decay alike: what they lose to rounding there is a thousand times larger, so their quotients and square root are
-// rounded as IEEE's are: one Newton step on the hardware's reciprocal (or reciprocal root), then one on the residual, and
-// the fix-up for zeros and infinities. Six instructions besides the reciprocal where the compiler's division takes ten, for
+// decay alike: what they lose to rounding there is a thousand times larger, so their quotients and square root take one
+// Newton step on the hardware's reciprocal and one on the residual (the root one on the residual alone), and the quotients
+// the fix-up for zeros and infinities: within a float step of IEEE's for normal operands, mostly equal to them, though
+// not shown to be in every case. Six instructions besides the reciprocal where the compiler's division takes ten, for
 // it does not scale: where b is denormal its reciprocal is infinite and the Newton step not a number, so what may vanish
 // is divided by only above TINY.
 constexpr fast TINY = ISW_FORM_MIXED ? (fast)1.17549435e-38f : (fast)0;
@@ -456,7 +458,8 @@ __global__ void __launch_bounds__(NGMAX) k_lw_column(int N, int cpb, RadP P, isw
           }
           // two-stream through the sub-level, the Planck radiance linear in optical depth, diffusivity 1.66
           // (air.cu:2123-2127): t = e^-x, E = B_far (1 - t) + (B_near - B_far) lin
-          const fast Bt = row_s.t0 + (fast)(row_s.t1 - row_s.t0) * spt[s], Bb = row_s.b0 + (fast)(row_s.b1 - row_s.b0) * spb[s];
+          const fast Bt = row_s.t0 + (fast)(row_s.t1 - row_s.t0) * spt[s];
+          const fast Bb = row_s.b0 + (fast)(row_s.b1 - row_s.b0) * spb[s];
           auto through = [&](fast y, fast& tt, fast& ed, fast& eup) {
             tt = fexp(-y);
             const fast om = 1 - tt, thin = y * ((fast)0.5 - y * (fast)(1.0 / 6.0)), thick = 1 - fquot(om, y);
@@ -619,9 +622,9 @@ __device__ double sun_lon(double t, const RadP& P) {
 // each sub-level's map of the light going down through it, Fdir' = d Fdir, Fdif' = a Fdif + c Fdir, with what lies
 // below already known. Only the nets at three edges per layer are wanted, so a layer keeps three maps (the second and
 // third sub-level's composed) with the albedos below each, 15 values per layer, and the way down is five multiply-adds
-// per edge. What bounds it then is the vector ALU: about 240 instructions and 17 transcendentals per sub-level. (Evaluating look-ups and optics again on the way down, with the tables' rows addressed per
-// lane and the sun's position found anew by one lane per column, the pass took 6.89 ms at 40,962 x 7 x 224 in the mixed
-// form.) The sun's direction at the four times of the interval is found once per block, one lane each.
+// per edge. What bounds it then is the vector ALU: about 240 instructions and 17 transcendentals per sub-level. (Evaluating
+// look-ups and optics again on the way down, with the tables' rows addressed per lane and the sun's position found anew by
+// one lane per column, the pass took 6.89 ms at 40,962 x 7 x 224 in the mixed form.) The sun's direction at the four times of the interval is found once per block, one lane each.
 // ---------------------------------------------------------------------------------------------------------------
 template <int L>
 __global__ void __launch_bounds__(NGMAX, ISW_FORM_MIXED ? 3 : 1) k_sw_column(int N, int cpb, RadP P, isw_sw_tables t, isw_air air,

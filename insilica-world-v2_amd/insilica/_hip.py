@@ -8,7 +8,7 @@ from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / '_lib' / 'libinsilica_hip.so'
 ISW_FP64, ISW_MIXED, ISW_EBADARG, LMAX, KSOIL = 0, 1, 9001, 8, 16
-ISW_PAIR_THREADS = 256            # the most edges a patch may own for the two-sub-step kernel (one thread each)
+ISW_PAIR_THREADS = 256            # with the ph2_* tables, the most edges a patch may own (checked; no kernel reads them)
 ISW_DSUM_NOALLOC_MAX_N = 1 << 25  # the most values isw_dsum_noalloc sums (its static workspace's limit)
 ISW_LLOYD_MAX_CHUNK = 4096        # the most Lloyd iterations isw_mesh_lloyd queues between reads of their moves
 

@@ -35,10 +35,11 @@ RING_STEPS = 4              # the rings of the fast sub-steps' patches: the most
 
 
 def fast_patches(grid, pcells=64):
-    """The air fast sub-step's patches (isw_grid's ph_* and pe_* tables): patch b holds cells [b pcells, (b + 1)
+    """The patches of consecutive cells (isw_grid's ph_* and pe_* tables): patch b holds cells [b pcells, (b + 1)
     pcells), its edges are those whose first cell is in it, its halo the second cells of those edges outside it. Each
-    edge's two cells get LDS slots (in the patch: their offset; in the halo: pcells + their index in the sorted halo).
-    Returns None for a mesh with an edge lacking a cell. Every invariant the kernel relies on is checked here."""
+    edge's two cells get slots (in the patch: their offset; in the halo: pcells + their index in the sorted halo). The
+    transport's kernels read the edge lists; the halos and slots are part of the mesh struct that no kernel reads now.
+    Returns None for a mesh with an edge lacking a cell. Every invariant is checked here."""
     N, E = int(grid.N), int(grid.E)
     eI, eJ = np.asarray(grid.eI, np.int64), np.asarray(grid.eJ, np.int64)
     if E == 0 or eI.min() < 0 or eJ.min() < 0 or eI.max() >= N or eJ.max() >= N:
@@ -70,7 +71,8 @@ def fast_patches(grid, pcells=64):
 
 
 def fast_patches2(grid, pt, max_owned=_hip.ISW_PAIR_THREADS):
-    """Two air fast sub-steps per launch on the same patches (isw_grid's ph2_*, px_*, pc_* tables): the cells of the
+    """Tables of two air fast sub-steps per launch on the same patches (isw_grid's ph2_*, px_*, pc_*: accepted and checked,
+    read by no kernel now; the ring tables of grid.rings took their place, and DeviceGrid builds those): the cells of the
     first sub-step are the patch, its halo (pt's) and the halo's own halo, the cells of the edges of patch and halo;
     the winds of the first sub-step are needed on every edge of patch and halo (the patch's own edges first, in pt's
     order, then the others); the second sub-step's cells are patch and halo again. Cell slots: the patch at its

@@ -134,8 +134,8 @@ def test_column_options_predicate():
 
 
 def test_grid_check_pair_tables():
-    """The two-sub-step patch tables are refused when a patch owns more edges than the pair kernel has threads, and
-    accepted at the limit (host check only, no launch)."""
+    """The two-sub-step patch tables (which no kernel reads now) are refused when a patch owns more than ISW_PAIR_THREADS
+    edges, and accepted at the limit (host check only, no launch)."""
     lib = _hip.lib()
     E = _hip.ISW_EBADARG
     buf = (ctypes.c_int32 * 8)()

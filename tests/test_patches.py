@@ -1,7 +1,9 @@
-"""The fast sub-steps' patch tables (insilica.gpu.fast_patches, fast_patches2), checked on the host against the data
-each phase of the patch kernels reads: one fused sub-step needs Phi* on both cells of every edge it steps; two fused
-sub-steps need the first sub-step's winds on every edge of the second's cells, and its Phi* on both cells of each of
-those edges. A wrong slot would read another cell's value; these checks name every slot's cell and edge."""
+"""The patch tables, checked on the host against the mesh: those that kernels read -- the transport's edge lists
+(fast_patches, transport_patches) and the fast sub-steps' rings (grid.rings) -- and those that the mesh struct still takes
+though no kernel reads them now: fast_patches' halos and slots (one fused sub-step needs Phi* on both cells of every edge it
+steps) and fast_patches2 (two fused sub-steps need the first's winds on every edge of the second's cells, and its Phi* on
+both cells of each of those edges). A wrong slot would read another cell's value; these checks name every slot's cell and
+edge."""
 import numpy as np
 import pytest
 
