@@ -19,6 +19,7 @@ def test_traffic_rows_from_the_profile():
             name = cells[0].strip('`')[2:].split('<')[0]
             rows.setdefault(name, float(cells[-1]) * 1e6)
     assert 'af_patch2' in rows and 'slow_e' in rows
+    assert 'af_rings' in rows                                          # (the dominant kernel)
     for name, want in rows.items():
         assert bench.pmc_traffic(name) == want, name
     assert bench.pmc_traffic('no_such_kernel') is None
