@@ -230,3 +230,45 @@ def test_shortwave_of_vanishing_depths(ray, haze, precision):
         torch.cuda.synchronize()
         out.append(_np(sw.swf))
     assert np.all(np.isfinite(out[0])) and np.max(np.abs(out[0] - out[1])) <= 1e-6
+
+
+@pytest.mark.parametrize('precision,bar', [('double', 1e-8), ('mixed', 1e-4)])
+@pytest.mark.parametrize('L', [3, 7])
+def test_options_of_the_column_passes(L, precision, bar):
+    """The branches of the column passes that the other tests leave out: absorption by collisions (cia) in both, another
+    air's Rayleigh scattering and oxygen, a fixed mean cosine (mode 1), clouds with the drops' optics for ice, a clear sky
+    without haze, g-points that do not fill the last eight: on the same sub-levels, against the oracle."""
+    from insilica.ktables import synthetic_lw, synthetic_sw
+    from insilica.radiation import Longwave, Shortwave
+    from oracle import radiation as orad
+    N = 100
+    print(f'case: radiation options L={L} {precision}', flush=True)
+    c, pos, par = case(N, L, 41 + L)
+    rng = np.random.default_rng(L)
+    lwk, swk = synthetic_lw(bands=7, g_per_band=11, seed=1), synthetic_sw(bands=5, g_per_band=13, seed=2)
+    air = dict(cia=1, ray=0.7, o2=0.1)
+    mu, th, q, co = (_dev(c[k]) for k in ('mu', 'theta', 'q', 'cloudo'))
+    for t in (lwk, swk):
+        t['cia'] = np.zeros((t['logk'].shape[2], t['logk'].shape[3]))
+    lw = Longwave(N, L, par, tables=lwk, precision=precision, air=air)
+    lw.setup(mu, th, q, co)
+    amount = _np(lw.sub).reshape(4 * L, 15, N)[:, 14]
+    assert amount.min() > 0
+    for t in (lwk, swk):
+        t['cia'] = rng.uniform(0.05, 2.0, t['cia'].shape) / np.median(amount)
+    lw = Longwave(N, L, par, tables=lwk, precision=precision, air=air)
+    lw(mu, th, q, co, _dev(c['Ts']))
+    sub = _np(lw.sub)
+    ora = orad.lw_column(N, L, par, orad.LwTables(lwk, cia=lwk['cia']), sub, c['Ts'])
+    none = orad.lw_column(N, L, par, orad.LwTables(lwk), sub, c['Ts'])
+    e_lw = np.max(np.abs(_np(lw.radf) - ora) / lw_scale(ora, L))
+    assert np.max(np.abs(none - ora) / lw_scale(ora, L)) > 0.01         # (the option matters here)
+    for mode, clouds, haze in ((0, True, True), (1, True, True), (1, False, False)):
+        k = dict(swk) if haze else dict(swk, haze_par=np.concatenate([[0.0], swk['haze_par'][1:]]))
+        sw = Shortwave(N, L, par, lw, tables=k, precision=precision, air=air)
+        sw(mode, _dev([3.0e6]), 3600.0, _dev(pos), _dev(c['alb']), co if clouds else None)
+        osw = orad.sw_column(N, L, par, orad.SwTables(k, cia=k['cia']), sub, c['alb'], mode=mode, tnow=3.0e6,
+                             interval=3600.0, pos=pos, cloudo=c['cloudo'] if clouds else None, air=air)
+        e_sw = np.max(np.abs(_np(sw.swf) - osw))
+        print(f'mode {mode} clouds {clouds} haze {haze}: lw {e_lw:.2e} sw {e_sw:.2e}', flush=True)
+        assert e_lw <= bar and e_sw <= bar
