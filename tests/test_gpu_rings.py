@@ -146,6 +146,19 @@ def test_level_7(grids, precision):
     _within(_step(g, precision, kw, h, u, 400.0, 8), precision)
 
 
+@pytest.mark.parametrize('precision', ['double', 'mixed'])
+@pytest.mark.parametrize('n,L,air', [(4, 3, True), (6, 3, True), (4, 5, True), (4, 2, False), (6, 3, False)])
+def test_shelf(grids, n, L, air, precision):
+    """Thin layers (thinner than shelf: their tendency blended with the nearest thick layers', or their pressure gradient
+    faded) and a drag, with a thread per layer of an edge and with one for all of them."""
+    print(f'case: shelf n={n} L={L} air={air} {precision}', flush=True)
+    g = grids(n)
+    kw, h, u, *theta = _air(g, n, L) if air else _ocean(g, n, L, True, 1.0)
+    h = np.ascontiguousarray(h * (1 + np.random.default_rng(n).uniform(-0.3, 0.3, h.shape)))
+    kw.update(shelf=float(h.mean()), drag=[1e-6 * (k + 1) for k in range(L)])
+    _within(_step(g, precision, kw, h, u, 120.0, 2, *theta), precision)
+
+
 def _no_rings(s):
     s.rg_head = None
 
