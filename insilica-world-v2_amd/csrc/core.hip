@@ -645,26 +645,27 @@ struct RingCell {
     }
     return ((((t[0] + t[1]) + t[2]) + t[3]) + t[4]) + t[5];
   }
-  // What flows out of the cell.
+  // What flows out of the cell (as the reference counts it: a flux that is not a number is its second cell's).
   __device__ __forceinline__ double out(const double* F) const {
     double s = 0;
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       const double f = F[at[k]];
       const double x = __hiloint2double((int)((unsigned)__double2hiint(f) ^ flip[k]), __double2loint(f));
-      if (x > 0) s += x;
+      if ((f > 0) != (flip[k] != 0)) s += x;
     }
     return s;
   }
 };
 // x / d with r = 1 / d at hand: the plain form's rounds as the division does (a quotient corrected by its exact
-// remainder), the mixed form's is the product (its Div holds reciprocals).
+// remainder; the fix-up keeps an infinite quotient infinite, whose remainder is not a number), the mixed form's is the
+// product (its Div holds reciprocals).
 __device__ __forceinline__ double over(double x, double d, double r) {
 #if ISW_FORM_MIXED
   return x * d;
 #else
   const double q = x * r;
-  return __builtin_fma(__builtin_fma(-q, d, x), r, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-q, d, x), r, q), d, x);
 #endif
 }
 __device__ __forceinline__ double recip(double d) {

@@ -159,6 +159,40 @@ def test_shelf(grids, n, L, air, precision):
     _within(_step(g, precision, kw, h, u, 120.0, 2, *theta), precision)
 
 
+@pytest.mark.parametrize('value', [1e200, 1e305, np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize('L,nfast', [(1, 1), (3, 1), (1, 4), (3, 4)])
+def test_lost_values_spread_as_the_reference_has_them(grids, L, nfast, value):
+    """A wind or a thickness that is infinite, not a number or about to overflow: after a step of the FP64 form the same
+    values are finite, infinite and not a number as the oracle's, and the finite ones (among them those whose limiter met a
+    flux that is not a number) agree."""
+    print(f'case: lost values L={L} nfast={nfast} {value}', flush=True)
+    import oracle
+    from insilica.gpu import DeviceGrid
+    from insilica.layers import Layers
+    g = grids(3)
+    for air in (True, False):
+        for name in ('u', 'h'):
+            kw, h, u, *theta = _air(g, 3, L) if air else _ocean(g, 3, L, False, 1.0)
+            (u if name == 'u' else h)[0, 5] = value
+            dg, og = DeviceGrid(g, 'double'), oracle.Grid(g)
+            lay, olay = Layers(dg, **kw), oracle.Layers(og, **kw)
+            got = dict(h=dg.asarray(h), u=dg.asarray(u), Fm=dg.zeros(L, g.E))
+            want = dict(h=h, u=u, Fm=np.zeros((L, g.E)))
+            td = dg.asarray(theta[0]) if air else None
+            with np.errstate(all='ignore'):
+                if air:
+                    lay.update_gfast(got['h'], td)
+                    olay.update_gfast(h, theta[0])
+                lay.step(got['h'], got['u'], 100.0 * nfast, nfast, got['Fm'], theta=td)
+                olay.step(h, u, 100.0 * nfast, nfast, want['Fm'], theta=theta[0] if air else None)
+            for k, b in want.items():
+                a = _np(got[k])
+                assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b)), (air, name, k)
+                m = np.isfinite(b)
+                scale = np.maximum(np.abs(b[m]), np.median(np.abs(b[m]))) if m.any() else 1.0
+                assert np.all(np.abs(a[m] - b[m]) <= 1e-9 * scale), (air, name, k)
+
+
 def _no_rings(s):
     s.rg_head = None
 
